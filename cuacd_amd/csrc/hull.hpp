@@ -99,6 +99,10 @@ template <int AS> struct HullWS {
     asptr<AS, uint16_t> vout;  // [VC] output index of a hull vertex
     asptr<AS, uint8_t> vref;   // [VC] vertex referenced by a live face / corner flag
     asptr<AS, int> cv;         // [2*VC] canonical form: facet list head, triangle offset per c0
+    // one-wave workspaces only (they have no ha, hb, hface, hedge)
+    asptr<AS, u4v> hz;         // [VC] horizon edge i: start, end vertex, (face beyond it << 2) | its edge slot there
+    asptr<AS, s4v> pq;         // [NP] grid coordinates of the points
+    asptr<AS, f4v> cpl;        // [WAVE_CPL] planes of the step's cone, horizon order
     // Always in LDS, whatever AS is: these are updated with atomics and then
     // read back; global atomics execute in L2 while plain loads may hit a
     // stale line of the CU's L1, so atomic-then-load state stays in LDS.
@@ -164,6 +168,8 @@ template <int AS> __device__ __forceinline__ HullWS<AS> hull_ma_attach(HullWS<AS
     return w;
 }
 
+constexpr int WAVE_CPL = 64;
+
 // FC = 2*VC + 8 faces bound the live faces of a hull with VC vertices plus the
 // transient pair created by one insertion (nhz <= nvis + 2). Face and vertex
 // ids are 16-bit, so VC <= 32760.
@@ -172,11 +178,14 @@ __host__ __device__ constexpr int hull_fc(int vc) { return 2 * vc + 8; }
 // Carves the workspace from `p` (16-byte aligned sub-arrays) and returns its
 // size; with p == nullptr it only sizes it. One routine for both, so the size
 // requested and the carve can never disagree. np = point capacity.
+// kind: what the quickhull needs beside the common arrays.
+enum HullWsKind { HULL_WS_BLOCK = 0, HULL_WS_MULTI = 1, HULL_WS_WAVE = 2 };
+
 template <int AS>
 __host__ __device__ __forceinline__ unsigned hull_ws_layout(char* p, int vc, int np, HullWS<AS>* out,
-                                                            bool multi = false) {
+                                                            int kind = HULL_WS_BLOCK) {
     HullWS<AS> w{};
-    const unsigned fc = (unsigned)hull_fc(vc), v = (unsigned)vc, nw = (unsigned)(np + 31) / 32u;
+    const unsigned fc = (unsigned)hull_fc(vc), v = (unsigned)vc;
     unsigned off = 0;
     auto take = [&](unsigned bytes) {
         char* r = p ? p + off : nullptr;
@@ -187,23 +196,29 @@ __host__ __device__ __forceinline__ unsigned hull_ws_layout(char* p, int vc, int
     w.fv = (asptr<AS, u4v>)take(fc * 8u);
     w.fn = (asptr<AS, u4v>)take(fc * 8u);
     w.fstamp = (asptr<AS, int>)take(fc * 4u);
-    w.fvis = (asptr<AS, uint8_t>)take(fc);
+    w.fvis = (asptr<AS, uint8_t>)take((fc + 63u) / 64u * 64u);
     w.ffree = (asptr<AS, uint16_t>)take(fc * 2u);
     w.vis = (asptr<AS, uint16_t>)take(fc * 2u);
     w.vq = (asptr<AS, s4v>)take(v * 8u);
     w.vpid = (asptr<AS, int>)take(v * 4u);
     w.smap = (asptr<AS, uint16_t>)take(v * 2u);
     w.emap = (asptr<AS, uint16_t>)take(v * 2u);
-    w.hface = (asptr<AS, uint16_t>)take(v * 2u);
-    w.hedge = (asptr<AS, uint8_t>)take(v);
-    w.ha = (asptr<AS, uint16_t>)take(v * 2u);
-    w.hb = (asptr<AS, uint16_t>)take(v * 2u);
+    if (kind == HULL_WS_WAVE) {
+        w.hz = (asptr<AS, u4v>)take(v * 8u);
+        w.pq = (asptr<AS, s4v>)take((unsigned)np * 8u);
+        w.cpl = (asptr<AS, f4v>)take(WAVE_CPL * 16u);
+    } else {
+        w.hface = (asptr<AS, uint16_t>)take(v * 2u);
+        w.hedge = (asptr<AS, uint8_t>)take(v);
+        w.ha = (asptr<AS, uint16_t>)take(v * 2u);
+        w.hb = (asptr<AS, uint16_t>)take(v * 2u);
+    }
     w.hnew = (asptr<AS, uint16_t>)take(v * 2u);
     w.vout = (asptr<AS, uint16_t>)take(v * 2u);
     w.vref = (asptr<AS, uint8_t>)take(v);
     w.cv = (asptr<AS, int>)take(v * 8u);
-    if (multi && AS == AS_LDS) off += hull_ma_layout(p ? p + off : nullptr, fc, &w);
-    (void)nw;  // bm / wpre / ctr live in HullBlockLDS (hull_ws_attach)
+    if (kind == HULL_WS_MULTI && AS == AS_LDS) off += hull_ma_layout(p ? p + off : nullptr, fc, &w);
+    // bm / wpre / ctr live in HullBlockLDS (hull_ws_attach)
     w.VC = vc;
     w.FC = (int)fc;
     w.NP = np;
@@ -211,13 +226,14 @@ __host__ __device__ __forceinline__ unsigned hull_ws_layout(char* p, int vc, int
     return off;
 }
 
-template <int AS> __host__ __device__ inline unsigned hull_ws_bytes(int vc, int np, bool multi = false) {
-    return hull_ws_layout<AS>(nullptr, vc, np, nullptr, multi);
+template <int AS> __host__ __device__ inline unsigned hull_ws_bytes(int vc, int np, int kind = HULL_WS_BLOCK) {
+    return hull_ws_layout<AS>(nullptr, vc, np, nullptr, kind);
 }
 
-template <int AS> __device__ __forceinline__ HullWS<AS> hull_ws_carve(char* p, int vc, int np, bool multi = false) {
+template <int AS>
+__device__ __forceinline__ HullWS<AS> hull_ws_carve(char* p, int vc, int np, int kind = HULL_WS_BLOCK) {
     HullWS<AS> w;
-    hull_ws_layout<AS>(p, vc, np, &w, multi);
+    hull_ws_layout<AS>(p, vc, np, &w, kind);
     return w;
 }
 
@@ -389,43 +405,47 @@ struct HullResult {
     int ftop;   // face ids in use are [0, ftop)
 };
 
-// Cooperative exact quickhull over NW waves (blockDim.x == 64*NW).
-// px/py/pz: grid coords of local points i = k*T + tid (valid iff i < n), T = 64*NW.
-template <int PPL, int AS, int NW, bool MULTI = false>
-__device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBlockLDS* sb, int n, const int (&px)[PPL],
-                                      const int (&py)[PPL], const int (&pz)[PPL]) {
+// Slot `slot` of a per-lane array, selected with masks: written as
+// `if (k == slot) v = a[k]` the compiler turns the loop into an indexed
+// access and moves the whole array to scratch memory.
+template <int PPL> __device__ __forceinline__ int hull_pick(const int (&a)[PPL], int slot) {
+    int v = 0;
+#pragma unroll
+    for (int k = 0; k < PPL; ++k) v |= a[k] & -(int)(k == slot);
+    return v;
+}
+
+// Coordinates of local point ip, broadcast to the whole block.
+template <int PPL, int NW>
+__device__ __forceinline__ void hull_fetch(HullBlockLDS* sb, const int (&px)[PPL], const int (&py)[PPL],
+                                           const int (&pz)[PPL], int ip, int& x, int& y, int& z) {
+    constexpr int T = 64 * NW;
+    const int tid = threadIdx.x, own = ip % T, slot = ip / T;
+    if (NW == 1) {
+        x = read_lane(hull_pick(px, slot), own);
+        y = read_lane(hull_pick(py, slot), own);
+        z = read_lane(hull_pick(pz, slot), own);
+    } else {
+        if (tid == own) {
+            sb->bc[0] = hull_pick(px, slot);
+            sb->bc[1] = hull_pick(py, slot);
+            sb->bc[2] = hull_pick(pz, slot);
+        }
+        __syncthreads();
+        x = sb->bc[0]; y = sb->bc[1]; z = sb->bc[2];
+        __syncthreads();
+    }
+}
+
+// The initial tetrahedron (vertices 0..3, faces 0..3 in the workspace) and
+// every other point's conflict face: conf = the face it is farthest above,
+// -1 inside, -2 a vertex; dist = the height. False for a flat set.
+template <int PPL, int AS, int NW>
+__device__ __forceinline__ bool hull_simplex(const HullWS<AS> w, HullBlockLDS* sb, int n, const int (&px)[PPL],
+                                             const int (&py)[PPL], const int (&pz)[PPL], int (&conf)[PPL],
+                                             float (&dist)[PPL]) {
     constexpr int T = 64 * NW;
     const int tid = threadIdx.x;
-    const int VC = w.VC, FC = w.FC;
-    int conf[PPL];
-    float dist[PPL];
-    HullResult res{HULL_OK, 0, 0};
-
-    // coordinates of local point ip, broadcast to the whole block
-    // Slot `slot` of a per-lane array, selected with masks: written as
-    // `if (k == slot) v = a[k]` the compiler turns the loop into an indexed
-    // access and moves the whole array to scratch memory.
-    auto pick = [&](const int (&a)[PPL], int slot) {
-        int v = 0;
-#pragma unroll
-        for (int k = 0; k < PPL; ++k) v |= a[k] & -(int)(k == slot);
-        return v;
-    };
-    auto fetch = [&](int ip, int& x, int& y, int& z) {
-        const int own = ip % T, slot = ip / T;
-        if (NW == 1) {
-            x = read_lane(pick(px, slot), own);
-            y = read_lane(pick(py, slot), own);
-            z = read_lane(pick(pz, slot), own);
-        } else {
-            if (tid == own) { sb->bc[0] = pick(px, slot); sb->bc[1] = pick(py, slot); sb->bc[2] = pick(pz, slot); }
-            __syncthreads();
-            x = sb->bc[0]; y = sb->bc[1]; z = sb->bc[2];
-            __syncthreads();
-        }
-    };
-
-    // ---- initial simplex --------------------------------------------------
     uint64_t key = ~0ull;
 #pragma unroll
     for (int k = 0; k < PPL; ++k) {
@@ -439,7 +459,7 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
     key = block_min_u64<NW>(key, sb);
     const int i0 = (int)(key & 0x1FFFFF);
     int x0, y0, z0;
-    fetch(i0, x0, y0, z0);
+    hull_fetch<PPL, NW>(sb, px, py, pz, i0, x0, y0, z0);
 
     key = 0;
 #pragma unroll
@@ -453,10 +473,10 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         }
     }
     key = block_max_u64<NW>(key, sb);
-    if ((key >> 32) == 0) { res.status = HULL_DEGENERATE; return res; }
+    if ((key >> 32) == 0) return false;
     int i1 = (int)(0xFFFFFFFFu - (uint32_t)key);
     int x1, y1, z1;
-    fetch(i1, x1, y1, z1);
+    hull_fetch<PPL, NW>(sb, px, py, pz, i1, x1, y1, z1);
 
     const int ex = x1 - x0, ey = y1 - y0, ez = z1 - z0;
     key = 0;
@@ -473,10 +493,10 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         }
     }
     key = block_max_u64<NW>(key, sb);
-    if ((key >> 32) == 0) { res.status = HULL_DEGENERATE; return res; }
+    if ((key >> 32) == 0) return false;
     int i2 = (int)(0xFFFFFFFFu - (uint32_t)key);
     int x2, y2, z2;
-    fetch(i2, x2, y2, z2);
+    hull_fetch<PPL, NW>(sb, px, py, pz, i2, x2, y2, z2);
 
     const s4v s0 = mk_s4(x0, y0, z0, 0);
     const s4v s1 = mk_s4(x1, y1, z1, 0);
@@ -493,10 +513,10 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         }
     }
     key = block_max_u64<NW>(key, sb);
-    if ((key >> 32) == 0) { res.status = HULL_DEGENERATE; return res; }
+    if ((key >> 32) == 0) return false;
     const int i3 = (int)(0xFFFFFFFFu - (uint32_t)key);
     int x3, y3, z3;
-    fetch(i3, x3, y3, z3);
+    hull_fetch<PPL, NW>(sb, px, py, pz, i3, x3, y3, z3);
     if (orient_exact(s0, s1, s2, x3, y3, z3) < 0.0) {  // make (p0,p1,p2,p3) positively oriented
         int t = i1; i1 = i2; i2 = t;
         t = x1; x1 = x2; x2 = t;
@@ -544,6 +564,27 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
                 }
             }
         }
+    }
+    return true;
+}
+
+// Cooperative exact quickhull over NW > 1 waves (blockDim.x == 64*NW).
+// px/py/pz: grid coords of local points i = k*T + tid (valid iff i < n), T = 64*NW.
+template <int PPL, int AS, int NW, bool MULTI = false>
+__device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBlockLDS* sb, int n, const int (&px)[PPL],
+                                      const int (&py)[PPL], const int (&pz)[PPL]) {
+    static_assert(NW > 1, "one wave: wave_quickhull");
+    constexpr int T = 64 * NW;
+    const int tid = threadIdx.x;
+    const int VC = w.VC, FC = w.FC;
+    int conf[PPL];
+    float dist[PPL];
+    HullResult res{HULL_OK, 0, 0};
+
+    auto pick = [&](const int (&a)[PPL], int slot) { return hull_pick(a, slot); };
+    if (!hull_simplex<PPL, AS, NW>(w, sb, n, px, py, pz, conf, dist)) {
+        res.status = HULL_DEGENERATE;
+        return res;
     }
 
     int nvert = 4, ftop = 4, nfree = 0;
@@ -1007,19 +1048,12 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         int qx, qy, qz, f0 = 0;
         {
             const int own = ip % T, slot = ip / T;
-            if (NW == 1) {
-                qx = read_lane(pick(px, slot), own);
-                qy = read_lane(pick(py, slot), own);
-                qz = read_lane(pick(pz, slot), own);
-                f0 = read_lane(pick(conf, slot), own);
-            } else {
-                if (tid == own) {
-                    sb->bc[0] = pick(px, slot); sb->bc[1] = pick(py, slot); sb->bc[2] = pick(pz, slot);
-                    sb->bc[3] = pick(conf, slot);
-                }
-                __syncthreads();
-                qx = sb->bc[0]; qy = sb->bc[1]; qz = sb->bc[2]; f0 = sb->bc[3];
+            if (tid == own) {
+                sb->bc[0] = pick(px, slot); sb->bc[1] = pick(py, slot); sb->bc[2] = pick(pz, slot);
+                sb->bc[3] = pick(conf, slot);
             }
+            __syncthreads();
+            qx = sb->bc[0]; qy = sb->bc[1]; qz = sb->bc[2]; f0 = sb->bc[3];
             // the apex leaves the conflict sets
 #pragma unroll
             for (int k = 0; k < PPL; ++k) {
@@ -1063,10 +1097,9 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
             head += cnt;
             __syncthreads();
             nvis = w.ctr[0];
-            if (NW == 1) nvis = uniform(nvis);
             // waves run independently: nobody may append to ctr[0] in the next
             // round before every wave has read this round's count
-            if (NW > 1) __syncthreads();
+            __syncthreads();
         }
 
         // ---- horizon edges (visible face -> non-visible neighbour) ---------
@@ -1094,7 +1127,6 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         }
         __syncthreads();
         int nhz = w.ctr[1];
-        if (NW == 1) nhz = uniform(nhz);
         if (nhz > VC || nhz < 3) { res.status = HULL_OVERFLOW; break; }
 
         // ---- face ids for the cone: reuse visible ids, then free list, then top
@@ -1173,6 +1205,250 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
     res.ftop = ftop;
     __syncthreads();
     return res;
+}
+
+// Exact quickhull on one wave, workspace (HULL_WS_WAVE) in LDS.
+//
+// A step inserts the conflict point of the largest key: its quantised height
+// above its face, then its index inverted in the low bits (points that
+// quantise to one position have one height, and the lowest index stands for
+// them). The visible region is found by
+// testing every face (lane l tests faces l, l + 64, ...; the planes of dead
+// faces are below every point): on a convex polytope the faces strictly below
+// the apex are exactly the region a walk from the conflict face would reach,
+// and one pass of independent LDS reads replaces the walk's four to five
+// dependent levels. Then the step goes lane per visible face, lane per
+// horizon edge, lane per point to re-home, with positions from ballots. LDS
+// operations of one wave complete in order, so the phases are only fenced
+// against compiler reordering.
+//
+// One wave issues an instruction every 8 to 9 cycles here, so the step is
+// bound by its instruction count as much as by its LDS round trips: neighbour
+// links carry the neighbour's edge slot (no second read to find it), a horizon
+// edge is one 8-byte record, point coordinates live in LDS (a slot chosen at
+// run time is a read, not a select chain over registers), loops are
+// wave-uniform, and the exact predicate is one rarely taken branch per pass.
+template <int PPL>
+__device__ __forceinline__ HullResult wave_quickhull(const HullWS<AS_LDS> w, HullBlockLDS* sb, int n,
+                                                     const int (&px)[PPL], const int (&py)[PPL],
+                                                     const int (&pz)[PPL]) {
+    const int lane = threadIdx.x;
+    const int VC = w.VC, FC = w.FC;
+    constexpr uint32_t IM = 64u * PPL - 1u;
+    static_assert((PPL & (PPL - 1)) == 0 && PPL <= 16, "keys hold the point index in their low bits");
+    HullResult res{HULL_OK, 0, 0};
+    auto order = [] {
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    auto mkkey = [&](float t, int k) {
+        return (__float_as_uint(fmaxf(t, 1e-6f)) & ~IM) | (IM - (uint32_t)(k * 64 + lane));
+    };
+    int conf[PPL];      // conflict face (any face where the key is 0)
+    uint32_t key[PPL];  // 0: inside, or a vertex
+    {
+        float dist[PPL];
+        if (!hull_simplex<PPL, AS_LDS, 1>(w, sb, n, px, py, pz, conf, dist)) {
+            res.status = HULL_DEGENERATE;
+            return res;
+        }
+#pragma unroll
+        for (int k = 0; k < PPL; ++k) {
+            key[k] = conf[k] >= 0 ? mkkey(dist[k], k) : 0u;
+            conf[k] = max(conf[k], 0);
+            w.pq[k * 64 + lane] = mk_s4(px[k], py[k], pz[k], 0);
+        }
+    }
+    if (lane < 4) {  // links of the tetrahedron: (neighbour << 2) | its edge slot
+        const u4v nb = w.fn[lane];
+        const int gg[3] = {nb.x, nb.y, nb.z};
+        int link[3];
+#pragma unroll
+        for (int e = 0; e < 3; ++e) {
+            const u4v gn = w.fn[gg[e]];
+            link[e] = (gg[e] << 2) | ((gn.x == lane) ? 0 : ((gn.y == lane) ? 1 : 2));
+        }
+        order();
+        w.fn[lane] = mk_u4(link[0], link[1], link[2], 1);
+    }
+    order();
+    const f4v dead = mk_f4(0.0f, 0.0f, 0.0f, -1.0f);
+    int nvert = 4, ftop = 4, nfree = 0;
+    for (;;) {
+        uint32_t sk = key[0];
+#pragma unroll
+        for (int k = 1; k < PPL; ++k) sk = max(sk, key[k]);
+        sk = wave_max_u32(sk);
+        if (sk == 0) break;
+        if (nvert >= VC) { res.status = HULL_OVERFLOW; break; }
+        const int ip = (int)(IM - (sk & IM)), vid = nvert++;
+        const s4v q = w.pq[ip];
+        const float fqx = (float)q.x, fqy = (float)q.y, fqz = (float)q.z;
+#pragma unroll
+        for (int k = 0; k < PPL; ++k) key[k] = key[k] == sk ? 0u : key[k];  // the apex leaves (keys differ)
+        if (lane == 0) {
+            w.vq[vid] = q;
+            w.vpid[vid] = ip;
+        }
+        // every face's visibility, and the visible faces in face order
+        int nvis = 0;
+        for (int b = 0; b < ftop; b += 64) {
+            const int f = b + lane;
+            const f4v pl = w.fpl[min(f, FC - 1)];
+            const float t = fmaf(pl.x, fqx, fmaf(pl.y, fqy, fmaf(pl.z, fqz, pl.w)));
+            bool v = t > HULL_FILTER_EPS;
+            const bool amb = fabsf(t) <= HULL_FILTER_EPS && f < ftop;
+            if (ballot(amb) && amb) {
+                const u4v c = w.fv[f];
+                v = orient_exact(w.vq[c.x], w.vq[c.y], w.vq[c.z], q.x, q.y, q.z) > 0.0;
+            }
+            v = v && f < ftop;
+            const uint64_t m = ballot(v);
+            w.fvis[f] = v ? 1 : 0;  // the array is padded to whole waves
+            if (v) w.vis[nvis + mask_rank(m)] = (uint16_t)f;
+            nvis += __popcll(m);
+        }
+        order();
+        // horizon edges (visible face -> non-visible neighbour), by slot
+        int nhz = 0;
+        for (int b = 0; b < nvis; b += 64) {
+            const bool act = b + lane < nvis;
+            const int f = w.vis[act ? b + lane : 0];
+            const u4v fvl = w.fv[f], nb = w.fn[f];
+            const int vv[4] = {fvl.x, fvl.y, fvl.z, fvl.x}, lk[3] = {nb.x, nb.y, nb.z};
+            const uint8_t g0 = w.fvis[lk[0] >> 2], g1 = w.fvis[lk[1] >> 2], g2 = w.fvis[lk[2] >> 2];
+            const bool h[3] = {act && !g0, act && !g1, act && !g2};
+#pragma unroll
+            for (int e = 0; e < 3; ++e) {
+                const uint64_t m = ballot(h[e]);
+                const int s = nhz + mask_rank(m);
+                if (h[e] && s < VC) {
+                    w.hz[s] = mk_u4(vv[e], vv[e + 1], lk[e], 0);
+                    w.smap[vv[e]] = (uint16_t)s;
+                    w.emap[vv[e + 1]] = (uint16_t)s;
+                }
+                nhz += __popcll(m);
+            }
+        }
+        if (nhz > VC || nhz < 3) { res.status = HULL_OVERFLOW; break; }
+        // face ids for the cone: the visible ids, then the free list, then
+        // the top; surplus visible faces die and go back to the free list
+        const int extra = nhz > nvis ? nhz - nvis : 0;
+        const int from_free = min(extra, nfree);
+        const int from_top = extra - from_free;
+        if (ftop + from_top > FC) { res.status = HULL_OVERFLOW; break; }
+        order();
+        for (int b = 0; b < max(nhz, nvis); b += 64) {
+            const int j = b + lane, over = j - nvis;
+            const int f = w.vis[min(j, nvis - 1)];
+            const int fr = w.ffree[max(nfree - 1 - max(over, 0), 0)];
+            const int id = over < 0 ? f : (over < from_free ? fr : ftop + over - from_free);
+            if (j < nhz) {
+                w.hnew[j] = (uint16_t)id;
+            } else if (j < nvis) {
+                w.ffree[nfree - from_free + (j - nhz)] = (uint16_t)f;
+                w.fn[f] = mk_u4(0, 0, 0, 0);
+                w.fpl[f] = dead;
+            }
+        }
+        nfree = nfree - from_free + (nvis > nhz ? nvis - nhz : 0);
+        ftop += from_top;
+        order();
+        // stitch the cone
+        for (int b = 0; b < nhz; b += 64) {
+            const int j = b + lane, jj = j < nhz ? j : 0;
+            const u4v h = w.hz[jj];
+            const int id = w.hnew[jj], js = w.smap[h.y], je = w.emap[h.x];
+            const s4v qa = w.vq[h.x], qc = w.vq[h.y];
+            const int ns = w.hnew[js], ne = w.hnew[je];
+            if (j < nhz) {
+                const f4v p = face_set_plane(w, id, qa, qc, q);
+                w.fv[id] = mk_u4(h.x, h.y, vid, 0);
+                w.fn[id] = mk_u4(h.z, (ns << 2) | 2, (ne << 2) | 1, 1);
+                *(((asptr<AS_LDS, uint16_t>)&w.fn[h.z >> 2]) + (h.z & 3)) = (uint16_t)(id << 2);
+                if (j < WAVE_CPL) w.cpl[j] = p;
+            } else if (j < WAVE_CPL) {
+                w.cpl[j] = dead;  // scans go four planes at a time
+            }
+        }
+        order();
+        // points of the replaced faces (their visibility byte is still set)
+        // move to the cone: each lane's as a bit mask, so the wave loops as
+        // often as its busiest lane needs
+        uint32_t need = 0;
+#pragma unroll
+        for (int k = 0; k < PPL; ++k) {
+            const uint32_t dv = w.fvis[conf[k]];
+            need |= (key[k] ? dv : 0u) << k;
+        }
+        while (ballot(need != 0)) {
+            const bool act = need != 0;
+            const int k = act ? __ffs(need) - 1 : 0;
+            need &= need - 1;
+            const s4v p = w.pq[k * 64 + lane];
+            const float fx = (float)p.x, fy = (float)p.y, fz = (float)p.z;
+            int bj = -1;
+            float bd = HULL_FILTER_EPS, near = 1.0f;
+            if (nhz <= WAVE_CPL) {
+                for (int j = 0; j < nhz; j += 4) {
+                    f4v c[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) c[u] = w.cpl[j + u];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const float t = fmaf(c[u].x, fx, fmaf(c[u].y, fy, fmaf(c[u].z, fz, c[u].w)));
+                        near = fminf(near, fabsf(t));
+                        bj = t > bd ? j + u : bj;
+                        bd = fmaxf(bd, t);
+                    }
+                }
+            } else {
+                near = 0.0f;
+            }
+            const bool amb = act && near <= HULL_FILTER_EPS;
+            if (ballot(amb) && amb) {  // some test is within the filter's error: decide all exactly
+                bj = -1;
+                for (int j = 0; j < nhz; ++j) {
+                    const int id = w.hnew[j];
+                    float t;
+                    if (face_above(w, id, p.x, p.y, p.z, &t) && (bj < 0 || t > bd)) {
+                        bj = j;
+                        bd = t;
+                    }
+                }
+            }
+            const int best = w.hnew[max(bj, 0)];
+            const uint32_t nk = bj >= 0 ? mkkey(bd, k) : 0u;
+#pragma unroll
+            for (int kk = 0; kk < PPL; ++kk)
+                if (act && kk == k) {
+                    conf[kk] = best;
+                    key[kk] = nk;
+                }
+        }
+    }
+    if (res.status == HULL_OK) {  // plain neighbour ids for what follows
+        for (int f = lane; f < ftop; f += 64) {
+            u4v t = w.fn[f];
+            t.x >>= 2;
+            t.y >>= 2;
+            t.z >>= 2;
+            w.fn[f] = t;
+        }
+    }
+    res.nvert = nvert;
+    res.ftop = ftop;
+    __syncthreads();
+    return res;
+}
+
+// Quickhull on NW waves: one wave has its own step, several share the block's.
+template <int PPL, int AS, int NW, bool MULTI = false>
+__device__ __forceinline__ HullResult hull_quickhull(const HullWS<AS> w, HullBlockLDS* sb, int n,
+                                                     const int (&px)[PPL], const int (&py)[PPL],
+                                                     const int (&pz)[PPL]) {
+    if constexpr (NW == 1) return wave_quickhull<PPL>(w, sb, n, px, py, pz);
+    else return block_quickhull<PPL, AS, NW, MULTI>(w, sb, n, px, py, pz);
 }
 
 // After block_quickhull: mark referenced vertices and give them output

@@ -153,7 +153,7 @@ __device__ __forceinline__ void hull_item(const HullItemArgs& a, int mode, int i
         }
     }
 
-    HullResult r = block_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
+    HullResult r = hull_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
     if (r.status == HULL_OVERFLOW) {
         if (tid == 0) {
             if (mode == 0) a.out_err[cloud] = KERR_HULL_CAPACITY;
@@ -217,7 +217,7 @@ __global__ __launch_bounds__(64) void hull_wave_kernel(HullItemArgs a, int mode)
     const int item = blockIdx.x;
     if (item >= a.n_items) return;
     // compile-time capacities: every sub-array address folds into ds offsets
-    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, 64 * PPL, 64 * PPL), &sb, &hb);
+    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, 64 * PPL, 64 * PPL, HULL_WS_WAVE), &sb, &hb);
     hull_item<PPL, AS_LDS, 1>(a, mode, item, w, &sb);
 }
 
@@ -277,7 +277,7 @@ int launch_wave(gpu_ctx_t ctx, HullItemArgs a, int maxn, int mode) {
     else { ppl = 16; k = hull_wave_kernel<16>; }
     a.VC = 64 * ppl;
     a.NP = 64 * ppl;
-    const unsigned lds = hull_ws_bytes<AS_LDS>(a.VC, a.NP);
+    const unsigned lds = hull_ws_bytes<AS_LDS>(a.VC, a.NP, HULL_WS_WAVE);
     if (lds > 65536u)
         HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipLaunchKernelGGL(k, dim3(a.n_items), dim3(64), lds, ctx->stream, a, mode);

@@ -97,10 +97,10 @@ __device__ __forceinline__ bool la_hull_item(LaHullTask& t, const HullWS<AS> w, 
         // multi-apex rounds (the workspace was carved or attached with their
         // scratch; the four-wave tiers keep single-apex steps and do not
         // compile them); the point index field of their keys holds 14 bits
-        if (multi && n <= PPL * T) r = block_quickhull<PPL, AS, NW, true>(w, sb, n, px, py, pz);
-        else r = block_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
+        if (multi && n <= PPL * T) r = hull_quickhull<PPL, AS, NW, true>(w, sb, n, px, py, pz);
+        else r = hull_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
     } else {
-        r = block_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
+        r = hull_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
     }
     if (r.status == HULL_OVERFLOW && retry) {
         if (tid == 0) {
@@ -176,7 +176,7 @@ __global__ __launch_bounds__(64) void la_hull_wave(LaHullTask* tasks, const int*
     // ids[0, n), or the first min(*dcount, n) when the count is on the device
     if ((int)blockIdx.x >= (dcount ? min(*dcount, n) : n)) return;
     LaHullTask& t = tasks[ids[blockIdx.x]];
-    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, 64 * PPL, 64 * PPL), &sb, &hb);
+    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, 64 * PPL, 64 * PPL, HULL_WS_WAVE), &sb, &hb);
     la_hull_item<PPL, AS_LDS, 1>(t, w, &sb, pool, err);
     if (threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
 }
@@ -360,14 +360,13 @@ __global__ __launch_bounds__(64) void la_kdop_ext_kernel(LaHullTask* tasks, cons
 // insertion's transient pair). A smaller workspace fits more of these
 // one-wave workgroups on a CU (14 at 11.5 KB of LDS each).
 constexpr int KD_VC = KD_NE;
-constexpr unsigned KD_WS = 9776;  // LDS of its workspace (la_launch_kdop checks the size)
+constexpr unsigned KD_WS = 11920;  // LDS of its workspace (la_launch_kdop checks the size)
 __global__ __launch_bounds__(64) void la_kdop_rough_kernel(LaHullTask* tasks, const int* ids, int n,
                                                            const int* dcount, KdopRec* rec, int2* res) {
     __shared__ HullBlockLDS sb;
     __shared__ HullBits<KD_NE> hb;
     __shared__ __align__(16) char lds[KD_WS];
     __shared__ float ep[KD_NE][3];
-    __shared__ int s_npl;
     if ((int)blockIdx.x >= (dcount ? min(*dcount, n) : n)) return;
     LaHullTask& t = tasks[ids[blockIdx.x]];
     KdopRec& R = rec[blockIdx.x];
@@ -375,7 +374,7 @@ __global__ __launch_bounds__(64) void la_kdop_rough_kernel(LaHullTask* tasks, co
     const int np = t.n;
     for (int i = tid; i < 3 * KD_NE; i += 64) (&ep[0][0])[i] = (&R.ep[0][0])[i];
     __syncthreads();
-    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, KD_VC, KD_VC), &sb, &hb);
+    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, KD_VC, 128, HULL_WS_WAVE), &sb, &hb);
     float emn[3] = {1e30f, 1e30f, 1e30f}, emx[3] = {-1e30f, -1e30f, -1e30f};
     for (int i = 0; i < KD_NE; ++i)
         for (int j = 0; j < 3; ++j) { emn[j] = fminf(emn[j], ep[i][j]); emx[j] = fmaxf(emx[j], ep[i][j]); }
@@ -393,7 +392,7 @@ __global__ __launch_bounds__(64) void la_kdop_rough_kernel(LaHullTask* tasks, co
         }
     }
     const QFrame full = R.full;
-    HullResult r = block_quickhull<2, AS_LDS, 1>(w, &sb, KD_NE, px, py, pz);
+    HullResult r = hull_quickhull<2, AS_LDS, 1>(w, &sb, KD_NE, px, py, pz);
     HullCanon rc;
     rc.nt = 0;
     if (r.status == HULL_OK) {
@@ -427,18 +426,21 @@ __global__ __launch_bounds__(64) void la_kdop_rough_kernel(LaHullTask* tasks, co
         }
     }
     // the live faces (hull_canon marks them), in face-id order
-    if (tid == 0) {
-        int c = 0;
-        for (int f = 0; f < r.ftop && c < KD_MAXPL; ++f) {
-            if (!(w.fvis[f] & 16)) continue;
-            const u4v fv = w.fv[f];
-            R.face[c][0] = (unsigned char)w.vpid[fv.x];
-            R.face[c][1] = (unsigned char)w.vpid[fv.y];
-            R.face[c][2] = (unsigned char)w.vpid[fv.z];
-            ++c;
+    int c = 0;
+    for (int b = 0; b < r.ftop; b += 64) {
+        const bool on = b + tid < r.ftop && (w.fvis[min(b + tid, r.ftop - 1)] & 16);
+        const uint64_t m = ballot(on);
+        const int o = c + mask_rank(m);
+        if (on && o < KD_MAXPL) {
+            const u4v fv = w.fv[b + tid];
+            R.face[o][0] = (unsigned char)w.vpid[fv.x];
+            R.face[o][1] = (unsigned char)w.vpid[fv.y];
+            R.face[o][2] = (unsigned char)w.vpid[fv.z];
         }
-        s_npl = c;
-        R.npl = c;
+        c += __popcll(m);
+    }
+    if (tid == 0) {
+        R.npl = min(c, KD_MAXPL);
         R.status = 0;
     }
 }
@@ -549,7 +551,7 @@ __global__ __launch_bounds__(KD_T) void la_kdop_filter_kernel(LaHullTask* tasks,
 int la_launch_kdop(gpu_ctx_t ctx, LaHullTask* d_tasks, const int* d_ids, int n, const int* dcount, int2* d_res,
                    KdopRec* d_rec, hipStream_t s) {
     if (n <= 0) return 0;
-    REQUIRE(hull_ws_bytes<AS_LDS>(KD_VC, KD_VC) <= KD_WS, "k-DOP rough hull workspace exceeds its LDS");
+    REQUIRE(hull_ws_bytes<AS_LDS>(KD_VC, 128, HULL_WS_WAVE) <= KD_WS, "k-DOP rough hull workspace exceeds its LDS");
     hipLaunchKernelGGL(la_kdop_ext_kernel, dim3((unsigned)n), dim3(64), 0, s, d_tasks, d_ids, n, dcount, d_rec);
     HIP_TRY(hipGetLastError());
     hipLaunchKernelGGL(la_kdop_rough_kernel, dim3((unsigned)n), dim3(64), 0, s, d_tasks, d_ids, n, dcount, d_rec,
@@ -1645,7 +1647,7 @@ int launch_wave_ids(HullCall& hc, int sk, LaHullTask* d_tasks, const int* d_ids,
     }
     WaveFn k = ppl == 1 ? la_hull_wave<1> : ppl == 2 ? la_hull_wave<2> : ppl == 4 ? la_hull_wave<4>
              : ppl == 8 ? la_hull_wave<8> : la_hull_wave<16>;
-    const unsigned lds = hull_ws_bytes<AS_LDS>(64 * ppl, 64 * ppl);
+    const unsigned lds = hull_ws_bytes<AS_LDS>(64 * ppl, 64 * ppl, HULL_WS_WAVE);
     if (lds > 65536u)
         HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
     hipStream_t s;

@@ -1,7 +1,7 @@
 // wave.hpp - wave64 primitives for gfx950 (CDNA4).
 //
 // Every kernel in this library is written for 64-lane wavefronts: ballots are
-// 64-bit masks, reductions are 6 butterfly steps, and a single-wave workgroup
+// 64-bit masks, reductions and scans are 6 DPP steps, and a single-wave workgroup
 // uses the LDS as wave-private memory with __syncthreads() as its fence.
 #pragma once
 #include <hip/hip_runtime.h>
@@ -30,37 +30,72 @@ __device__ __forceinline__ float read_lane(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
 
+// Wave-wide reductions and scans on DPP: four row_shr steps inside the rows of
+// 16 lanes, then row_bcast 15 and 31 across them, so lane 63 ends with the
+// whole wave's value. Each step is one VALU operation; the same butterfly on
+// __shfl_xor goes through the LDS crossbar (ds_bpermute, about 130 cycles a
+// step: 64-bit keys cost 12 of them, 0.8k cycles of a hull insertion's 1.2k
+// selection). All 64 lanes have to be active. Lanes without a source keep
+// `old`. FP64 and FP32 sums stay on the butterfly: their bits depend on the
+// order of the additions.
+template <int CTRL, int ROWS> __device__ __forceinline__ int dpp_i(int old, int v) {
+    return __builtin_amdgcn_update_dpp(old, v, CTRL, ROWS, 0xf, false);
+}
+constexpr int DPP_SHR1 = 0x111, DPP_SHR2 = 0x112, DPP_SHR4 = 0x114, DPP_SHR8 = 0x118, DPP_BC15 = 0x142, DPP_BC31 = 0x143;
+
+// idempotent operations: a lane without a source combines with itself
+template <class Op> __device__ __forceinline__ int wave_reduce_idem(int v, Op op) {
+    v = op(v, dpp_i<DPP_SHR1, 0xf>(v, v));
+    v = op(v, dpp_i<DPP_SHR2, 0xf>(v, v));
+    v = op(v, dpp_i<DPP_SHR4, 0xf>(v, v));
+    v = op(v, dpp_i<DPP_SHR8, 0xf>(v, v));
+    v = op(v, dpp_i<DPP_BC15, 0xa>(v, v));
+    v = op(v, dpp_i<DPP_BC31, 0xc>(v, v));
+    return read_lane(v, 63);
+}
+// 0 is the identity, so each step folds into one v_max_u32 with DPP operand
+__device__ __forceinline__ uint32_t wave_max_u32(uint32_t v) {
+    v = max(v, (uint32_t)dpp_i<DPP_SHR1, 0xf>(0, (int)v));
+    v = max(v, (uint32_t)dpp_i<DPP_SHR2, 0xf>(0, (int)v));
+    v = max(v, (uint32_t)dpp_i<DPP_SHR4, 0xf>(0, (int)v));
+    v = max(v, (uint32_t)dpp_i<DPP_SHR8, 0xf>(0, (int)v));
+    v = max(v, (uint32_t)dpp_i<DPP_BC15, 0xa>(0, (int)v));
+    v = max(v, (uint32_t)dpp_i<DPP_BC31, 0xc>(0, (int)v));
+    return (uint32_t)read_lane((int)v, 63);
+}
+__device__ __forceinline__ uint32_t wave_min_u32(uint32_t v) {
+    return (uint32_t)wave_reduce_idem((int)v, [](int a, int b) { return (int)min((uint32_t)a, (uint32_t)b); });
+}
+// 64-bit: the high words, then the low words of the lanes that hold the best one
 __device__ __forceinline__ uint64_t wave_max_u64(uint64_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        uint64_t w = __shfl_xor(v, o);
-        v = w > v ? w : v;
-    }
-    return v;
+    const uint32_t hi = wave_max_u32((uint32_t)(v >> 32));
+    const uint32_t lo = wave_max_u32((uint32_t)(v >> 32) == hi ? (uint32_t)v : 0u);
+    return ((uint64_t)hi << 32) | lo;
 }
 __device__ __forceinline__ uint64_t wave_min_u64(uint64_t v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) {
-        uint64_t w = __shfl_xor(v, o);
-        v = w < v ? w : v;
-    }
-    return v;
+    const uint32_t hi = wave_min_u32((uint32_t)(v >> 32));
+    const uint32_t lo = wave_min_u32((uint32_t)(v >> 32) == hi ? (uint32_t)v : ~0u);
+    return ((uint64_t)hi << 32) | lo;
 }
 __device__ __forceinline__ float wave_min_f(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fminf(v, __shfl_xor(v, o));
-    return v;
+    return __int_as_float(wave_reduce_idem(
+        __float_as_int(v), [](int a, int b) { return __float_as_int(fminf(__int_as_float(a), __int_as_float(b))); }));
 }
 __device__ __forceinline__ float wave_max_f(float v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v = fmaxf(v, __shfl_xor(v, o));
+    return __int_as_float(wave_reduce_idem(
+        __float_as_int(v), [](int a, int b) { return __float_as_int(fmaxf(__int_as_float(a), __int_as_float(b))); }));
+}
+// Inclusive prefix sum across the wave.
+__device__ __forceinline__ int wave_incl_scan(int v) {
+    v += dpp_i<DPP_SHR1, 0xf>(0, v);
+    v += dpp_i<DPP_SHR2, 0xf>(0, v);
+    v += dpp_i<DPP_SHR4, 0xf>(0, v);
+    v += dpp_i<DPP_SHR8, 0xf>(0, v);
+    v += dpp_i<DPP_BC15, 0xa>(0, v);
+    v += dpp_i<DPP_BC31, 0xc>(0, v);
     return v;
 }
-__device__ __forceinline__ int wave_sum_i(int v) {
-#pragma unroll
-    for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
+__device__ __forceinline__ int wave_sum_i(int v) { return read_lane(wave_incl_scan(v), 63); }
 __device__ __forceinline__ double wave_sum_d(double v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
@@ -69,17 +104,6 @@ __device__ __forceinline__ double wave_sum_d(double v) {
 __device__ __forceinline__ float wave_sum_f(float v) {
 #pragma unroll
     for (int o = 32; o > 0; o >>= 1) v += __shfl_xor(v, o);
-    return v;
-}
-
-// Inclusive prefix sum across the wave (Hillis-Steele over 64 lanes).
-__device__ __forceinline__ int wave_incl_scan(int v) {
-    const int l = lane_id();
-#pragma unroll
-    for (int o = 1; o < 64; o <<= 1) {
-        int w = __shfl_up(v, o);
-        if (l >= o) v += w;
-    }
     return v;
 }
 
