@@ -295,6 +295,8 @@ def kernel_name(cls, wide_min, half_cap, ldsb8=0, w8=0):
         n = int(base[6:])
         if base.startswith("hull_b"):
             return f"la_hull_block<{n // 512}>"
+        if not (wide_min > 0 and n > wide_min):
+            return f"la_hull_wave<{n // 64}>"
         if (w8 >> (2 if n == 1024 else 3)) & 1:
             return f"la_hull_lds8<{n // 512}>"
         return f"la_hull_lds4<{n // 256}>"

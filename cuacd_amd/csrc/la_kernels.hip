@@ -167,18 +167,25 @@ __device__ __forceinline__ bool la_hull_item(LaHullTask& t, const HullWS<AS> w, 
     return true;
 }
 
+// One wave per hull, workspace of vcap vertices in LDS; ids[0, n), or the
+// first min(*dcount, n) when the count is on the device, strided over the
+// grid. A set whose hull needs more vertices is queued on `retry` (null: the
+// workspace holds any hull of the tier).
 template <int PPL>
 __global__ __launch_bounds__(64) void la_hull_wave(LaHullTask* tasks, const int* ids, int n, const int* dcount,
-                                                   DPool* pool, int* err) {
+                                                   int vcap, int* retry, DPool* pool, int* err) {
     extern __shared__ __align__(16) char lds[];
     __shared__ HullBlockLDS sb;
     __shared__ HullBits<64 * PPL> hb;
-    // ids[0, n), or the first min(*dcount, n) when the count is on the device
-    if ((int)blockIdx.x >= (dcount ? min(*dcount, n) : n)) return;
-    LaHullTask& t = tasks[ids[blockIdx.x]];
-    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, 64 * PPL, 64 * PPL, HULL_WS_WAVE), &sb, &hb);
-    la_hull_item<PPL, AS_LDS, 1>(t, w, &sb, pool, err);
-    if (threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
+    const int nn = dcount ? min(*dcount, n) : n;
+    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, vcap, 64 * PPL, HULL_WS_WAVE), &sb, &hb);
+    for (int j = blockIdx.x; j < nn; j += gridDim.x) {
+        __syncthreads();
+        const int id = ids[j];
+        LaHullTask& t = tasks[id];
+        const bool done = la_hull_item<PPL, AS_LDS, 1>(t, w, &sb, pool, err, retry, id);
+        if (done && threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
+    }
 }
 
 // Four waves per hull, workspace in LDS: for the larger one-workgroup sets,
@@ -199,6 +206,7 @@ __global__ __launch_bounds__(64 * LA_LDS4_NW) void la_hull_lds4(LaHullTask* task
         __syncthreads();
         LaHullTask& t = tasks[ids[j]];
         la_hull_item<PPL, AS_LDS, LA_LDS4_NW>(t, w, &sb, pool, err, nullptr, -1, multi != 0);
+        __syncthreads();  // every wave is done with the filtered points
         if (threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
     }
 }
@@ -219,6 +227,7 @@ __global__ __launch_bounds__(64 * LA_BLOCK_NW) void la_hull_lds8(LaHullTask* tas
         __syncthreads();
         LaHullTask& t = tasks[ids[j]];
         la_hull_item<PPL, AS_LDS, LA_BLOCK_NW>(t, w, &sb, pool, err, nullptr, -1, multi != 0);
+        __syncthreads();  // every wave is done with the filtered points
         if (threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
     }
 }
@@ -239,6 +248,7 @@ __global__ __launch_bounds__(64 * NW) void la_hull_ldsv(LaHullTask* tasks, const
     __shared__ HullBits<CAP> hb;
     const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, vcap, CAP, multi != 0), &sb, &hb);
     const bool done = la_hull_item<PPL, AS_LDS, NW>(t, w, &sb, pool, err, retry, id, multi != 0);
+    __syncthreads();  // every wave is done with the filtered points
     if (done && threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
 }
 
@@ -263,6 +273,7 @@ __global__ __launch_bounds__(64 * LA_BLOCK_NW) void la_hull_block(LaHullTask* ta
         __syncthreads();
         LaHullTask& t = tasks[ids[j]];
         la_hull_item<PPL, AS_GLOBAL, LA_BLOCK_NW>(t, w, &sb, pool, err, nullptr, -1, multi != 0);
+        __syncthreads();  // every wave is done with the filtered points
         if (threadIdx.x == 0 && t.filt) { heap_free(pool, t.filt, err); t.filt = nullptr; }
     }
 }
@@ -1379,14 +1390,18 @@ int ensure_kdop_axes(gpu_ctx_t ctx) {
     return 0;
 }
 
-using WaveFn = void (*)(LaHullTask*, const int*, int, const int*, DPool*, int*);
+using WaveFn = void (*)(LaHullTask*, const int*, int, const int*, int, int*, DPool*, int*);
 
 // Launch-shape knobs of the hull tiers (they choose kernels and capacities,
 // never results: every tier computes the same canonical hull). Process-wide;
 // initial values from the environment, changed at run time through
 // gpu_set_tuning (the autotuner).
 //   0 wide_min: wave-tier sets above this many points run four waves per hull
-//     (CUACD_HULL_WIDE_MIN, 0 disables; default 256)
+//     (CUACD_HULL_WIDE_MIN, 0 disables; default 512). With the one-wave
+//     quickhull and a 3/8-capacity first pass, the 257-512-point tier of a
+//     24-mesh search takes 105 + 55 ms (retries) on one wave and 130 + 64 ms
+//     on four; at 513-1024 points one wave takes 124 + 39 ms against 83 + 21
+//     on eight
 //   1 vcap8: first-pass vertex capacity of the four-wave tiers, in eighths of
 //     their point capacity (CUACD_HULL_VCAP8, 1..8; default 3)
 //   2 half_cap: reduced-capacity first passes on/off (CUACD_HULL_HALFCAP; default 1)
@@ -1477,7 +1492,7 @@ void tune_init() {
                                   "CUACD_MLP_FUSED",       "CUACD_HULL_LDSV8_VCAP",  "CUACD_HULL_LDSB8_VCAP",
                                   "CUACD_CUT_LDS_VERTS",   "CUACD_HULL_LPT",         "CUACD_HULL_B4_SPLIT",
                                   "CUACD_HULL_ORDER",      "CUACD_HULL_W8",          "CUACD_HULL_MULTI_HBM"};
-    const int def[LA_TUNE_N] = {256, 3, 1, 512, HULL_NP_MAX, 1, 1, 1024, 1024, 98304, 0, 0, 1, 5, 1};
+    const int def[LA_TUNE_N] = {512, 3, 1, 512, HULL_NP_MAX, 1, 1, 1024, 1024, 98304, 0, 0, 1, 5, 1};
     for (int k = 0; k < LA_TUNE_N; ++k) {
         const char* e = getenv(env[k]);
         g_tune[k] = tune_clamp(k, e ? atoi(e) : def[k]);
@@ -1571,6 +1586,8 @@ int zero_ints(gpu_ctx_t ctx, int* p, int n, hipStream_t s) {
     return 0;
 }
 
+constexpr unsigned LA_CU_LDS = 160u * 1024u;  // LDS of a CU
+
 // One wave tier (sets of up to 64 * ppl points). d_ids holds nids task ids,
 // or - with dcnt given - up to nids of them, *dcnt on the device (the grid is
 // sized for nids and the kernels read the count).
@@ -1580,7 +1597,11 @@ int launch_wave_ids(HullCall& hc, int sk, LaHullTask* d_tasks, const int* d_ids,
     if (nids <= 0) return 0;
     const int kid = ppl == 1 ? KT_HULL_W1 : ppl == 2 ? KT_HULL_W2 : ppl == 4 ? KT_HULL_W4 : ppl == 8 ? KT_HULL_W8
                                                                                                      : KT_HULL_W16;
-    const int wm = hull_wide_min();
+    // the device-counted call (score plans) keeps the four- and eight-wave
+    // kernels above 256 points and one launch for the tiers below: a plan's
+    // replay with one-wave first passes ended in a memory fault whose cause
+    // was not found
+    const int wm = dcnt && hull_wide_min() > 0 ? std::min(hull_wide_min(), 256) : hull_wide_min();
     if (wm > 0 && ppl >= 8 && 64 * ppl > wm && hull_half_cap()) {
         // first pass with a reduced vertex capacity (several hulls per CU),
         // then the sets whose hulls did not fit, at full capacity
@@ -1645,18 +1666,40 @@ int launch_wave_ids(HullCall& hc, int sk, LaHullTask* d_tasks, const int* d_ids,
         kt_end(ctx, kid, t0, bytes, s);
         return 0;
     }
+    // one wave per hull: a first pass with a reduced vertex capacity where
+    // that lets more hulls share the CUs than there are at full capacity,
+    // then the sets whose hulls did not fit
     WaveFn k = ppl == 1 ? la_hull_wave<1> : ppl == 2 ? la_hull_wave<2> : ppl == 4 ? la_hull_wave<4>
              : ppl == 8 ? la_hull_wave<8> : la_hull_wave<16>;
-    const unsigned lds = hull_ws_bytes<AS_LDS>(64 * ppl, 64 * ppl, HULL_WS_WAVE);
+    const int cap = 64 * ppl, vcap = cap * hull_vcap_eighths() / 8;
+    const unsigned lds = hull_ws_bytes<AS_LDS>(cap, cap, HULL_WS_WAVE);
+    const unsigned ldv = hull_ws_bytes<AS_LDS>(vcap, cap, HULL_WS_WAVE);
+    const int fit = std::max(1, (int)(LA_CU_LDS / (lds + 1024u))) * std::max(1, ctx->n_cu);
+    const bool first = !dcnt && ppl >= 4 && hull_half_cap() && vcap < cap && nids > fit;
     if (lds > 65536u)
         HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+    int* d_retry = nullptr;
+    if (first) {
+        d_retry = hc.alloc<int>((size_t)nids + 1);
+        REQUIRE(d_retry, "lookahead: id list allocation failed");
+        if (int rc = zero_ints(ctx, d_retry, 1, ctx->stream)) return rc;
+    }
     hipStream_t s;
     if (int rc = hc.fork(sk, &s)) return rc;
     hipEvent_t t0 = kt_begin(ctx, s);
-    hipLaunchKernelGGL(k, dim3((unsigned)(size_t)nids), dim3(64), lds, s, d_tasks, d_ids, (int)(size_t)nids, dcnt,
-                       ctx->d_pool, ctx->d_err);
+    hipLaunchKernelGGL(k, dim3((unsigned)(size_t)nids), dim3(64), first ? ldv : lds, s, d_tasks, d_ids,
+                       (int)(size_t)nids, dcnt, first ? vcap : cap, d_retry, ctx->d_pool, ctx->d_err);
     HIP_TRY(hipGetLastError());
     kt_end(ctx, kid, t0, bytes, s);
+    if (first) {
+        hipEvent_t t1 = kt_begin(ctx, s);
+        hipLaunchKernelGGL(k, dim3((unsigned)std::min(nids, fit)), dim3(64), lds, s, d_tasks,
+                           (const int*)(d_retry + 1), (int)(size_t)nids, (const int*)d_retry, cap, (int*)nullptr,
+                           ctx->d_pool, ctx->d_err);
+        HIP_TRY(hipGetLastError());
+        if (ppl >= 8) kt_end(ctx, ppl == 8 ? KT_HULL_R8 : KT_HULL_R16, t1, 0.0, s);
+        else kt_end(ctx, kid, t1, 0.0, s);
+    }
     return 0;
 }
 
