@@ -40,6 +40,20 @@ void* cuacd::stage_buf(gpu_ctx_t ctx, int slot, size_t bytes) {
     return ctx->stage[slot];
 }
 
+char* cuacd::pinned_stage(gpu_ctx_t ctx, size_t bytes) {
+    if (bytes <= ctx->la_pinned_cap) return ctx->la_pinned;
+    if (ctx->la_pinned) (void)hipHostFree(ctx->la_pinned);
+    ctx->la_pinned = nullptr;
+    ctx->la_pinned_cap = 0;
+    const size_t cap = bytes + bytes / 2 > ((size_t)1 << 20) ? bytes + bytes / 2 : (size_t)1 << 20;
+    if (hipHostMalloc((void**)&ctx->la_pinned, cap, hipHostMallocDefault) != hipSuccess) {
+        ctx->la_pinned = nullptr;
+        return nullptr;
+    }
+    ctx->la_pinned_cap = cap;
+    return ctx->la_pinned;
+}
+
 hipEvent_t cuacd::kt_begin(gpu_ctx_t ctx, hipStream_t s) {
     KTimers* k = ctx->kt;
     if (!k) return nullptr;

@@ -81,6 +81,10 @@ void set_error(gpu_ctx_t ctx, const char* fmt, ...);
 // Grow-only device staging buffer `slot` of at least `bytes`.
 void* stage_buf(gpu_ctx_t ctx, int slot, size_t bytes);
 
+// Pinned host staging of at least `bytes` (grow-only, the context's); null
+// when it cannot be had.
+char* pinned_stage(gpu_ctx_t ctx, size_t bytes);
+
 // Read the kernel error word written by the last launches (synchronises) and
 // clear it. Applies host-injected bits. Returns the word.
 int read_and_clear_err(gpu_ctx_t ctx);

@@ -3,26 +3,36 @@
 // Backs gpu_hull_dandc / batch_hull_volume / batch_hull_dandc_mesh
 // (reference: csrc/test.c:95-160, cuda/test_hull_dandc.cu:24-77).
 //
-// Three tiers, all exact on the same quantization grid:
-//   * clouds of <= 1024 points: one wave64 workgroup, points in registers,
-//     workspace in LDS (hull_wave_kernel);
-//   * clouds of <= 16384 points: eight waves, points in registers, workspace
-//     in global memory (hull_block_kernel);
+// Size tiers, all exact on the same quantization grid:
+//   * clouds of <= 512 points: one wave64 workgroup, workspace in LDS
+//     (hull_wave_kernel, by the largest such cloud's size);
+//   * clouds of <= 4096 points: eight waves with multi-apex rounds and an LDS
+//     workspace of 384 (up to 1024 points) or 1024 vertices (hull_lds_kernel);
+//     hulls with more corners are redone with a larger workspace;
+//   * clouds of <= 16384 points: the same rounds with the workspace in global
+//     memory (hull_block_kernel), one class per factor of two;
 //   * larger clouds: divide and conquer - chunks of 1024 points are hulled
 //     independently on the cloud's grid, the union of their hull vertices
 //     (kept in ascending input order, so lowest-index duplicate resolution is
 //     preserved) replaces the cloud, until the block kernel can finish it.
+// Every tier's launch covers all items and leaves those of other sizes alone
+// (the sizes are on the device); the tiers above 1024 points run on the
+// context's side streams beside the small ones, so a call lasts as long as
+// its slowest cloud. With one kernel per 1024-point bound sized for the
+// largest cloud and single-apex steps, 192 clouds of 5-12000 points (balls,
+// spheres, lattices) took 200 ms.
 #include <stdlib.h>
+#include <string.h>
 #include <algorithm>
 #include <vector>
-#include "ctx.hpp"
-#include "hull.hpp"
+#include "lookahead.hpp"
 
 using namespace cuacd;
 
 namespace {
 
-constexpr int WAVE_MAX = 1024;    // points per cloud for the one-wave tier
+constexpr int WAVE_MAX = 1024;    // points per cloud one wave can hull
+constexpr int WAVE_TIER = 512;    // points per cloud for the one-wave tier
 constexpr int BLOCK_NW = 8;       // waves of the block tier
 constexpr int BLOCK_MAX = 16384;  // points per cloud for the block tier
 constexpr int CHUNK = 1024;
@@ -38,6 +48,9 @@ struct HullItemArgs {
     int VC;                  // vertex capacity of the workspace
     int NP;                  // point capacity of the workspace
     int min_n, max_n;        // items outside [min_n, max_n] are left to another tier
+    const int* list;         // optional item list: list[0, min(*list_n, n_items))
+    const int* list_n;
+    int* retry;              // optional: items whose hull exceeds VC are queued here (count first)
     char* gws;               // global workspaces (block tier), gws_stride bytes each
     unsigned long long gws_stride;
     // mesh output (mode 0), indexed by cloud
@@ -53,7 +66,7 @@ struct HullItemArgs {
     int* out_cnt;
 };
 
-template <int PPL, int AS, int NW>
+template <int PPL, int AS, int NW, bool MULTI = false>
 __device__ __forceinline__ void hull_item(const HullItemArgs& a, int mode, int item, const HullWS<AS> w,
                                           HullBlockLDS* sb) {
     constexpr int T = 64 * NW;
@@ -153,9 +166,11 @@ __device__ __forceinline__ void hull_item(const HullItemArgs& a, int mode, int i
         }
     }
 
-    HullResult r = hull_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
+    HullResult r = hull_quickhull<PPL, AS, NW, MULTI>(w, sb, n, px, py, pz);
     if (r.status == HULL_OVERFLOW) {
-        if (tid == 0) {
+        if (tid == 0 && a.retry) {
+            a.retry[1 + atomicAdd(a.retry, 1)] = item;
+        } else if (tid == 0) {
             if (mode == 0) a.out_err[cloud] = KERR_HULL_CAPACITY;
             else a.out_cnt[item] = -1;
         }
@@ -221,15 +236,49 @@ __global__ __launch_bounds__(64) void hull_wave_kernel(HullItemArgs a, int mode)
     hull_item<PPL, AS_LDS, 1>(a, mode, item, w, &sb);
 }
 
+// Item j of a launch, or -1 past the end.
+__device__ __forceinline__ int hull_item_at(const HullItemArgs& a, int j) {
+    if (a.list) return j < min(*a.list_n, a.n_items) ? a.list[j] : -1;
+    return j < a.n_items ? j : -1;
+}
+
+// Eight waves, workspace of VC vertices in LDS, multi-apex rounds; strides
+// over its items.
+template <int PPL>
+__global__ __launch_bounds__(64 * BLOCK_NW) void hull_lds_kernel(HullItemArgs a, int mode) {
+    extern __shared__ __align__(16) char lds[];
+    __shared__ HullBlockLDS sb;
+    __shared__ HullBits<64 * BLOCK_NW * PPL> hb;
+    const HullWS<AS_LDS> w = hull_ws_attach(hull_ws_carve<AS_LDS>(lds, a.VC, a.NP, HULL_WS_MULTI), &sb, &hb);
+    for (int j = blockIdx.x;; j += gridDim.x) {
+        const int item = hull_item_at(a, j);
+        if (item < 0) return;
+        __syncthreads();
+        hull_item<PPL, AS_LDS, BLOCK_NW, true>(a, mode, item, w, &sb);
+    }
+}
+
+// The same with the faces and vertices in global workspace blockIdx.x; the
+// rounds' marks and keys in dynamic LDS (hull_ma_bytes(VC)).
 template <int PPL>
 __global__ __launch_bounds__(64 * BLOCK_NW) void hull_block_kernel(HullItemArgs a, int mode) {
+    extern __shared__ __align__(16) char lds[];
     __shared__ HullBlockLDS sb;
     __shared__ HullBits<HULL_NP_MAX> hb;
-    const int item = blockIdx.x;
-    if (item >= a.n_items) return;
-    const HullWS<AS_GLOBAL> w = hull_ws_attach(
-        hull_ws_carve<AS_GLOBAL>(a.gws + (unsigned long long)item * a.gws_stride, a.VC, a.NP), &sb, &hb);
-    hull_item<PPL, AS_GLOBAL, BLOCK_NW>(a, mode, item, w, &sb);
+    const HullWS<AS_GLOBAL> w = hull_ma_attach(
+        hull_ws_attach(hull_ws_carve<AS_GLOBAL>(a.gws + (unsigned long long)blockIdx.x * a.gws_stride, a.VC, a.NP),
+                       &sb, &hb),
+        lds);
+    for (int j = blockIdx.x;; j += gridDim.x) {
+        const int item = hull_item_at(a, j);
+        if (item < 0) return;
+        __syncthreads();
+        hull_item<PPL, AS_GLOBAL, BLOCK_NW, true>(a, mode, item, w, &sb);
+    }
+}
+
+__global__ void hull_zero_kernel(int* p, int stride, int n) {
+    if ((int)threadIdx.x < n) p[(size_t)threadIdx.x * stride] = 0;
 }
 
 // Per-cloud AABB -> quantization frame (for the chunked path).
@@ -285,63 +334,166 @@ int launch_wave(gpu_ctx_t ctx, HullItemArgs a, int maxn, int mode) {
     return 0;
 }
 
-int launch_block(gpu_ctx_t ctx, HullItemArgs a, int maxn, int mode) {
+// Kernel and workspace of the global-memory tier for clouds of up to maxn
+// points; raises the kernel's dynamic-LDS limit to the rounds' scratch.
+int block_shape(gpu_ctx_t ctx, HullItemArgs* a, int maxn, KernelFn k4, KernelFn k8, KernelFn k16, KernelFn k32,
+                KernelFn* k, unsigned* lds) {
+    constexpr int T = 64 * BLOCK_NW;
+    *k = maxn <= 4 * T ? k4 : maxn <= 8 * T ? k8 : maxn <= 16 * T ? k16 : k32;
+    a->NP = (maxn + 63) / 64 * 64;
+    a->VC = a->NP;
+    a->gws_stride = (hull_ws_bytes<AS_GLOBAL>(a->VC, a->NP) + 255ull) & ~255ull;
+    *lds = hull_ma_bytes(a->VC);
+    HIP_TRY(hipFuncSetAttribute((const void*)*k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds));
+    return 0;
+}
+
+// The global-memory tier over a's items; `ws` holds grid workspaces of
+// a.gws_stride bytes for clouds of up to maxn points.
+int launch_block(gpu_ctx_t ctx, HullItemArgs a, int maxn, int mode, char* ws, int grid, hipStream_t s) {
     if (a.n_items <= 0) return 0;
     KernelFn k;
-    int ppl;
-    constexpr int T = 64 * BLOCK_NW;
-    if (maxn <= 4 * T) { ppl = 4; k = hull_block_kernel<4>; }
-    else if (maxn <= 8 * T) { ppl = 8; k = hull_block_kernel<8>; }
-    else if (maxn <= 16 * T) { ppl = 16; k = hull_block_kernel<16>; }
-    else { ppl = 32; k = hull_block_kernel<32>; }
-    int np = maxn;
-    np = (np + 63) / 64 * 64;
-    a.NP = np;
-    a.VC = np < 32704 ? np : 32704;
-    a.gws_stride = (hull_ws_bytes<AS_GLOBAL>(a.VC, a.NP) + 255ull) & ~255ull;
-    a.gws = (char*)stage_buf(ctx, 6, a.gws_stride * (unsigned long long)a.n_items);
-    REQUIRE(a.gws, "hull workspace allocation failed (%llu bytes)", a.gws_stride * (unsigned long long)a.n_items);
-    hipLaunchKernelGGL(k, dim3(a.n_items), dim3(T), 0, ctx->stream, a, mode);
+    unsigned lds;
+    if (int rc = block_shape(ctx, &a, maxn, hull_block_kernel<4>, hull_block_kernel<8>, hull_block_kernel<16>,
+                             hull_block_kernel<32>, &k, &lds))
+        return rc;
+    a.gws = ws;
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(64 * BLOCK_NW), lds, s, a, mode);
     HIP_TRY(hipGetLastError());
     return 0;
+}
+
+unsigned long long block_ws_bytes(int maxn) {
+    const int np = (maxn + 63) / 64 * 64;
+    return (hull_ws_bytes<AS_GLOBAL>(np, np) + 255ull) & ~255ull;
+}
+
+int launch_lds(gpu_ctx_t ctx, HullItemArgs a, int maxn, int vc, int grid, hipStream_t s) {
+    constexpr int T = 64 * BLOCK_NW;
+    const KernelFn k = maxn <= 2 * T ? hull_lds_kernel<2> : maxn <= 4 * T ? hull_lds_kernel<4> : hull_lds_kernel<8>;
+    a.VC = vc;
+    a.NP = maxn;
+    const unsigned lds = hull_ws_bytes<AS_LDS>(vc, maxn, HULL_WS_MULTI);
+    // the widest workspace of any launch of the kernel: the limit is the
+    // kernel's, and calls on other threads may launch it too
+    const unsigned most = hull_ws_bytes<AS_LDS>(1024, maxn, HULL_WS_MULTI);
+    HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)most));
+    hipLaunchKernelGGL(k, dim3((unsigned)grid), dim3(T), lds, s, a, 0);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+// Tiers of a call (bit t): 0 up to 512 points, 1 up to 1024, 2 up to 2048,
+// 3 up to 4096, 4 up to 8192, 5 up to 16384.
+constexpr int TIER_MAX[6] = {WAVE_TIER, 1024, 2048, 4096, 8192, BLOCK_MAX};
+int tier_of(int n) {
+    int t = 0;
+    while (t < 5 && n > TIER_MAX[t]) ++t;
+    return t;
+}
+
+// Every tier in `tiers` over a's items (clouds of up to max_pts <= BLOCK_MAX
+// points; wave_max the largest of the one-wave tier).
+// `top`: the largest cloud the last tier still answers for (with an error
+// where it exceeds the kernel's capacity).
+int launch_tiers(gpu_ctx_t ctx, HullItemArgs a, unsigned tiers, int wave_max, int top) {
+    const int n = a.n_items;
+    if (n <= 0) return 0;
+    const int grid = std::min(n, 2 * std::max(1, ctx->n_cu));
+    // workspaces: one region per tier that may need one, then the retry lists
+    unsigned long long off[6], ws = 0;
+    for (int t = 2; t < 6; ++t) {
+        off[t] = ws;
+        if (tiers >> t & 1) ws += block_ws_bytes(TIER_MAX[t]) * (unsigned long long)grid;
+    }
+    const size_t rs = ((size_t)n + 1 + 63) / 64 * 64;  // ints per retry list
+    char* base = nullptr;
+    int* retry = nullptr;
+    if (tiers & ~1u) {
+        base = (char*)stage_buf(ctx, 6, ws + 4 * 4 * rs);
+        REQUIRE(base, "hull workspace allocation failed (%llu bytes)", ws + 4ull * 4 * rs);
+        retry = (int*)(base + ws);
+        hipLaunchKernelGGL(hull_zero_kernel, dim3(1), dim3(64), 0, ctx->stream, retry, (int)rs, 4);
+        HIP_TRY(hipGetLastError());
+    }
+    auto args = [&](int t) {
+        HullItemArgs x = a;
+        x.min_n = t ? TIER_MAX[t - 1] + 1 : 0;
+        x.max_n = tiers >> (t + 1) ? TIER_MAX[t] : std::max(TIER_MAX[t], top);
+        return x;
+    };
+    bool used[3] = {false, false, false};
+    if (tiers & ~3u) HIP_TRY(hipEventRecord(ctx->ev_fork, ctx->stream));
+    auto fork = [&](int k, hipStream_t* s) -> int {
+        if (!used[k]) HIP_TRY(hipStreamWaitEvent(ctx->aux[k], ctx->ev_fork, 0));
+        used[k] = true;
+        *s = ctx->aux[k];
+        return 0;
+    };
+    int rc = 0;
+    hipStream_t s;
+    // the longest insertion chains first
+    for (int t = 5; t >= 4 && !rc; --t)
+        if (tiers >> t & 1) {
+            rc = fork(0, &s);
+            if (!rc) rc = launch_block(ctx, args(t), TIER_MAX[t], 0, base + off[t], grid, s);
+        }
+    for (int t = 3; t >= 1 && !rc; --t) {
+        if (!(tiers >> t & 1)) continue;
+        if (t == 1) s = ctx->stream;
+        else rc = fork(t - 1, &s);
+        HullItemArgs x = args(t);
+        x.retry = retry + (size_t)t * rs;
+        if (!rc) rc = launch_lds(ctx, x, TIER_MAX[t], t == 1 ? 384 : 1024, n, s);
+        x.list = x.retry + 1;
+        x.list_n = x.retry;
+        x.retry = nullptr;
+        if (!rc)
+            rc = t == 1 ? launch_lds(ctx, x, TIER_MAX[t], 1024, std::min(n, std::max(1, ctx->n_cu)), s)
+                        : launch_block(ctx, x, TIER_MAX[t], 0, base + off[t], grid, s);
+    }
+    if (!rc && (tiers & 1)) rc = launch_wave(ctx, args(0), std::min(wave_max, WAVE_TIER), 0);
+    for (int k = 0; k < 3; ++k)
+        if (used[k]) {
+            HIP_TRY(hipEventRecord(ctx->ev_join[k], ctx->aux[k]));
+            HIP_TRY(hipStreamWaitEvent(ctx->stream, ctx->ev_join[k], 0));
+        }
+    return rc;
 }
 
 // ---- the allocation-free entry point --------------------------------------
 // gpu_hull_dandc_dev_noalloc's block tier: the work of hull_block_kernel for
 // items item0 + b (workgroup b), each in workspace b of the caller's region.
 template <int PPL>
-__global__ __launch_bounds__(64 * BLOCK_NW) void hull_block_pass_kernel(HullItemArgs a, int mode, int item0) {
+__global__ __launch_bounds__(64 * BLOCK_NW) void hull_block_pass_kernel(HullItemArgs a, int item0) {
+    extern __shared__ __align__(16) char lds[];
     __shared__ HullBlockLDS sb;
     __shared__ HullBits<HULL_NP_MAX> hb;
     const int item = item0 + (int)blockIdx.x;
     if (item >= a.n_items) return;
-    const HullWS<AS_GLOBAL> w = hull_ws_attach(
-        hull_ws_carve<AS_GLOBAL>(a.gws + (unsigned long long)blockIdx.x * a.gws_stride, a.VC, a.NP), &sb, &hb);
-    hull_item<PPL, AS_GLOBAL, BLOCK_NW>(a, mode, item, w, &sb);
+    const HullWS<AS_GLOBAL> w = hull_ma_attach(
+        hull_ws_attach(hull_ws_carve<AS_GLOBAL>(a.gws + (unsigned long long)blockIdx.x * a.gws_stride, a.VC, a.NP),
+                       &sb, &hb),
+        lds);
+    hull_item<PPL, AS_GLOBAL, BLOCK_NW, true>(a, 0, item, w, &sb);
 }
 
 // Block tier over a fixed workspace region of ws_cap bytes: passes of as
 // many items as fit (same kernel choice and workspace layout as launch_block).
 int launch_block_passes(gpu_ctx_t ctx, HullItemArgs a, int maxn, char* ws, unsigned long long ws_cap) {
     if (a.n_items <= 0) return 0;
-    using PassFn = void (*)(HullItemArgs, int, int);
-    PassFn k;
-    constexpr int T = 64 * BLOCK_NW;
-    if (maxn <= 4 * T) k = hull_block_pass_kernel<4>;
-    else if (maxn <= 8 * T) k = hull_block_pass_kernel<8>;
-    else if (maxn <= 16 * T) k = hull_block_pass_kernel<16>;
-    else k = hull_block_pass_kernel<32>;
-    const int np = (maxn + 63) / 64 * 64;
-    a.NP = np;
-    a.VC = np < 32704 ? np : 32704;
-    a.gws_stride = (hull_ws_bytes<AS_GLOBAL>(a.VC, a.NP) + 255ull) & ~255ull;
+    KernelFn k;
+    unsigned lds;
+    if (int rc = block_shape(ctx, &a, maxn, hull_block_pass_kernel<4>, hull_block_pass_kernel<8>,
+                             hull_block_pass_kernel<16>, hull_block_pass_kernel<32>, &k, &lds))
+        return rc;
     const unsigned long long per = ws_cap / a.gws_stride;
     REQUIRE(per >= 1, "a %d-point cloud needs %llu workspace bytes, above the %llu-byte scratch", maxn,
             a.gws_stride, ws_cap);
     a.gws = ws;
     for (long long i0 = 0; i0 < a.n_items; i0 += (long long)per) {
         const long long cnt = std::min<long long>((long long)per, a.n_items - i0);
-        hipLaunchKernelGGL(k, dim3((unsigned)cnt), dim3(T), 0, ctx->stream, a, 0, (int)i0);
+        hipLaunchKernelGGL(k, dim3((unsigned)cnt), dim3(64 * BLOCK_NW), lds, ctx->stream, a, (int)i0);
         HIP_TRY(hipGetLastError());
     }
     return 0;
@@ -375,13 +527,25 @@ static int hull_batch_device(gpu_ctx_t ctx, const float* d_pts, const int* d_off
     a.out_nt = d_nt;
     a.out_err = d_err;
     a.out_vol = d_vol;
-    a.min_n = 0;
-    a.max_n = WAVE_MAX;
-    int rc = launch_wave(ctx, a, max_pts < WAVE_MAX ? max_pts : WAVE_MAX, 0);
-    if (rc || max_pts <= WAVE_MAX) return rc;
-    a.min_n = WAVE_MAX + 1;
-    a.max_n = BLOCK_MAX;
-    rc = launch_block(ctx, a, max_pts < BLOCK_MAX ? max_pts : BLOCK_MAX, 0);
+    // the tiers with members where the sizes are known on the host, else all
+    // up to the largest cloud's
+    unsigned tiers = 0;
+    int wave_max = std::min(max_pts, WAVE_TIER);
+    if (h_offsets) {
+        wave_max = 0;
+        for (int c = 0; c < n_hulls; ++c) {
+            const int n = h_offsets[c + 1] - h_offsets[c];
+            if (n > BLOCK_MAX) continue;
+            const int t = tier_of(n);
+            tiers |= 1u << t;
+            if (t == 0) wave_max = std::max(wave_max, n);
+        }
+    } else {
+        tiers = (2u << tier_of(std::min(max_pts, BLOCK_MAX))) - 1u;
+    }
+    // sizes above a device caller's max_pts are answered with an error, as far
+    // as one kernel of the smaller or larger tiers could have hulled them
+    int rc = launch_tiers(ctx, a, tiers, wave_max, h_offsets ? 0 : max_pts <= WAVE_MAX ? WAVE_MAX : BLOCK_MAX);
     if (rc || max_pts <= BLOCK_MAX) return rc;
 
     REQUIRE(h_offsets != nullptr, "clouds above %d points need the host entry point", BLOCK_MAX);
@@ -480,7 +644,55 @@ static int hull_batch_device(gpu_ctx_t ctx, const float* d_pts, const int* d_off
     f.n_items = nb;
     f.min_n = 0;
     f.max_n = BLOCK_MAX;
-    return launch_block(ctx, f, maxn, 0);
+    const int grid = std::min(nb, 2 * std::max(1, ctx->n_cu));
+    const unsigned long long wsb = block_ws_bytes(maxn) * (unsigned long long)grid;
+    char* ws = (char*)stage_buf(ctx, 6, wsb);
+    REQUIRE(ws, "hull workspace allocation failed (%llu bytes)", wsb);
+    return launch_block(ctx, f, maxn, 0, ws, grid, ctx->stream);
+}
+
+// Above this many bytes of padded output slots (every hull has one for the
+// call's largest cloud), the hulls' own vertices and triangles are packed on
+// the device and read back through pinned staging; the counts come first, one
+// more wait of about 20 us. 192 clouds of 5-12000 points have 83 MB of slots
+// for 1.3 MB of hulls.
+constexpr size_t PACKED_READBACK = 1 << 20;
+
+static int packed_readback(gpu_ctx_t ctx, int n, int max_hv, int max_ht, const float* d_v, const int* d_t,
+                           const int* nv, const int* nt, float* out_verts, int* out_tris) {
+    HIP_TRY(ctx_stream_sync(ctx, ctx->stream));  // the counts
+    std::vector<LaSeg> segs;
+    std::vector<std::pair<void*, size_t>> to;  // host destination, offset in the staging
+    size_t total = 0;
+    auto add = [&](const void* src, void* dst, size_t bytes) {
+        if (!bytes) return;
+        segs.push_back({src, nullptr, bytes});
+        to.push_back({dst, total});
+        total += (bytes + 15) / 16 * 16;
+    };
+    for (int i = 0; i < n; ++i) {
+        // a hull above its slot's capacity is not written
+        if (nv[i] <= max_hv) {
+            const size_t o = 3 * (size_t)max_hv * i;
+            add(d_v + o, out_verts + o, 12 * (size_t)nv[i]);
+        }
+        if (nt[i] <= max_ht) {
+            const size_t o = 3 * (size_t)max_ht * i;
+            add(d_t + o, out_tris + o, 12 * (size_t)nt[i]);
+        }
+    }
+    if (segs.empty()) return 0;
+    const size_t seg_bytes = (sizeof(LaSeg) * segs.size() + 255) / 256 * 256;
+    char* dev = (char*)stage_buf(ctx, 7, seg_bytes + total);
+    char* host = pinned_stage(ctx, total);
+    REQUIRE(dev && host, "hull readback staging allocation failed (%zu bytes)", total);
+    for (size_t k = 0; k < segs.size(); ++k) segs[k].dst = dev + seg_bytes + to[k].second;
+    HIP_TRY(hipMemcpyAsync(dev, segs.data(), sizeof(LaSeg) * segs.size(), hipMemcpyHostToDevice, ctx->stream));
+    if (int rc = la_launch_segcopy(ctx, (const LaSeg*)dev, (int)segs.size())) return rc;
+    HIP_TRY(hipMemcpyAsync(host, dev + seg_bytes, total, hipMemcpyDeviceToHost, ctx->stream));
+    HIP_TRY(ctx_stream_sync(ctx, ctx->stream));
+    for (size_t k = 0; k < segs.size(); ++k) memcpy(to[k].first, host + to[k].second, segs[k].bytes);
+    return 0;
 }
 
 extern "C" {
@@ -573,14 +785,18 @@ int gpu_hull_dandc_vol(gpu_ctx_t ctx, const float* pts, int total_pts, const int
     int rc = hull_batch_device(ctx, d_pts, d_off, offsets, n_hulls, mx, max_hv, max_ht, d_v, d_t, d_nv, d_nt, d_e,
                                out_volumes ? d_vol : nullptr);
     if (rc == 0) {
-        if (b_v) HIP_TRY(hipMemcpyAsync(out_verts, d_v, b_v, hipMemcpyDeviceToHost, ctx->stream));
-        if (b_t) HIP_TRY(hipMemcpyAsync(out_tris, d_t, b_t, hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(hipMemcpyAsync(out_nv, d_nv, b_i, hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(hipMemcpyAsync(out_nt, d_nt, b_i, hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(hipMemcpyAsync(out_errors, d_e, b_i, hipMemcpyDeviceToHost, ctx->stream));
         if (out_volumes)
             HIP_TRY(hipMemcpyAsync(out_volumes, d_vol, sizeof(double) * n_hulls, hipMemcpyDeviceToHost,
                                    ctx->stream));
+        if (b_v + b_t <= PACKED_READBACK) {
+            if (b_v) HIP_TRY(hipMemcpyAsync(out_verts, d_v, b_v, hipMemcpyDeviceToHost, ctx->stream));
+            if (b_t) HIP_TRY(hipMemcpyAsync(out_tris, d_t, b_t, hipMemcpyDeviceToHost, ctx->stream));
+        } else {
+            rc = packed_readback(ctx, n_hulls, max_hv, max_ht, d_v, d_t, out_nv, out_nt, out_verts, out_tris);
+        }
     }
     HIP_TRY(hipFreeAsync(d_inbuf, ctx->stream));
     HIP_TRY(hipFreeAsync(d_outbuf, ctx->stream));

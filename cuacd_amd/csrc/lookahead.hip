@@ -229,20 +229,12 @@ struct Engine {
             offs[k] = total;
             total += (src[k].second + 15) / 16 * 16;
         }
-        char*& pinned = ctx->la_pinned;
-        if (total == 0) return pinned;
-        if (total > ctx->la_pinned_cap) {
-            if (pinned) (void)hipHostFree(pinned);
-            pinned = nullptr;
-            ctx->la_pinned_cap = 0;
-            const size_t cap = std::max(total + total / 2, (size_t)(1 << 20));
-            if (hipHostMalloc((void**)&pinned, cap, hipHostMallocDefault) != hipSuccess) {
-                pinned = nullptr;
-                set_error(ctx, "lookahead: pinned staging allocation failed");
-                *rc = -1;
-                return nullptr;
-            }
-            ctx->la_pinned_cap = cap;
+        if (total == 0) return ctx->la_pinned;
+        char* pinned = pinned_stage(ctx, total);
+        if (!pinned) {
+            set_error(ctx, "lookahead: pinned staging allocation failed");
+            *rc = -1;
+            return nullptr;
         }
         DevBuf<char> stage;
         DevBuf<LaSeg> dsegs;
