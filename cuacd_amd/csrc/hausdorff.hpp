@@ -18,9 +18,13 @@
 //   * the tree is implicit: level 0 groups 4 consecutive sorted triangles into
 //     a leaf, every level above groups 8 nodes, so child/parent are index
 //     arithmetic and there are no pointers;
-//   * each lane answers one sample: a greedy descent to the nearest-looking
-//     leaf gives an upper bound, then a stackless in-order walk of the
-//     implicit tree prunes every box farther than the current best.
+//   * a greedy descent to the nearest-looking leaf gives each sample an upper
+//     bound (lane per sample); the exact search opens the nearest boxes first
+//     and passes over every box farther than the current best;
+//   * only the largest of the nearest distances counts, so a sample whose
+//     upper bound is not above the maximum found so far is done: every sample
+//     gets its bound first, and the samples of the highest bounds are searched
+//     first, a whole wave each.
 // Distances are fp32 (closest point on triangle by Voronoi regions).
 #pragma once
 #include "wave.hpp"
@@ -295,9 +299,9 @@ __device__ __forceinline__ float leaf_d2(const HdBvh& b, int j, V3 p, float best
     return best;
 }
 
-// Exact squared distance from p to the nearest target triangle.
-__device__ inline float hd_nearest_d2(const HdBvh& b, V3 p) {
-    // greedy descent for an upper bound
+// Greedy descent to the nearest-looking leaf: an upper bound of the squared
+// distance from p to the target, and the leaf it comes from.
+__device__ __forceinline__ float hd_greedy_d2(const HdBvh& b, V3 p, int* leaf) {
     int L = b.top, i = 0;
     while (L > 0) {
         const int c0 = 8 * i, c1 = min(8 * i + 8, b.cnt[L - 1]);
@@ -310,33 +314,71 @@ __device__ inline float hd_nearest_d2(const HdBvh& b, V3 p) {
         --L;
         i = bi;
     }
-    float best = leaf_d2(b, i, p, 3.4e38f);
-    const int greedy_leaf = i;
-    // stackless in-order walk of the implicit tree with pruning
-    L = b.top;
-    i = 0;
-    for (;;) {
-        const float d = box_d2(b, L, i, p);
-        if (d < best) {
-            if (L == 0) {
-                if (i != greedy_leaf) best = leaf_d2(b, i, p, best);
-            } else {
-                --L;
-                i *= 8;
-                continue;
-            }
-        }
-        // advance to the next sibling, climbing while the group is exhausted
+    *leaf = i;
+    return leaf_d2(b, i, p, 3.4e38f);
+}
+
+// The bound tightened by the greedy leaf's siblings (until it is not above
+// `floor`).
+__device__ __forceinline__ float hd_siblings_d2(const HdBvh& b, V3 p, float best, int leaf, float floor) {
+    const int c0 = leaf & ~7, c1 = min(c0 + 8, b.cnt[0]);
+    for (int c = c0; c < c1 && best > floor; ++c)
+        if (c != leaf && box_d2(b, 0, c, p) < best) best = leaf_d2(b, c, p, best);
+    return best;
+}
+
+// Exact squared distance from p to the nearest target triangle, by the whole
+// wave for one sample (p and the upper bound `best` wave-uniform); may stop at
+// any upper bound not above `floor`. Level-1 nodes (32 sorted triangles) are
+// tested 64 at a time - 64 consecutive ones are a level-3 node, tested first -
+// and the two nearest that remain are opened together, a triangle per lane. A
+// lane walking the tree alone is a chain of several hundred dependent reads;
+// this is two to six rounds.
+__device__ inline float hd_wave_nearest_d2(const HdBvh& b, V3 p, float best, float floor) {
+    if (b.top == 0) return best;  // one leaf: the bound is exact
+    const int lane = lane_id();
+    const int n1 = b.cnt[1], ntp = (b.nt + 3) / 4 * 4;
+    const int groups = (n1 + 63) / 64;
+    // a box is passed over only when it is farther by more than the rounding
+    // of its distance and a triangle's, so the visiting order cannot change
+    // which triangle is found nearest
+    auto near = [&](float d) { return d * 0.99999f < best; };
+    for (int g0 = 0; g0 < groups; g0 += 64) {
+        const int g = g0 + lane;
+        float gd = 3.4e38f;
+        if (groups == 1) gd = lane == 0 ? 0.0f : gd;
+        else if (g < groups) gd = box_d2(b, 3, g, p);
         for (;;) {
-            if (L == b.top) return best;
-            if ((i & 7) != 7 && i + 1 < b.cnt[L]) {
-                ++i;
-                break;
+            const uint32_t gk = wave_min_u32(near(gd) ? __float_as_uint(gd) : ~0u);
+            if (gk == ~0u) break;
+            const int gl = __builtin_ctzll(ballot(near(gd) && __float_as_uint(gd) == gk));
+            if (lane == gl) gd = __builtin_inff();
+            const int i1 = 64 * (g0 + gl) + lane;
+            float d = i1 < n1 ? box_d2(b, 1, i1, p) : __builtin_inff();
+            for (;;) {
+                // the two nearest nodes not yet opened
+                const uint32_t k0 = wave_min_u32(near(d) ? __float_as_uint(d) : ~0u);
+                if (k0 == ~0u) break;
+                const int l0 = __builtin_ctzll(ballot(near(d) && __float_as_uint(d) == k0));
+                if (lane == l0) d = __builtin_inff();
+                const uint32_t k1 = wave_min_u32(near(d) ? __float_as_uint(d) : ~0u);
+                int l1 = l0;
+                if (k1 != ~0u) {
+                    l1 = __builtin_ctzll(ballot(near(d) && __float_as_uint(d) == k1));
+                    if (lane == l1) d = __builtin_inff();
+                }
+                const int t = 32 * (64 * (g0 + gl) + (lane < 32 ? l0 : l1)) + (lane & 31);
+                float d2 = 3.4e38f;
+                if (t < ntp) {
+                    const f4v x = b.tri[3 * t], y = b.tri[3 * t + 1], z = b.tri[3 * t + 2];
+                    d2 = pt_tri_d2(p, {x.x, x.y, x.z}, {y.x, y.y, y.z}, {z.x, z.y, z.z});
+                }
+                best = fminf(best, wave_min_f(d2));
+                if (best <= floor) return best;
             }
-            ++L;
-            i >>= 3;
         }
     }
+    return best;
 }
 
 // One directed Hausdorff task: samples on the source surface, nearest
