@@ -9,11 +9,11 @@
 // 4 -> 128 -> 128 -> 128 (ReLU); the features are max-pooled separately over
 // the samples on each side of the plane (g+, g-: the two halves' shapes) and a
 // head [g+, g-, n, d] -> 128 -> 128 -> 1 (ReLU between) predicts the plane's
-// exact cut score. BF16 operands, FP32 accumulation: every layer is one
-// call of a wave64 MFMA GEMM (v_mfma_f32_16x16x16_bf16) with a fused epilogue
-// (bias, ReLU, backward ReLU mask, FP32 and BF16 stores). Training keeps FP32
-// master weights and Adam state on the device and runs forward, backward and
-// the update as kernels (mean squared error on the score).
+// exact cut score. BF16 operands, FP32 accumulation on v_mfma_f32_16x16x16_bf16.
+// Inference and training run fused kernels whose activations stay in registers
+// (see "Register chains"); a layer-by-layer GEMM path is kept for inference
+// (tuning knob mlp_fused; the same scores). Training keeps FP32 master weights
+// and Adam state on the device (mean squared error on the score).
 //
 // Parameter layout (FP32, padded to multiples of 16; the padding stays zero):
 //   W1 [16 x 128] (rows 0..3 used), b1 [128], W2 [128 x 128], b2, W3, b3,
@@ -167,159 +167,554 @@ __global__ __launch_bounds__(256) void mlp_gemm_kernel(GemmArgs g) {
 }
 
 // ---------------------------------------------------------------------------
-// Fused inference of the point layers and the pooling: a persistent grid of
-// 256-thread workgroups, each with the transposed point-layer weights in LDS,
-// strides over the candidates; per candidate wave w owns samples 64w..64w+63
-// (4 x 8 MFMA 16 x 16 x 16 tiles) and the activations stay in LDS as BF16.
-// The MFMA operand layout, the k order (16-wide steps, ascending; layer 1
-// adds the GEMM's second, all-zero step), the epilogue (bias, ReLU, BF16
-// rounding) and the pooling rule are those of mlp_gemm_kernel and
-// mlp_maxpool, so G equals the layer-by-layer path's bit for bit; only
-// G [C x 256] reaches memory.
+// Register chains: a wave carries 16 rows (samples, candidates) per tile through
+// consecutive layers without LDS or memory in between. With the weights as the
+// MFMA's A operand (rows = output channels) and the activations as its B
+// operand (columns = rows of the batch), lane l of the result holds output
+// channels 4 (l / 16) .. +3 of row l % 16 - exactly the B operand of the next
+// layer's product over those channels. The k order (16-wide steps, ascending),
+// the epilogue (bias, ReLU, BF16 rounding) and so the results are those of
+// mlp_gemm_kernel, bit for bit.
 // ---------------------------------------------------------------------------
-constexpr int FP = HD + 8;    // activation / weight row pitch in LDS (bf16)
+constexpr int FP = HD + 8;    // weight row pitch in LDS (bf16)
 constexpr int FP1 = KIN + 8;  // pitch of the transposed first layer
-constexpr unsigned FUSED_LDS = (unsigned)(NS * FP * 2 + 2 * HD * FP * 2 + HD * FP1 * 2 + NS * 4 + 2 * 4 * HD * 4);
 
-__device__ __forceinline__ s4v_t lds_frag(const bf16_t* p) { return *reinterpret_cast<const s4v_t*>(p); }
+typedef __bf16 bf2_t __attribute__((ext_vector_type(2)));
+typedef float f2v_t __attribute__((ext_vector_type(2)));
 
-__global__ __launch_bounds__(256) void mlp_encode_pool_kernel(const float* pts, const float* planes,
-                                                              const int* part_of, int C, const bf16_t* W,
-                                                              const float* Wf, float* G) {
+__device__ __forceinline__ s4v_t ld_frag(const bf16_t* p) { return *reinterpret_cast<const s4v_t*>(p); }
+__device__ __forceinline__ f4v_t mma(s4v_t a, s4v_t b, f4v_t c) {
+    return __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a, b, c, 0, 0, 0);
+}
+// round to nearest even (v_cvt_pk_bf16_f32)
+__device__ __forceinline__ s4v_t pack4(float x, float y, float z, float w) {
+    const bf2_t lo = __builtin_convertvector((f2v_t{x, y}), bf2_t), hi = __builtin_convertvector((f2v_t{z, w}), bf2_t);
+    const uint2 u = make_uint2(__builtin_bit_cast(uint32_t, lo), __builtin_bit_cast(uint32_t, hi));
+    return __builtin_bit_cast(s4v_t, u);
+}
+__device__ __forceinline__ s4v_t relu4(f4v_t a, f4v_t b) {
+    return pack4(fmaxf(a[0] + b[0], 0.0f), fmaxf(a[1] + b[1], 0.0f), fmaxf(a[2] + b[2], 0.0f),
+                 fmaxf(a[3] + b[3], 0.0f));
+}
+// the gradient where the activation is positive
+__device__ __forceinline__ s4v_t mask4(f4v_t v, s4v_t act) {
+    return pack4((act[0] & 0x7fff) ? v[0] : 0.0f, (act[1] & 0x7fff) ? v[1] : 0.0f, (act[2] & 0x7fff) ? v[2] : 0.0f,
+                 (act[3] & 0x7fff) ? v[3] : 0.0f);
+}
+// First-layer operand of a sample: (x, y, z, s) in the lanes of channels 0..3.
+__device__ __forceinline__ s4v_t point_frag(const float* p, float sd, bool on) {
+    const s4v_t z = {0, 0, 0, 0};
+    return on ? s4v_t{(short)f2bf(p[0]), (short)f2bf(p[1]), (short)f2bf(p[2]), (short)f2bf(sd)} : z;
+}
+// The transpose of a 16 x 16 tile as the same lane layout: a product with the
+// identity (BF16 values pass through exactly).
+__device__ __forceinline__ s4v_t identity_frag() {
+    const int fr = lane_id() & 15, fk = 4 * (lane_id() >> 4);
+    s4v_t r;
+#pragma unroll
+    for (int q = 0; q < 4; ++q) r[q] = (short)(fk + q == fr ? 0x3f80 : 0);
+    return r;
+}
+__device__ __forceinline__ s4v_t transpose4(s4v_t a, s4v_t eye) {
+    const f4v_t d = mma(a, eye, f4v_t{0.f, 0.f, 0.f, 0.f});
+    return pack4(d[0], d[1], d[2], d[3]);
+}
+
+// rows x cols of a row-major BF16 matrix into LDS rows of `pitch` (16-byte pieces)
+__device__ __forceinline__ void stage_rows(bf16_t* dst, int pitch, const bf16_t* src, int rows, int cols) {
+    const int per = cols / 8;
+    for (int i = threadIdx.x; i < rows * per; i += blockDim.x)
+        *reinterpret_cast<uint4*>(dst + (i / per) * pitch + (i % per) * 8) =
+            *reinterpret_cast<const uint4*>(src + (i / per) * cols + (i % per) * 8);
+}
+
+// Point layers and pooling: a persistent grid of 512-thread workgroups with the
+// transposed point-layer weights in LDS; four waves take a candidate, each 64
+// samples (4 tiles), and only the head's input row (Hin: pooled features, the
+// plane, zeros) - and for training the pooled rows - reach memory. Two waves
+// per SIMD: one's MFMAs cover the other's epilogue. An output tile's weight
+// fragment (512 B of LDS) feeds four MFMAs. Pooling takes integer maxima of
+// (BF16 bits, inverted sample), so ties go to the first sample. 12,032
+// candidates: the activations in LDS, one wave per SIMD, took 0.87 ms.
+constexpr unsigned ENC_LDS = 2 * HD * FP * 2 + HD * FP1 * 2 + 3 * HD * 4 + 2 * 2 * 4 * 2 * HD * 4;
+
+template <int CTRL> __device__ __forceinline__ int row_max(int v) {
+    return max(v, __builtin_amdgcn_update_dpp(0, v, CTRL, 0xf, 0xf, true));  // rotation in a row of 16
+}
+
+__global__ __launch_bounds__(512) void mlp_encode_kernel(const float* pts, const float* planes, const int* part_of,
+                                                         int C, const bf16_t* Wt, const float* Wf, bf16_t* Hin,
+                                                         uint8_t* arg) {
     extern __shared__ __align__(16) char fl[];
-    bf16_t* H = (bf16_t*)fl;                    // [NS][FP] X, then the layer outputs
-    bf16_t* W2t = H + NS * FP;                  // [HD][FP] W2 transposed: W2t[n][k]
-    bf16_t* W3t = W2t + HD * FP;                // [HD][FP]
-    bf16_t* W1t = W3t + HD * FP;                // [HD][FP1]
-    float* Sd = (float*)(W1t + HD * FP1);       // [NS] signed distances
-    float* red = Sd + NS;                       // [2][4][HD] per-wave side maxima
+    bf16_t* W2t = (bf16_t*)fl;            // [HD][FP] W2t[n][k]
+    bf16_t* W3t = W2t + HD * FP;          // [HD][FP]
+    bf16_t* W1t = W3t + HD * FP;          // [HD][FP1]
+    float* bs = (float*)(W1t + HD * FP1); // [3][HD] biases
+    int* red = (int*)(bs + 3 * HD);       // [2 rounds][2 candidates][4 waves][2 sides x HD] keys
     const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
-    for (int i = tid; i < HD * HD; i += 256) {
-        const int k = i / HD, n = i % HD;
-        W2t[n * FP + k] = W[P_W2 + i];
-        W3t[n * FP + k] = W[P_W3 + i];
+    stage_rows(W2t, FP, Wt + P_W2, HD, HD);
+    stage_rows(W3t, FP, Wt + P_W3, HD, HD);
+    stage_rows(W1t, FP1, Wt + P_W1, HD, KIN);
+    for (int i = tid; i < HD; i += 512) {
+        bs[i] = Wf[P_B1 + i];
+        bs[HD + i] = Wf[P_B2 + i];
+        bs[2 * HD + i] = Wf[P_B3 + i];
     }
-    for (int i = tid; i < KIN * HD; i += 256) {
-        const int k = i / HD, n = i % HD;
-        W1t[n * FP1 + k] = W[P_W1 + i];
-    }
-    const int r0 = 64 * wv;
+    __syncthreads();
     const int fr = lane & 15, fk = 4 * (lane >> 4);
-    for (int c = blockIdx.x; c < C; c += gridDim.x) {
-        __syncthreads();
-        {
-            // sample tid of the candidate's part (the rows of mlp_pack_points)
-            const float* pp = pts + ((long long)part_of[c] * NS + tid) * 3;
-            const float* pl = planes + 4ll * c;
+    const int cw = wv >> 2, ws = wv & 3;
+    const f4v_t zero = {0.f, 0.f, 0.f, 0.f};
+    int round = 0;
+    for (int pr = blockIdx.x; 2 * pr < C; pr += gridDim.x, round ^= 1) {
+        const int c = min(2 * pr + cw, C - 1);
+        const float* pl = planes + 4ll * c;
+        const float* base = pts + (long long)part_of[c] * NS * 3;
+        s4v_t x[4], a1[8][4], a2[8][4];
+        bool pos[4];
+#pragma unroll
+        for (int j = 0; j < 4; ++j) {
+            const float* pp = base + 3 * (64 * ws + 16 * j + fr);
             const float sd = pl[0] * pp[0] + pl[1] * pp[1] + pl[2] * pp[2] + pl[3];
-            Sd[tid] = sd;
-            bf16_t* x = H + tid * FP;
-            x[0] = f2bf(pp[0]);
-            x[1] = f2bf(pp[1]);
-            x[2] = f2bf(pp[2]);
-            x[3] = f2bf(sd);
-            for (int j = 4; j < KIN; ++j) x[j] = 0;
+            pos[j] = sd >= 0.0f;
+            x[j] = point_frag(pp, sd, fk == 0);
         }
-        __syncthreads();
-        f4v_t acc[4][8];
-        // layer 1: K = 16
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i) {
+            const s4v_t a = ld_frag(W1t + (16 * i + fr) * FP1 + fk);
+            const f4v_t b = *(const f4v_t*)(bs + 16 * i + fk);
 #pragma unroll
-            for (int j = 0; j < 8; ++j) acc[i][j] = f4v_t{0.f, 0.f, 0.f, 0.f};
-        {
-            s4v_t a[4], b[8];
-            const s4v_t z = s4v_t{0, 0, 0, 0};
-#pragma unroll
-            for (int i = 0; i < 4; ++i) a[i] = lds_frag(H + (r0 + 16 * i + fr) * FP + fk);
-#pragma unroll
-            for (int j = 0; j < 8; ++j) b[j] = lds_frag(W1t + (16 * j + fr) * FP1 + fk);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
-                    acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(z, z, acc[i][j], 0, 0, 0);
-                }
+            for (int j = 0; j < 4; ++j) a1[i][j] = relu4(mma(a, x[j], zero), b);
         }
-        __syncthreads();
-        auto store = [&](const float* bias) {
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i) {
+            f4v_t acc[4] = {zero, zero, zero, zero};
 #pragma unroll
-                for (int j = 0; j < 8; ++j) {
-                    const int n = 16 * j + fr;
-                    const float bn = bias[n];
+            for (int k = 0; k < 8; ++k) {
+                const s4v_t a = ld_frag(W2t + (16 * i + fr) * FP + 16 * k + fk);
 #pragma unroll
-                    for (int r = 0; r < 4; ++r) {
-                        float v = 1.0f * acc[i][j][r];
-                        v += bn;
-                        v = fmaxf(v, 0.0f);
-                        H[(r0 + 16 * i + fk + r) * FP + n] = f2bf(v);
-                    }
-                }
-        };
-        auto layer = [&](const bf16_t* Wt) {
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-#pragma unroll
-                for (int j = 0; j < 8; ++j) acc[i][j] = f4v_t{0.f, 0.f, 0.f, 0.f};
-#pragma unroll 2
-            for (int k0 = 0; k0 < HD; k0 += 16) {
-                s4v_t a[4], b[8];
-#pragma unroll
-                for (int i = 0; i < 4; ++i) a[i] = lds_frag(H + (r0 + 16 * i + fr) * FP + k0 + fk);
-#pragma unroll
-                for (int j = 0; j < 8; ++j) b[j] = lds_frag(Wt + (16 * j + fr) * FP + k0 + fk);
-#pragma unroll
-                for (int i = 0; i < 4; ++i)
-#pragma unroll
-                    for (int j = 0; j < 8; ++j)
-                        acc[i][j] = __builtin_amdgcn_mfma_f32_16x16x16bf16_1k(a[i], b[j], acc[i][j], 0, 0, 0);
+                for (int j = 0; j < 4; ++j) acc[j] = mma(a, a1[k][j], acc[j]);
             }
-        };
-        store(Wf + P_B1);
-        __syncthreads();
-        layer(W2t);
-        __syncthreads();
-        store(Wf + P_B2);
-        __syncthreads();
-        layer(W3t);
-        // layer 3 epilogue: BF16-rounded activations pooled per side of the plane
+            const f4v_t b = *(const f4v_t*)(bs + HD + 16 * i + fk);
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-            const int n = 16 * j + fr;
-            const float bn = Wf[P_B3 + n];
-            float bp = -1e30f, bq = -1e30f;
+            for (int j = 0; j < 4; ++j) a2[i][j] = relu4(acc[j], b);
+        }
+        int* rd = red + ((round * 2 + cw) * 4 + ws) * 2 * HD;
 #pragma unroll
-            for (int i = 0; i < 4; ++i)
+        for (int i = 0; i < 8; ++i) {
+            f4v_t acc[4] = {zero, zero, zero, zero};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const s4v_t a = ld_frag(W3t + (16 * i + fr) * FP + 16 * k + fk);
+#pragma unroll
+                for (int j = 0; j < 4; ++j) acc[j] = mma(a, a2[k][j], acc[j]);
+            }
+            const f4v_t b = *(const f4v_t*)(bs + 2 * HD + 16 * i + fk);
+            int kp[4] = {-1, -1, -1, -1}, kn[4] = {-1, -1, -1, -1};
+#pragma unroll
+            for (int j = 0; j < 4; ++j) {
+                const uint2 u = __builtin_bit_cast(uint2, relu4(acc[j], b));
+                const int inv = 255 - (64 * ws + 16 * j + fr);
+                const int key[4] = {(int)((u.x & 0x7fffu) << 8) | inv, (int)((u.x >> 8) & 0x7fff00u) | inv,
+                                    (int)((u.y & 0x7fffu) << 8) | inv, (int)((u.y >> 8) & 0x7fff00u) | inv};
 #pragma unroll
                 for (int r = 0; r < 4; ++r) {
-                    float v = 1.0f * acc[i][j][r];
-                    v += bn;
-                    v = fmaxf(v, 0.0f);
-                    v = bf2f(f2bf(v));
-                    if (Sd[r0 + 16 * i + fk + r] >= 0.0f) bp = fmaxf(bp, v);
-                    else bq = fmaxf(bq, v);
+                    kp[r] = max(kp[r], pos[j] ? key[r] : -1);
+                    kn[r] = max(kn[r], pos[j] ? -1 : key[r]);
                 }
-            bp = fmaxf(bp, __shfl_xor(bp, 16));
-            bp = fmaxf(bp, __shfl_xor(bp, 32));
-            bq = fmaxf(bq, __shfl_xor(bq, 16));
-            bq = fmaxf(bq, __shfl_xor(bq, 32));
-            if (lane < 16) {
-                red[(0 * 4 + wv) * HD + n] = bp;
-                red[(1 * 4 + wv) * HD + n] = bq;
+            }
+#pragma unroll
+            for (int r = 0; r < 4; ++r) {
+                kp[r] = row_max<0x121>(row_max<0x122>(row_max<0x124>(row_max<0x128>(kp[r]))));
+                kn[r] = row_max<0x121>(row_max<0x122>(row_max<0x124>(row_max<0x128>(kn[r]))));
+            }
+            if (fr == 0) {
+                *(int4*)(rd + 16 * i + fk) = make_int4(kp[0], kp[1], kp[2], kp[3]);
+                *(int4*)(rd + HD + 16 * i + fk) = make_int4(kn[0], kn[1], kn[2], kn[3]);
             }
         }
-        __syncthreads();
-        {
-            const int side = tid >> 7, n = tid & (HD - 1);
-            float m = red[(side * 4 + 0) * HD + n];
-#pragma unroll
-            for (int q = 1; q < 4; ++q) m = fmaxf(m, red[(side * 4 + q) * HD + n]);
-            G[(long long)c * 2 * HD + tid] = m > -1e30f ? m : 0.0f;
+        __syncthreads();  // the next round writes the other half of red
+        const int cd = tid >> 8, q = tid & 255;
+        const long long co = 2ll * pr + cd;
+        if (co < C) {
+            const int* r0 = red + (round * 2 + cd) * 4 * 2 * HD + q;
+            const int m = max(max(r0[0], r0[2 * HD]), max(r0[4 * HD], r0[6 * HD]));
+            Hin[co * KH + q] = m >= 0 ? (bf16_t)(m >> 8) : (bf16_t)0;
+            if (arg) arg[co * 2 * HD + q] = m >= 0 ? (uint8_t)(255 - (m & 255)) : (uint8_t)0;
+            if (q < KH - 2 * HD) Hin[co * KH + 2 * HD + q] = q < 4 ? f2bf(planes[4 * co + q]) : (bf16_t)0;
         }
     }
+}
+
+// Operand tiles of the weight gradients, [group of 16 rows][tile][64 lanes]:
+// lane l holds channel l % 16 of rows 4 (l / 16) .. +3.
+constexpr int HT_HIN = 0, HT_B1 = 17, HT_B2 = 25, HT_D1 = 33, HT_D2 = 41, HT_DY = 49, HT_N = 50;      // head
+constexpr int ET_X = 0, ET_A1 = 1, ET_A2 = 9, ET_D3 = 17, ET_D2 = 25, ET_D1 = 33, ET_N = 41;          // encoder
+
+// Head, a wave per 16 candidates, weights from L2. Training adds the loss
+// terms, the head's backward (gb: the pooled features' gradients, zero where
+// the feature is) and the operand tiles. One launch instead of the three
+// forward GEMMs and, in training, six backward ones with their column sums.
+template <bool TRAIN>
+__global__ __launch_bounds__(256) void mlp_head_kernel(const bf16_t* Hin, int C, const bf16_t* Wt, const bf16_t* W,
+                                                       const float* Wf, float* Y, const float* target, float* err2,
+                                                       bf16_t* gb, s4v_t* tiles) {
+    const int lane = threadIdx.x & 63, grp = blockIdx.x * 4 + (threadIdx.x >> 6);
+    if (grp * 16 >= C) return;
+    const int fr = lane & 15, fk = 4 * (lane >> 4);
+    const long long c = 16ll * grp + fr;
+    const bool on = c < C;
+    const f4v_t zero = {0.f, 0.f, 0.f, 0.f};
+    const s4v_t z4 = {0, 0, 0, 0};
+    s4v_t h[17], b1[8], b2[8];
+#pragma unroll
+    for (int k = 0; k < 17; ++k) h[k] = on ? ld_frag(Hin + c * KH + 16 * k + fk) : z4;
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        f4v_t acc = zero;
+#pragma unroll
+        for (int k = 0; k < 17; ++k) acc = mma(ld_frag(Wt + P_H1 + (16 * i + fr) * KH + 16 * k + fk), h[k], acc);
+        b1[i] = relu4(acc, *(const f4v_t*)(Wf + P_C1 + 16 * i + fk));
+    }
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+        f4v_t acc = zero;
+#pragma unroll
+        for (int k = 0; k < 8; ++k) acc = mma(ld_frag(Wt + P_H2 + (16 * i + fr) * HD + 16 * k + fk), b1[k], acc);
+        b2[i] = relu4(acc, *(const f4v_t*)(Wf + P_C2 + 16 * i + fk));
+    }
+    f4v_t acc = zero;
+#pragma unroll
+    for (int k = 0; k < 8; ++k) acc = mma(ld_frag(Wt + P_H3 + fr * HD + 16 * k + fk), b2[k], acc);
+    const float y = acc[0] + Wf[P_C3];  // output 0: lanes of channels 0..3
+    if (fk == 0 && on) Y[c] = y;
+    if constexpr (TRAIN) {
+        s4v_t dy = z4;
+        if (fk == 0 && on) {
+            const float e = y - target[c];
+            err2[c] = e * e;
+            dy[0] = (short)f2bf(2.0f * e / (float)C);
+        }
+        s4v_t d2[8], d1[8];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) d2[i] = mask4(mma(ld_frag(W + P_H3 + (16 * i + fr) * NO + fk), dy, zero), b2[i]);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f4v_t v = zero;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v = mma(ld_frag(W + P_H2 + (16 * i + fr) * HD + 16 * k + fk), d2[k], v);
+            d1[i] = mask4(v, b1[i]);
+        }
+#pragma unroll
+        for (int i = 0; i < 16; ++i) {
+            f4v_t v = zero;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) v = mma(ld_frag(W + P_H1 + (16 * i + fr) * HD + 16 * k + fk), d1[k], v);
+            if (on) *(s4v_t*)(gb + c * 2 * HD + 16 * i + fk) = mask4(v, h[i]);
+        }
+        const s4v_t eye = identity_frag();
+        s4v_t* o = tiles + (long long)grp * HT_N * 64 + lane;
+#pragma unroll
+        for (int i = 0; i < 17; ++i) o[(HT_HIN + i) * 64] = transpose4(h[i], eye);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            o[(HT_B1 + i) * 64] = transpose4(b1[i], eye);
+            o[(HT_B2 + i) * 64] = transpose4(b2[i], eye);
+            o[(HT_D1 + i) * 64] = transpose4(d1[i], eye);
+            o[(HT_D2 + i) * 64] = transpose4(d2[i], eye);
+        }
+        o[HT_DY * 64] = transpose4(dy, eye);
+    }
+}
+
+// ---------------------------------------------------------------------------
+// Encoder backward. The max-pool passes a gradient to one sample per side and
+// channel, so of a candidate's 256 rows only the pooled ones - some 60 of them
+// - have any: the rest contribute exact zeros to every gradient. The pooled
+// rows of all candidates are listed (in order, by a scan, so sums do not
+// depend on timing), their two layers recomputed, and their gradients formed
+// densely over the list. Layer by layer over all 1.3 million rows of 5,056
+// candidates a training step took 11.5 ms, most of it in GEMMs, column sums
+// and the unpooling, all through memory.
+// ---------------------------------------------------------------------------
+// pooled rows of each candidate as a bit mask, and their number
+__global__ __launch_bounds__(256) void mlp_rows_mark(const bf16_t* Hin, const uint8_t* arg,
+                                                     unsigned long long* mask, int* cnt) {
+    __shared__ uint8_t mark[NS];
+    __shared__ int wc[4];
+    const long long c = blockIdx.x;
+    const int t = threadIdx.x;
+    mark[t] = 0;
+    __syncthreads();
+    if (Hin[c * KH + t] & 0x7fff) mark[arg[c * 2 * HD + t]] = 1;
+    __syncthreads();
+    const unsigned long long m = ballot(mark[t] != 0);
+    if ((t & 63) == 0) {
+        mask[c * 4 + (t >> 6)] = m;
+        wc[t >> 6] = __popcll(m);
+    }
+    __syncthreads();
+    if (t == 0) cnt[c] = wc[0] + wc[1] + wc[2] + wc[3];
+}
+
+// exclusive prefix of cnt, in place; *total; the list's tail up to a whole
+// pair of 16-row groups is empty rows
+__global__ __launch_bounds__(1024) void mlp_rows_scan(int* cnt, int C, int* total, int* list) {
+    __shared__ int ws[16];
+    int carry = 0;
+    const int t = threadIdx.x, wv = t >> 6;
+    for (int b = 0; b < C; b += 1024) {
+        const int v = b + t < C ? cnt[b + t] : 0;
+        const int incl = wave_incl_scan(v);
+        if ((t & 63) == 63) ws[wv] = incl;
+        __syncthreads();
+        int base = 0, all = 0;
+        for (int q = 0; q < 16; ++q) {
+            if (q < wv) base += ws[q];
+            all += ws[q];
+        }
+        if (b + t < C) cnt[b + t] = carry + base + incl - v;
+        carry += all;
+        __syncthreads();
+    }
+    if (t == 0) *total = carry;
+    const int end = (carry + 31) / 32 * 32;
+    if (carry + t < end) list[carry + t] = -1;
+}
+
+__global__ __launch_bounds__(256) void mlp_rows_fill(const unsigned long long* mask, const int* off, int* list) {
+    const long long c = blockIdx.x;
+    const int t = threadIdx.x, wv = t >> 6;
+    int o = off[c];
+    for (int q = 0; q < wv; ++q) o += __popcll(mask[c * 4 + q]);
+    const unsigned long long m = mask[c * 4 + wv];
+    if ((m >> (t & 63)) & 1ull) list[o + mask_rank(m)] = (int)(c * NS + t);
+}
+
+constexpr unsigned ROWS_LDS = 3 * HD * FP * 2 + HD * FP1 * 2 + 2 * HD * 4;
+
+// Recomputed layers and gradients of the listed rows: a persistent grid, two
+// 16-row groups per wave, so each weight fragment read from LDS feeds two
+// MFMAs. Writes the operand tiles.
+__global__ __launch_bounds__(512) void mlp_rows_kernel(const float* pts, const float* planes, const int* part_of,
+                                                       const bf16_t* Wt, const bf16_t* W, const float* Wf,
+                                                       const uint8_t* arg, const bf16_t* gb, const int* list,
+                                                       const int* total, s4v_t* tiles) {
+    extern __shared__ __align__(16) char fl[];
+    bf16_t* W2t = (bf16_t*)fl;      // [HD][FP] transposed
+    bf16_t* W2n = W2t + HD * FP;    // [HD][FP] as stored
+    bf16_t* W3n = W2n + HD * FP;    // [HD][FP] as stored
+    bf16_t* W1t = W3n + HD * FP;    // [HD][FP1]
+    float* bs = (float*)(W1t + HD * FP1);
+    const int tid = threadIdx.x, lane = tid & 63;
+    stage_rows(W2t, FP, Wt + P_W2, HD, HD);
+    stage_rows(W2n, FP, W + P_W2, HD, HD);
+    stage_rows(W3n, FP, W + P_W3, HD, HD);
+    stage_rows(W1t, FP1, Wt + P_W1, HD, KIN);
+    for (int i = tid; i < HD; i += 512) {
+        bs[i] = Wf[P_B1 + i];
+        bs[HD + i] = Wf[P_B2 + i];
+    }
+    __syncthreads();
+    const int fr = lane & 15, fk = 4 * (lane >> 4);
+    const f4v_t zero = {0.f, 0.f, 0.f, 0.f};
+    const s4v_t eye = identity_frag();
+    const int pairs = (*total + 31) / 32;
+    for (int pr = blockIdx.x * 8 + (tid >> 6); pr < pairs; pr += gridDim.x * 8) {
+        s4v_t x[2], a1[8][2], a2[8][2], d3[8][2];
+#pragma unroll
+        for (int j = 0; j < 2; ++j) {
+            const int row = list[32 * pr + 16 * j + fr];
+            const bool on = row >= 0;
+            const int c = on ? row / NS : 0, sm = on ? row % NS : 0;
+            const float* pl = planes + 4ll * c;
+            const float* pp = pts + ((long long)part_of[c] * NS + sm) * 3;
+            const float sd = pl[0] * pp[0] + pl[1] * pp[1] + pl[2] * pp[2] + pl[3];
+            x[j] = point_frag(pp, sd, on && fk == 0);
+            const uint8_t* ar = arg + (long long)c * 2 * HD + fk;
+            const bf16_t* gr = gb + (long long)c * 2 * HD + fk;
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                // a side without the feature has gradient 0, whatever its row
+                const uint32_t ap = *(const uint32_t*)(ar + 16 * k), an = *(const uint32_t*)(ar + HD + 16 * k);
+                const s4v_t gp = ld_frag(gr + 16 * k), gn = ld_frag(gr + HD + 16 * k);
+#pragma unroll
+                for (int q = 0; q < 4; ++q) {
+                    const int vp = (int)((ap >> (8 * q)) & 255u) == sm ? gp[q] : 0;
+                    const int vn = (int)((an >> (8 * q)) & 255u) == sm ? gn[q] : 0;
+                    d3[k][j][q] = (short)(on ? vp | vn : 0);
+                }
+            }
+        }
+        s4v_t* o = tiles + 2ll * pr * ET_N * 64 + lane;
+        auto put = [&](int tile, int j, s4v_t v) { o[(j * ET_N + tile) * 64] = transpose4(v, eye); };
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            const s4v_t a = ld_frag(W1t + (16 * i + fr) * FP1 + fk);
+            const f4v_t b = *(const f4v_t*)(bs + 16 * i + fk);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) a1[i][j] = relu4(mma(a, x[j], zero), b);
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f4v_t acc[2] = {zero, zero};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const s4v_t a = ld_frag(W2t + (16 * i + fr) * FP + 16 * k + fk);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[j] = mma(a, a1[k][j], acc[j]);
+            }
+            const f4v_t b = *(const f4v_t*)(bs + HD + 16 * i + fk);
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                a2[i][j] = relu4(acc[j], b);
+                put(ET_A2 + i, j, a2[i][j]);
+                put(ET_D3 + i, j, d3[i][j]);
+            }
+        }
+        s4v_t d2[8][2];
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f4v_t acc[2] = {zero, zero};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const s4v_t a = ld_frag(W3n + (16 * i + fr) * FP + 16 * k + fk);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[j] = mma(a, d3[k][j], acc[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) {
+                d2[i][j] = mask4(acc[j], a2[i][j]);
+                put(ET_D2 + i, j, d2[i][j]);
+                put(ET_A1 + i, j, a1[i][j]);
+            }
+        }
+#pragma unroll
+        for (int i = 0; i < 8; ++i) {
+            f4v_t acc[2] = {zero, zero};
+#pragma unroll
+            for (int k = 0; k < 8; ++k) {
+                const s4v_t a = ld_frag(W2n + (16 * i + fr) * FP + 16 * k + fk);
+#pragma unroll
+                for (int j = 0; j < 2; ++j) acc[j] = mma(a, d2[k][j], acc[j]);
+            }
+#pragma unroll
+            for (int j = 0; j < 2; ++j) put(ET_D1 + i, j, mask4(acc[j], a1[i][j]));
+        }
+#pragma unroll
+        for (int j = 0; j < 2; ++j) put(ET_X, j, x[j]);
+    }
+}
+
+// One weight gradient P^T Q over the rows of a tile table (np x nq tiles from
+// p0 / q0), and the bias gradient (column sums of Q) as a product with ones.
+// Workgroup z of nz takes groups z, z + nz, ...; a wave owns two of the P
+// tiles and all of Q; FP32 partial sums, added in order by mlp_grad_reduce.
+struct GradJob {
+    const s4v_t* tiles;
+    int stride;        // tiles per group
+    int p0, np, q0, nq;
+    const int* rows;   // rows on the device, or null
+    int groups;        // else the group count
+    int nz, block0;    // workgroups, the first one's index
+    float* part;       // [nz][np*16 x nq*16 (+ nq*16)]
+    int w_off, w_cols; // the gradient's place: w_off + row * w_cols + column
+    int b_off;         // the bias's, or -1
+};
+constexpr int GRAD_JOBS = 8;
+struct GradJobs {
+    GradJob j[GRAD_JOBS];
+};
+
+__global__ __launch_bounds__(256) void mlp_grad_kernel(GradJobs jobs) {
+    int ji = 0;
+#pragma unroll
+    for (int k = 1; k < GRAD_JOBS; ++k)
+        if ((int)blockIdx.x >= jobs.j[k].block0) ji = k;
+    const GradJob& J = jobs.j[ji];
+    const int z = blockIdx.x - J.block0;
+    const int lane = threadIdx.x & 63, wv = threadIdx.x >> 6;
+    const int i0 = 2 * wv;
+    if (i0 >= J.np) return;
+    const int groups = J.rows ? (*J.rows + 15) / 16 : J.groups;
+    const bool two = i0 + 1 < J.np, bias = J.b_off >= 0 && wv == 0;
+    const int nq = J.nq;
+    const f4v_t zero = {0.f, 0.f, 0.f, 0.f};
+    const s4v_t z4 = {0, 0, 0, 0};
+    const s4v_t ones = {0x3f80, 0x3f80, 0x3f80, 0x3f80};
+    f4v_t acc[2][8], ab[8];
+#pragma unroll
+    for (int j = 0; j < 8; ++j) acc[0][j] = acc[1][j] = ab[j] = zero;
+    const s4v_t* src = J.tiles + lane;
+    auto load = [&](int g, s4v_t (&p)[2], s4v_t (&q)[8]) {
+        const s4v_t* b = src + (long long)g * J.stride * 64;
+        p[0] = b[(J.p0 + i0) * 64];
+        p[1] = two ? b[(J.p0 + i0 + 1) * 64] : z4;
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = j < nq ? b[(J.q0 + j) * 64] : z4;
+    };
+    s4v_t p[2], q[8];
+    if (z < groups) load(z, p, q);
+    for (int g = z; g < groups; g += J.nz) {
+        s4v_t pn[2], qn[8];
+        load(min(g + J.nz, groups - 1), pn, qn);
+#pragma unroll
+        for (int j = 0; j < 8; ++j) {
+            acc[0][j] = mma(p[0], q[j], acc[0][j]);
+            acc[1][j] = mma(p[1], q[j], acc[1][j]);
+        }
+        if (bias)
+#pragma unroll
+            for (int j = 0; j < 8; ++j) ab[j] = mma(ones, q[j], ab[j]);
+        p[0] = pn[0];
+        p[1] = pn[1];
+#pragma unroll
+        for (int j = 0; j < 8; ++j) q[j] = qn[j];
+    }
+    const int fr = lane & 15, fk = 4 * (lane >> 4), cols = nq * 16, rows = J.np * 16;
+    float* o = J.part + (long long)z * (rows * cols + (J.b_off >= 0 ? cols : 0));
+#pragma unroll
+    for (int a = 0; a < 2; ++a) {
+        if (a && !two) break;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (j < nq)
+#pragma unroll
+                for (int r = 0; r < 4; ++r) o[(16 * (i0 + a) + fk + r) * cols + 16 * j + fr] = acc[a][j][r];
+    }
+    if (bias && fk == 0)
+#pragma unroll
+        for (int j = 0; j < 8; ++j)
+            if (j < nq) o[rows * cols + 16 * j + fr] = ab[j][0];
+}
+
+// Sums the partial gradients in order; the last row of workgroups also forms
+// the loss, the mean of the squared errors.
+__global__ __launch_bounds__(256) void mlp_grad_reduce(GradJobs jobs, float* g, const float* err2, int C, float* loss) {
+    const int tid = threadIdx.x;
+    if (blockIdx.y == GRAD_JOBS) {
+        __shared__ float red[4];
+        if (blockIdx.x) return;
+        float s = 0.0f;
+        for (int c = tid; c < C; c += 256) s += err2[c];
+        s = wave_sum_f(s);
+        if ((tid & 63) == 0) red[tid >> 6] = s;
+        __syncthreads();
+        if (tid == 0) loss[0] = (red[0] + red[1] + red[2] + red[3]) / (float)C;
+        return;
+    }
+    const GradJob& J = jobs.j[blockIdx.y];
+    const int cols = J.nq * 16, rows = J.np * 16, n = rows * cols + (J.b_off >= 0 ? cols : 0);
+    const int i = blockIdx.x * 256 + tid;
+    if (i >= n) return;
+    float s[4] = {0.f, 0.f, 0.f, 0.f};
+    int z = 0;
+    for (; z + 4 <= J.nz; z += 4)
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[u] += J.part[(long long)(z + u) * n + i];
+    for (; z < J.nz; ++z) s[0] += J.part[(long long)z * n + i];
+    const float v = (s[0] + s[1]) + (s[2] + s[3]);
+    if (i < rows * cols) g[J.w_off + (i / cols) * J.w_cols + i % cols] = v;
+    else g[J.b_off + i - rows * cols] = v;
 }
 
 // Split-K reduction with the GEMM's epilogue: C = alpha * sum_z part[z] ...
@@ -335,24 +730,6 @@ __global__ void mlp_splitk_reduce(GemmArgs g, int nz) {
     if (g.mask && !(bf2f(g.mask[(long long)m * g.ldm + n]) > 0.0f)) v = 0.0f;
     if (g.C) g.C[(long long)m * g.ldc + n] = v;
     if (g.Cb) g.Cb[(long long)m * g.ldcb + n] = f2bf(v);
-}
-
-// out[n] = sum over rows of D [R x N] (BF16): per block a 1024-row chunk of
-// 128 columns into part[chunk][n], then a sum over the chunks
-__global__ __launch_bounds__(128) void mlp_colsum_part(const bf16_t* D, int R, int N, float* part) {
-    const int n = blockIdx.x * 128 + threadIdx.x, r0 = blockIdx.y * 1024;
-    if (n >= N) return;
-    float s = 0.0f;
-    const int r1 = min(R, r0 + 1024);
-    for (int r = r0; r < r1; ++r) s += bf2f(D[(long long)r * N + n]);
-    part[(long long)blockIdx.y * N + n] = s;
-}
-__global__ void mlp_colsum_fin(const float* part, int chunks, int N, float* out) {
-    const int n = blockIdx.x * blockDim.x + threadIdx.x;
-    if (n >= N) return;
-    float s = 0.0f;
-    for (int c = 0; c < chunks; ++c) s += part[(long long)c * N + n];
-    out[n] = s;
 }
 
 // ---------------------------------------------------------------------------
@@ -379,27 +756,19 @@ __global__ void mlp_pack_points(const float* pts, const float* planes, const int
 }
 
 // per candidate and channel: max of A [C*NS x 128] over its rows with s >= 0
-// (G[c][j]) and with s < 0 (G[c][128 + j]); arg = the row, -1 (and 0) when a
-// side has no sample
-__global__ __launch_bounds__(HD) void mlp_maxpool(const bf16_t* A, const float* S, int C, float* G, int* arg) {
+// (G[c][j]) and with s < 0 (G[c][128 + j]); 0 when a side has no sample
+__global__ __launch_bounds__(HD) void mlp_maxpool(const bf16_t* A, const float* S, int C, float* G) {
     const int c = blockIdx.x, j = threadIdx.x;
     if (c >= C) return;
     float bp = -1e30f, bn = -1e30f;
-    int ip = -1, in = -1;
     for (int i = 0; i < NS; ++i) {
         const long long r = (long long)c * NS + i;
         const float v = bf2f(A[r * HD + j]);
-        if (S[r] >= 0.0f) {
-            if (v > bp) { bp = v; ip = (int)r; }
-        } else if (v > bn) {
-            bn = v;
-            in = (int)r;
-        }
+        if (S[r] >= 0.0f) bp = fmaxf(bp, v);
+        else bn = fmaxf(bn, v);
     }
-    G[(long long)c * 2 * HD + j] = ip >= 0 ? bp : 0.0f;
-    G[(long long)c * 2 * HD + HD + j] = in >= 0 ? bn : 0.0f;
-    arg[(long long)c * 2 * HD + j] = ip;
-    arg[(long long)c * 2 * HD + HD + j] = in;
+    G[(long long)c * 2 * HD + j] = bp > -1e30f ? bp : 0.0f;
+    G[(long long)c * 2 * HD + HD + j] = bn > -1e30f ? bn : 0.0f;
 }
 
 // head input [C x 272] BF16: g+, g-, plane (n, d), zeros
@@ -414,42 +783,23 @@ __global__ void mlp_head_input(const float* G, const float* planes, int C, bf16_
     Hin[i] = f2bf(v);
 }
 
-// loss = mean (y - t)^2 over the C candidates; dY [C x 16] BF16 (column 0)
-__global__ __launch_bounds__(256) void mlp_loss(const float* Y, const float* t, int C, bf16_t* dY, float* loss) {
-    __shared__ float red[4];
-    float s = 0.0f;
-    for (int c = threadIdx.x; c < C; c += 256) {
-        const float e = Y[(long long)c * NO] - t[c];
-        s += e * e;
-        for (int j = 0; j < NO; ++j) dY[(long long)c * NO + j] = j == 0 ? f2bf(2.0f * e / (float)C) : (bf16_t)0;
+// Place of parameter i in the transposed copy: each weight block [K x N] as
+// [N x K], everything else where it is.
+__device__ __forceinline__ int wt_index(int i) {
+    const int off[6] = {P_W1, P_W2, P_W3, P_H1, P_H2, P_H3}, K[6] = {KIN, HD, HD, KH, HD, HD},
+              N[6] = {HD, HD, HD, HD, HD, NO};
+    int r = i;
+#pragma unroll
+    for (int b = 0; b < 6; ++b) {
+        const int j = i - off[b];
+        if (j >= 0 && j < K[b] * N[b]) r = off[b] + (j % N[b]) * K[b] + j / N[b];
     }
-    for (int o = 32; o > 0; o >>= 1) s += __shfl_xor(s, o);
-    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = s;
-    __syncthreads();
-    if (threadIdx.x == 0) loss[0] = (red[0] + red[1] + red[2] + red[3]) / (float)C;
+    return r;
 }
 
-
-// dZ3 [C*NS x 128] BF16: each pooled gradient dHin[c][0, 256) back to its
-// max row, where the max was positive (ReLU)
-__global__ void mlp_unpool(const float* dHin, const int* arg, const bf16_t* A3, int C, bf16_t* dZ) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    const long long R = (long long)C * NS;
-    if (i >= R * HD) return;
-    const long long r = i / HD;
-    const int j = (int)(i % HD);
-    const long long c = r / NS;
-    float v = 0.0f;
-    if (bf2f(A3[i]) > 0.0f) {
-        if (arg[c * 2 * HD + j] == r) v += dHin[c * KH + j];
-        if (arg[c * 2 * HD + HD + j] == r) v += dHin[c * KH + HD + j];
-    }
-    dZ[i] = f2bf(v);
-}
-
-// Adam (FP32 master weights), then the BF16 copy used by the GEMMs
-__global__ void mlp_adam(float* w, const float* gr, float* m, float* v, bf16_t* wb, int n, float lr, float b1,
-                         float b2, float eps, float c1, float c2) {
+// Adam (FP32 master weights), then the BF16 copies used by the products
+__global__ void mlp_adam(float* w, const float* gr, float* m, float* v, bf16_t* wb, bf16_t* wt, int n, float lr,
+                         float b1, float b2, float eps, float c1, float c2) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
     if (i >= n) return;
     const float g = gr[i];
@@ -460,11 +810,14 @@ __global__ void mlp_adam(float* w, const float* gr, float* m, float* v, bf16_t* 
     const float upd = lr * (mi / c1) / (sqrtf(vi / c2) + eps);
     w[i] -= upd;
     wb[i] = f2bf(w[i]);
+    wt[wt_index(i)] = wb[i];
 }
 
-__global__ void mlp_to_bf16(const float* w, bf16_t* wb, int n) {
+__global__ void mlp_to_bf16(const float* w, bf16_t* wb, bf16_t* wt, int n) {
     const int i = blockIdx.x * blockDim.x + threadIdx.x;
-    if (i < n) wb[i] = f2bf(w[i]);
+    if (i >= n) return;
+    wb[i] = f2bf(w[i]);
+    wt[wt_index(i)] = wb[i];
 }
 
 // ---------------------------------------------------------------------------
@@ -570,11 +923,12 @@ __global__ __launch_bounds__(256) void mlp_sample_kernel(const SampleTask* tasks
 struct gpu_mlp {
     float* w;      // FP32 master weights [P_TOTAL]
     bf16_t* wb;    // BF16 copy
+    bf16_t* wt;    // BF16 copy, every weight block transposed
     float* g;      // gradients
     float* m;      // Adam moments
     float* v;
     int step;
-    // grow-only activations and split-K / column-sum partials
+    // grow-only activations and partial sums
     char* act;
     size_t act_cap;
     float* part;
@@ -631,26 +985,59 @@ int gemm(gpu_ctx_t ctx, gpu_mlp* mp, int M, int N, int K, const bf16_t* A, long 
 }
 
 struct Act {
-    bf16_t *X, *A1, *A2, *A3, *Hin, *B1, *B2, *dY, *dZ2h, *dZ1h, *dA3, *dZ2e, *dZ1e;
-    float *S, *G, *Y, *dHin, *loss, *csum;
-    size_t csum_cap;
-    int* arg;
+    // layer by layer
+    bf16_t *X, *A1, *A2, *A3, *B1, *B2;
+    float *S, *G, *Yw;
+    // fused
+    bf16_t* Hin;
+    float* Y;
+    // training
+    bf16_t* gb;
+    uint8_t* arg;
+    float *err2, *loss;
+    unsigned long long* mask;
+    int *off, *total, *list;
+    s4v_t *htiles, *etiles;
 };
 
-// activations of C candidates (C * NS encoder rows); `train` adds the
-// backward buffers
-int act_layout(gpu_ctx_t ctx, gpu_mlp* mp, int C, bool train, Act* a, bool fused = false) {
-    // the fused inference keeps the encoder rows (X, A1-A3, S) in LDS
-    const size_t R = fused ? 0 : (size_t)C * NS;
-    size_t need = 0;
-    auto sz = [&](size_t n, size_t e) { need += (n * e + 255) / 256 * 256; };
-    sz(R * KIN, 2); sz(R * HD, 2); sz(R * HD, 2); sz(R * HD, 2);
-    sz((size_t)C * KH, 2); sz((size_t)C * HD, 2); sz((size_t)C * HD, 2); sz((size_t)C * NO, 2);
-    if (train) { sz((size_t)C * HD, 2); sz((size_t)C * HD, 2); sz(R * HD, 2); sz(R * HD, 2); sz(R * HD, 2); }
-    sz(R, 4); sz((size_t)C * 2 * HD, 4); sz((size_t)C * NO, 4); sz((size_t)C * KH, 4); sz(64, 4);
-    sz((size_t)C * 2 * HD, 4);
-    const size_t csum = ((R + 1023) / 1024 + 1) * (size_t)HD;
-    if (train) sz(csum, 4);
+enum ActKind { ACT_LAYERS, ACT_FUSED, ACT_TRAIN };
+
+// Buffers of C candidates in the network's grow-only block. Training's largest
+// part is the encoder's operand tiles, for as many rows as there could be.
+int act_layout(gpu_ctx_t ctx, gpu_mlp* mp, int C, ActKind kind, Act* a) {
+    const size_t n = (size_t)C, R = n * NS;
+    auto carve_all = [&](char* p) -> size_t {
+        char* const p0 = p;
+        *a = Act{};
+        a->Hin = carve<bf16_t>(p, n * KH);
+        if (kind == ACT_LAYERS) {
+            a->X = carve<bf16_t>(p, R * KIN);
+            a->A1 = carve<bf16_t>(p, R * HD);
+            a->A2 = carve<bf16_t>(p, R * HD);
+            a->A3 = carve<bf16_t>(p, R * HD);
+            a->B1 = carve<bf16_t>(p, n * HD);
+            a->B2 = carve<bf16_t>(p, n * HD);
+            a->S = carve<float>(p, R);
+            a->G = carve<float>(p, n * 2 * HD);
+            a->Yw = carve<float>(p, n * NO);
+        } else {
+            a->Y = carve<float>(p, n);
+        }
+        if (kind == ACT_TRAIN) {
+            a->gb = carve<bf16_t>(p, n * 2 * HD);
+            a->arg = carve<uint8_t>(p, n * 2 * HD);
+            a->err2 = carve<float>(p, n);
+            a->loss = carve<float>(p, 64);
+            a->mask = carve<unsigned long long>(p, n * 4);
+            a->off = carve<int>(p, n);
+            a->total = carve<int>(p, 1);
+            a->list = carve<int>(p, R + 32);
+            a->htiles = carve<s4v_t>(p, (n + 15) / 16 * HT_N * 64);
+            a->etiles = carve<s4v_t>(p, (R / 16 + 2) * ET_N * 64);
+        }
+        return (size_t)(p - p0);
+    };
+    const size_t need = carve_all(nullptr);
     if (need > mp->act_cap) {
         if (mp->act) HIP_TRY(hipFree(mp->act));
         mp->act = nullptr;
@@ -658,38 +1045,13 @@ int act_layout(gpu_ctx_t ctx, gpu_mlp* mp, int C, bool train, Act* a, bool fused
         HIP_TRY(hipMalloc((void**)&mp->act, need));
         mp->act_cap = need;
     }
-    char* p = mp->act;
-    *a = Act{};
-    a->X = carve<bf16_t>(p, R * KIN);
-    a->A1 = carve<bf16_t>(p, R * HD);
-    a->A2 = carve<bf16_t>(p, R * HD);
-    a->A3 = carve<bf16_t>(p, R * HD);
-    a->Hin = carve<bf16_t>(p, (size_t)C * KH);
-    a->B1 = carve<bf16_t>(p, (size_t)C * HD);
-    a->B2 = carve<bf16_t>(p, (size_t)C * HD);
-    a->dY = carve<bf16_t>(p, (size_t)C * NO);
-    if (train) {
-        a->dZ2h = carve<bf16_t>(p, (size_t)C * HD);
-        a->dZ1h = carve<bf16_t>(p, (size_t)C * HD);
-        a->dA3 = carve<bf16_t>(p, R * HD);
-        a->dZ2e = carve<bf16_t>(p, R * HD);
-        a->dZ1e = carve<bf16_t>(p, R * HD);
-    }
-    a->S = carve<float>(p, R);
-    a->G = carve<float>(p, (size_t)C * 2 * HD);
-    a->Y = carve<float>(p, (size_t)C * NO);
-    a->dHin = carve<float>(p, (size_t)C * KH);
-    a->loss = carve<float>(p, 64);
-    a->arg = carve<int>(p, (size_t)C * 2 * HD);
-    if (train) {
-        a->csum = carve<float>(p, csum);
-        a->csum_cap = csum;
-    }
+    (void)carve_all(mp->act);
     return 0;
 }
 
-// forward over device inputs: points [P*NS x 3], planes [C x 4], part_of [C]
-int forward(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_planes, const int* d_part, int C,
+// layer by layer over device inputs: points [P*NS x 3], planes [C x 4],
+// part_of [C]; the scores in column 0 of Yw [C x NO]
+int forward_layers(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_planes, const int* d_part, int C,
             Act& a) {
     const int R = C * NS;
     const bf16_t* W = mp->wb;
@@ -703,7 +1065,7 @@ int forward(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_plane
         return rc;
     if (int rc = gemm(ctx, mp, R, HD, HD, a.A2, HD, 1, W + P_W3, HD, 1, Wf + P_B3, 1, nullptr, 0, nullptr, 0, a.A3, HD))
         return rc;
-    hipLaunchKernelGGL(mlp_maxpool, dim3((unsigned)C), dim3(HD), 0, ctx->stream, a.A3, a.S, C, a.G, a.arg);
+    hipLaunchKernelGGL(mlp_maxpool, dim3((unsigned)C), dim3(HD), 0, ctx->stream, a.A3, a.S, C, a.G);
     HIP_TRY(hipGetLastError());
     {
         const long long n = (long long)C * KH;
@@ -715,91 +1077,95 @@ int forward(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_plane
         return rc;
     if (int rc = gemm(ctx, mp, C, HD, HD, a.B1, HD, 1, W + P_H2, HD, 1, Wf + P_C2, 1, nullptr, 0, nullptr, 0, a.B2, HD))
         return rc;
-    return gemm(ctx, mp, C, NO, HD, a.B2, HD, 1, W + P_H3, NO, 1, Wf + P_C3, 0, nullptr, 0, a.Y, NO, nullptr, 0);
+    return gemm(ctx, mp, C, NO, HD, a.B2, HD, 1, W + P_H3, NO, 1, Wf + P_C3, 0, nullptr, 0, a.Yw, NO, nullptr, 0);
 }
 
-// forward through the fused point-layer kernel (inference only): G, then the head
+// point layers and pooling (arg: also the pooled rows)
+int encode(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_planes, const int* d_part, int C, Act& a) {
+    HIP_TRY(hipFuncSetAttribute((const void*)mlp_encode_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)ENC_LDS));
+    const int grid = std::max(1, std::min((C + 1) / 2, ctx->n_cu));
+    hipLaunchKernelGGL(mlp_encode_kernel, dim3((unsigned)grid), dim3(512), ENC_LDS, ctx->stream, d_pts, d_planes,
+                       d_part, C, (const bf16_t*)mp->wt, (const float*)mp->w, a.Hin, a.arg);
+    HIP_TRY(hipGetLastError());
+    return 0;
+}
+
+// inference through the fused kernels: the scores into d_out [C]
 int forward_fused(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_planes, const int* d_part, int C,
-                  Act& a) {
-    const bf16_t* W = mp->wb;
-    const float* Wf = mp->w;
-    HIP_TRY(hipFuncSetAttribute((const void*)mlp_encode_pool_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                (int)FUSED_LDS));
-    const int grid = std::max(1, std::min(C, ctx->n_cu));
-    hipLaunchKernelGGL(mlp_encode_pool_kernel, dim3((unsigned)grid), dim3(256), FUSED_LDS, ctx->stream, d_pts,
-                       d_planes, d_part, C, W, Wf, a.G);
+                  Act& a, float* d_out) {
+    if (int rc = encode(ctx, mp, d_pts, d_planes, d_part, C, a)) return rc;
+    hipLaunchKernelGGL(mlp_head_kernel<false>, dim3((unsigned)((C + 63) / 64)), dim3(256), 0, ctx->stream,
+                       (const bf16_t*)a.Hin, C, (const bf16_t*)mp->wt, (const bf16_t*)mp->wb, (const float*)mp->w, d_out,
+                       (const float*)nullptr, (float*)nullptr, (bf16_t*)nullptr, (s4v_t*)nullptr);
     HIP_TRY(hipGetLastError());
-    {
-        const long long n = (long long)C * KH;
-        hipLaunchKernelGGL(mlp_head_input, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, a.G,
-                           d_planes, C, a.Hin);
-        HIP_TRY(hipGetLastError());
-    }
-    if (int rc = gemm(ctx, mp, C, HD, KH, a.Hin, KH, 1, W + P_H1, HD, 1, Wf + P_C1, 1, nullptr, 0, nullptr, 0, a.B1, HD))
-        return rc;
-    if (int rc = gemm(ctx, mp, C, HD, HD, a.B1, HD, 1, W + P_H2, HD, 1, Wf + P_C2, 1, nullptr, 0, nullptr, 0, a.B2, HD))
-        return rc;
-    return gemm(ctx, mp, C, NO, HD, a.B2, HD, 1, W + P_H3, NO, 1, Wf + P_C3, 0, nullptr, 0, a.Y, NO, nullptr, 0);
+    return 0;
 }
 
-// gradients of the mean squared error into mp->g (after forward)
-int backward(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_t, int C, Act& a) {
-    const int R = C * NS;
-    // column sums use the part of the activation block reserved for them
-    float* colsum_ws = a.csum;
-    const size_t colsum_cap = a.csum_cap;
-    const bf16_t* W = mp->wb;
-    float* g = mp->g;
-    hipLaunchKernelGGL(mlp_loss, dim3(1), dim3(256), 0, ctx->stream, a.Y, d_t, C, a.dY, a.loss);
+// forward, loss and gradients of the mean squared error (into mp->g)
+int train_grads(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_planes, const int* d_part,
+                const float* d_t, int C, Act& a) {
+    const bf16_t *wt = mp->wt, *wb = mp->wb;
+    const float* wf = mp->w;
+    if (int rc = encode(ctx, mp, d_pts, d_planes, d_part, C, a)) return rc;
+    hipLaunchKernelGGL(mlp_head_kernel<true>, dim3((unsigned)((C + 63) / 64)), dim3(256), 0, ctx->stream,
+                       (const bf16_t*)a.Hin, C, wt, wb, wf, a.Y, d_t, a.err2, a.gb, a.htiles);
     HIP_TRY(hipGetLastError());
-    auto colsum = [&](const bf16_t* D, int rows, int N, float* out) -> int {
-        const int chunks = (rows + 1023) / 1024;
-        float* part = colsum_ws;
-        REQUIRE(part && (size_t)chunks * N <= colsum_cap, "mlp: column-sum workspace too small");
-        hipLaunchKernelGGL(mlp_colsum_part, dim3((unsigned)((N + 127) / 128), (unsigned)chunks), dim3(128), 0,
-                           ctx->stream, D, rows, N, part);
-        HIP_TRY(hipGetLastError());
-        hipLaunchKernelGGL(mlp_colsum_fin, dim3((unsigned)((N + 127) / 128)), dim3(128), 0, ctx->stream, part, chunks,
-                           N, out);
-        HIP_TRY(hipGetLastError());
-        return 0;
+    hipLaunchKernelGGL(mlp_rows_mark, dim3((unsigned)C), dim3(256), 0, ctx->stream, (const bf16_t*)a.Hin,
+                       (const uint8_t*)a.arg, a.mask, a.off);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(mlp_rows_scan, dim3(1), dim3(1024), 0, ctx->stream, a.off, C, a.total, a.list);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(mlp_rows_fill, dim3((unsigned)C), dim3(256), 0, ctx->stream,
+                       (const unsigned long long*)a.mask, (const int*)a.off, a.list);
+    HIP_TRY(hipGetLastError());
+    HIP_TRY(hipFuncSetAttribute((const void*)mlp_rows_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)ROWS_LDS));
+    const int grid = std::max(1, std::min((C * (NS / 32) + 7) / 8, ctx->n_cu));
+    hipLaunchKernelGGL(mlp_rows_kernel, dim3((unsigned)grid), dim3(512), ROWS_LDS, ctx->stream, d_pts, d_planes, d_part,
+                       wt, wb, wf, (const uint8_t*)a.arg, (const bf16_t*)a.gb, (const int*)a.list,
+                       (const int*)a.total, a.etiles);
+    HIP_TRY(hipGetLastError());
+    // the weight gradients: enough workgroups per job that each sees a few
+    // dozen groups at most (the loads of a group are its latency)
+    const int hg = (C + 15) / 16, eg = C * (NS / 16);
+    const int nzh = std::max(1, std::min(hg / 8, 32)), nze = std::max(1, std::min(eg / 16, 256));
+    GradJobs jobs{};
+    size_t floats = 0;
+    int blocks = 0, most = 0;
+    auto job = [&](int k, bool enc, int p0, int np, int q0, int nq, int w_off, int w_cols, int b_off) {
+        GradJob& J = jobs.j[k];
+        J.tiles = enc ? a.etiles : a.htiles;
+        J.stride = enc ? ET_N : HT_N;
+        J.p0 = p0; J.np = np; J.q0 = q0; J.nq = nq;
+        J.rows = enc ? a.total : nullptr;
+        J.groups = hg;
+        J.nz = enc ? nze : nzh;
+        J.block0 = blocks;
+        J.w_off = w_off; J.w_cols = w_cols; J.b_off = b_off;
+        blocks += J.nz;
+        const int n = np * nq * 256 + (b_off >= 0 ? nq * 16 : 0);
+        most = std::max(most, n);
+        J.part = (float*)(uintptr_t)floats;  // its offset until the block is known
+        floats += (size_t)J.nz * n;
     };
-    // head
-    if (int rc = gemm(ctx, mp, HD, NO, C, a.B2, 1, HD, a.dY, NO, 1, nullptr, 0, nullptr, 0, g + P_H3, NO, nullptr, 0))
-        return rc;
-    if (int rc = colsum(a.dY, C, NO, g + P_C3)) return rc;
-    if (int rc = gemm(ctx, mp, C, HD, NO, a.dY, NO, 1, W + P_H3, 1, NO, nullptr, 0, a.B2, HD, nullptr, 0, a.dZ2h, HD))
-        return rc;
-    if (int rc = gemm(ctx, mp, HD, HD, C, a.B1, 1, HD, a.dZ2h, HD, 1, nullptr, 0, nullptr, 0, g + P_H2, HD, nullptr, 0))
-        return rc;
-    if (int rc = colsum(a.dZ2h, C, HD, g + P_C2)) return rc;
-    if (int rc = gemm(ctx, mp, C, HD, HD, a.dZ2h, HD, 1, W + P_H2, 1, HD, nullptr, 0, a.B1, HD, nullptr, 0, a.dZ1h, HD))
-        return rc;
-    if (int rc = gemm(ctx, mp, KH, HD, C, a.Hin, 1, KH, a.dZ1h, HD, 1, nullptr, 0, nullptr, 0, g + P_H1, HD, nullptr, 0))
-        return rc;
-    if (int rc = colsum(a.dZ1h, C, HD, g + P_C1)) return rc;
-    if (int rc = gemm(ctx, mp, C, KH, HD, a.dZ1h, HD, 1, W + P_H1, 1, HD, nullptr, 0, nullptr, 0, a.dHin, KH, nullptr, 0))
-        return rc;
-    // encoder
-    {
-        const long long n = (long long)R * HD;
-        hipLaunchKernelGGL(mlp_unpool, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, a.dHin, a.arg,
-                           a.A3, C, a.dA3);
-        HIP_TRY(hipGetLastError());
-    }
-    if (int rc = gemm(ctx, mp, HD, HD, R, a.A2, 1, HD, a.dA3, HD, 1, nullptr, 0, nullptr, 0, g + P_W3, HD, nullptr, 0))
-        return rc;
-    if (int rc = colsum(a.dA3, R, HD, g + P_B3)) return rc;
-    if (int rc = gemm(ctx, mp, R, HD, HD, a.dA3, HD, 1, W + P_W3, 1, HD, nullptr, 0, a.A2, HD, nullptr, 0, a.dZ2e, HD))
-        return rc;
-    if (int rc = gemm(ctx, mp, HD, HD, R, a.A1, 1, HD, a.dZ2e, HD, 1, nullptr, 0, nullptr, 0, g + P_W2, HD, nullptr, 0))
-        return rc;
-    if (int rc = colsum(a.dZ2e, R, HD, g + P_B2)) return rc;
-    if (int rc = gemm(ctx, mp, R, HD, HD, a.dZ2e, HD, 1, W + P_W2, 1, HD, nullptr, 0, a.A1, HD, nullptr, 0, a.dZ1e, HD))
-        return rc;
-    if (int rc = gemm(ctx, mp, KIN, HD, R, a.X, 1, KIN, a.dZ1e, HD, 1, nullptr, 0, nullptr, 0, g + P_W1, HD, nullptr, 0))
-        return rc;
-    return colsum(a.dZ1e, R, HD, g + P_B1);
+    job(0, true, ET_A2, 8, ET_D3, 8, P_W3, HD, P_B3);
+    job(1, true, ET_A1, 8, ET_D2, 8, P_W2, HD, P_B2);
+    job(2, true, ET_X, 1, ET_D1, 8, P_W1, HD, P_B1);
+    job(3, false, HT_HIN, 8, HT_D1, 8, P_H1, HD, P_C1);
+    job(4, false, HT_HIN + 8, 8, HT_D1, 8, P_H1 + 128 * HD, HD, -1);
+    job(5, false, HT_HIN + 16, 1, HT_D1, 8, P_H1 + 256 * HD, HD, -1);
+    job(6, false, HT_B1, 8, HT_D2, 8, P_H2, HD, P_C2);
+    job(7, false, HT_B2, 8, HT_DY, 1, P_H3, NO, P_C3);
+    float* part = part_ws(ctx, mp, floats);
+    REQUIRE(part, "mlp: partial-sum workspace allocation failed");
+    for (GradJob& J : jobs.j) J.part = part + (size_t)(uintptr_t)J.part;
+    hipLaunchKernelGGL(mlp_grad_kernel, dim3((unsigned)blocks), dim3(256), 0, ctx->stream, jobs);
+    HIP_TRY(hipGetLastError());
+    hipLaunchKernelGGL(mlp_grad_reduce, dim3((unsigned)((most + 255) / 256), GRAD_JOBS + 1), dim3(256), 0, ctx->stream,
+                       jobs, mp->g, (const float*)a.err2, C, a.loss);
+    HIP_TRY(hipGetLastError());
+    return 0;
 }
 
 // Inputs staged on the device (points [P*NS*3], planes [C*4], part_of, cand
@@ -863,13 +1229,15 @@ int mlp_forward_dev(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, int P, const
     const bool fused = mlp_fused_on() != 0;
     const int slice = fused ? 65536 : 8192;
     Act a;
-    if (int rc = act_layout(ctx, mp, std::min(slice, C), false, &a, fused)) return rc;
+    if (int rc = act_layout(ctx, mp, std::min(slice, C), fused ? ACT_FUSED : ACT_LAYERS, &a)) return rc;
     for (int c0 = 0; c0 < C; c0 += slice) {
         const int n = std::min(slice, C - c0);
-        if (int rc = fused ? forward_fused(ctx, mp, d_pts, d_planes + 4ll * c0, d_part + c0, n, a)
-                           : forward(ctx, mp, d_pts, d_planes + 4ll * c0, d_part + c0, n, a))
-            return rc;
-        HIP_TRY(hipMemcpy2DAsync(d_out + c0, 4, a.Y, 4 * NO, 4, n, hipMemcpyDeviceToDevice, ctx->stream));
+        if (fused) {
+            if (int rc = forward_fused(ctx, mp, d_pts, d_planes + 4ll * c0, d_part + c0, n, a, d_out + c0)) return rc;
+            continue;
+        }
+        if (int rc = forward_layers(ctx, mp, d_pts, d_planes + 4ll * c0, d_part + c0, n, a)) return rc;
+        HIP_TRY(hipMemcpy2DAsync(d_out + c0, 4, a.Yw, 4 * NO, 4, n, hipMemcpyDeviceToDevice, ctx->stream));
     }
     return 0;
 }
@@ -934,6 +1302,7 @@ int gpu_mlp_create(gpu_ctx_t ctx, const float* params, int seed, gpu_mlp_t* out)
     REQUIRE(m, "out of host memory");
     const size_t fb = sizeof(float) * P_TOTAL;
     if (hipMalloc((void**)&m->w, fb) != hipSuccess || hipMalloc((void**)&m->wb, 2 * P_TOTAL) != hipSuccess ||
+        hipMalloc((void**)&m->wt, 2 * P_TOTAL) != hipSuccess ||
         hipMalloc((void**)&m->g, fb) != hipSuccess || hipMalloc((void**)&m->m, fb) != hipSuccess ||
         hipMalloc((void**)&m->v, fb) != hipSuccess) {
         gpu_mlp_destroy(ctx, m);
@@ -944,7 +1313,7 @@ int gpu_mlp_create(gpu_ctx_t ctx, const float* params, int seed, gpu_mlp_t* out)
     HIP_TRY(hipMemsetAsync(m->g, 0, fb, ctx->stream));
     HIP_TRY(hipMemsetAsync(m->m, 0, fb, ctx->stream));
     HIP_TRY(hipMemsetAsync(m->v, 0, fb, ctx->stream));
-    hipLaunchKernelGGL(mlp_to_bf16, dim3((P_TOTAL + 255) / 256), dim3(256), 0, ctx->stream, m->w, m->wb, P_TOTAL);
+    hipLaunchKernelGGL(mlp_to_bf16, dim3((P_TOTAL + 255) / 256), dim3(256), 0, ctx->stream, m->w, m->wb, m->wt, P_TOTAL);
     HIP_TRY(hipGetLastError());
     HIP_TRY(hipStreamSynchronize(ctx->stream));
     *out = m;
@@ -956,6 +1325,7 @@ void gpu_mlp_destroy(gpu_ctx_t ctx, gpu_mlp_t m) {
     if (ctx) (void)hipStreamSynchronize(ctx->stream);
     if (m->w) (void)hipFree(m->w);
     if (m->wb) (void)hipFree(m->wb);
+    if (m->wt) (void)hipFree(m->wt);
     if (m->g) (void)hipFree(m->g);
     if (m->m) (void)hipFree(m->m);
     if (m->v) (void)hipFree(m->v);
@@ -999,9 +1369,8 @@ int gpu_mlp_train_step(gpu_ctx_t ctx, gpu_mlp_t m, const float* points, int n_pa
     std::vector<int> coff;
     if (int rc = s.load(ctx, points, n_parts, planes, part_of, n_cand, targets, coff)) return stage_err(ctx, rc);
     Act a;
-    if (int rc = act_layout(ctx, m, n_cand, true, &a)) return rc;
-    if (int rc = forward(ctx, m, s.pts, s.planes, s.part, n_cand, a)) return rc;
-    if (int rc = backward(ctx, m, s.t, n_cand, a)) return rc;
+    if (int rc = act_layout(ctx, m, n_cand, ACT_TRAIN, &a)) return rc;
+    if (int rc = train_grads(ctx, m, s.pts, s.planes, s.part, s.t, n_cand, a)) return rc;
     if (out_grads)
         HIP_TRY(hipMemcpyAsync(out_grads, m->g, sizeof(float) * P_TOTAL, hipMemcpyDeviceToHost, ctx->stream));
     if (apply) {
@@ -1009,7 +1378,7 @@ int gpu_mlp_train_step(gpu_ctx_t ctx, gpu_mlp_t m, const float* points, int n_pa
         const float b1 = 0.9f, b2 = 0.999f;
         const float c1 = 1.0f - std::pow(b1, (float)m->step), c2 = 1.0f - std::pow(b2, (float)m->step);
         hipLaunchKernelGGL(mlp_adam, dim3((P_TOTAL + 255) / 256), dim3(256), 0, ctx->stream, m->w, m->g, m->m, m->v,
-                           m->wb, P_TOTAL, lr, b1, b2, 1e-8f, c1, c2);
+                           m->wb, m->wt, P_TOTAL, lr, b1, b2, 1e-8f, c1, c2);
         HIP_TRY(hipGetLastError());
     }
     float loss = 0.0f;
