@@ -57,7 +57,22 @@ struct PcResult {
     int has_box;  // 1: PcLDS::boxr holds both halves' vertex bounds (LDS-resident cut, status 0)
 };
 
+// Boundaries of up to PC_CAP_LDS edges (and polygons of as many vertices) are
+// linked, labelled and ear-clipped in LDS.
+constexpr int PC_CAP_LDS = 512;
+
 struct PcLDS {
+    union {
+        struct {  // boundary edges
+            uint16_t succ[PC_CAP_LDS], lab[PC_CAP_LDS], rank[PC_CAP_LDS], jmp[PC_CAP_LDS];
+            int tmp[PC_CAP_LDS];
+        } e;
+        struct {  // the polygon being clipped
+            float u[PC_CAP_LDS], v[PC_CAP_LDS];
+            uint16_t prv[PC_CAP_LDS], nxt[PC_CAP_LDS];
+        } c;
+    };
+    int flag[2];
     int ired[PC_T / 64];
     double dred[PC_T / 64];
     int cnt[8];
@@ -204,111 +219,162 @@ __device__ __forceinline__ bool pc_pt_in_tri(P2 X, P2 A, P2 B, P2 C) {
 // vertex is clipped when it is reflex only by rounding (a sliver: cross above
 // -1e-6 of the squared extent); otherwise the cap fails (-1). Writes n - 2
 // triangles (vertex ids) to out_tris and returns that count.
-__device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv, int* nxt, uint8_t* unused,
-                                 int* out_tris) {
-    (void)unused;
+//
+// A serial chain: a step's vertex follows from the last step's verdict. With
+// LDS (up to PC_CAP_LDS vertices) the ring and the coordinates live in LDS and
+// every lane keeps its share of the vertices in registers; the candidate's
+// corners are carried from step to step, so a step costs two dependent LDS
+// reads and the containment test, whose distance checks run only where some
+// vertex is in the triangle. Triangles are written as ring positions and
+// translated afterwards (a load per clip would stall the wave). With the ring
+// in global memory (larger polygons) a step is two dependent memory reads.
+template <bool LDS>
+__device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv, int* nxt, int* out_tris, PcLDS* s) {
     const int lane = lane_id();
     if (n < 3) return 0;
+    auto P = [&](int i) { return LDS ? P2{s->c.u[i], s->c.v[i]} : uv[i]; };
+    auto next = [&](int i) -> int { return LDS ? (int)s->c.nxt[i] : nxt[i]; };
+    auto prev = [&](int i) -> int { return LDS ? (int)s->c.prv[i] : prv[i]; };
+    auto order = [&] {  // one wave: LDS operations complete in order
+        if (LDS) {
+            __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+            __builtin_amdgcn_wave_barrier();
+        } else {
+            __threadfence_block();
+        }
+    };
+    // lane l keeps vertices l + 64 k in registers with a bit each that is set
+    // once the vertex is removed (or was never there)
+    constexpr int R = LDS ? PC_CAP_LDS / 64 : 1;
+    float ru[R], rv[R];
+    uint32_t gone = 0;
     float mnu = 3.4e38f, mxu = -3.4e38f, mnv = 3.4e38f, mxv = -3.4e38f;
-    for (int i = lane; i < n; i += 64) {
-        mnu = fminf(mnu, uv[i].u); mxu = fmaxf(mxu, uv[i].u);
-        mnv = fminf(mnv, uv[i].v); mxv = fmaxf(mxv, uv[i].v);
-        prv[i] = i == 0 ? n - 1 : i - 1;
-        nxt[i] = i == n - 1 ? 0 : i + 1;
+    auto init = [&](int i) {
+        const P2 x = uv[i];
+        mnu = fminf(mnu, x.u); mxu = fmaxf(mxu, x.u);
+        mnv = fminf(mnv, x.v); mxv = fmaxf(mxv, x.v);
+        const int before = i == 0 ? n - 1 : i - 1, after = i == n - 1 ? 0 : i + 1;
+        if (LDS) {
+            s->c.u[i] = x.u;
+            s->c.v[i] = x.v;
+            s->c.prv[i] = (uint16_t)before;
+            s->c.nxt[i] = (uint16_t)after;
+        } else {
+            prv[i] = before;
+            nxt[i] = after;
+        }
+        return x;
+    };
+    if constexpr (LDS) {
+#pragma unroll
+        for (int k = 0; k < R; ++k) {
+            const int i = lane + 64 * k;
+            ru[k] = rv[k] = 0.0f;
+            if (i < n) {
+                const P2 x = init(i);
+                ru[k] = x.u;
+                rv[k] = x.v;
+            } else {
+                gone |= 1u << k;
+            }
+        }
+    } else {
+        for (int i = lane; i < n; i += 64) (void)init(i);
     }
     mnu = wave_min_f(mnu); mxu = wave_max_f(mxu); mnv = wave_min_f(mnv); mxv = wave_max_f(mxv);
     const float ext = fmaxf(mxu - mnu, mxv - mnv);
     const float sliver = -1e-6f * ext * ext;
-    // up to 64 R vertices: lane l keeps vertices l + 64 k in registers with a
-    // removed bit each (a clipped vertex is exactly one whose predecessor no
-    // longer links to it), so the ear test reads no LDS
-    constexpr int R = 8;
-    const bool regs = n <= 64 * R;
-    float ru[R], rv[R];
-    uint32_t rem = 0;
-#pragma unroll
-    for (int k = 0; k < R; ++k) {
-        const int i = lane + 64 * k;
-        ru[k] = 0.0f;
-        rv[k] = 0.0f;
-        if (regs && i < n) { ru[k] = uv[i].u; rv[k] = uv[i].v; }
-    }
-    __threadfence_block();
-    auto conv = [&](int p, int c, int q) { return cross2(uv[p], uv[c], uv[q]); };
+    order();
+    auto bit = [&](int i) { return lane == (i & 63) ? 1u << (i >> 6) : 0u; };
     int nt = 0, remaining = n, cur = 0, lap = 0;
+    int p = prev(0), q = next(0);
+    P2 A = P(p), B = P(cur), C = P(q);
     while (remaining > 3) {
-        int p = prv[cur], q = nxt[cur];
-        const float cr = conv(p, cur, q);
+        const float cr = cross2(A, B, C);
         bool ear;
         if (lap >= remaining) {
             // a lap without an ear: least reflex vertex, first in ring order from cur
             int best = cur, c = cur;
             float bc = cr;
             for (int k = 0; k < remaining; ++k) {
-                const float x = conv(prv[c], c, nxt[c]);
+                const float x = cross2(P(prev(c)), P(c), P(next(c)));
                 if (x > bc) { bc = x; best = c; }
-                c = nxt[c];
+                c = next(c);
             }
             if (bc < sliver) return -1;
             cur = best;
-            p = prv[cur];
-            q = nxt[cur];
+            p = prev(cur);
+            q = next(cur);
+            A = P(p);
+            C = P(q);
             ear = true;
         } else if (cr < -1e-9f) {
             ear = false;
         } else if (cr <= 1e-9f) {
             ear = true;
         } else {
-            const P2 A = uv[p], B = uv[cur], C = uv[q];
-            bool bad = false;
-            auto inside = [&](const P2& X) {
+            auto apart = [&](const P2& X) {
                 return fabsf(X.u - A.u) + fabsf(X.v - A.v) > 1e-6f && fabsf(X.u - B.u) + fabsf(X.v - B.v) > 1e-6f &&
-                       fabsf(X.u - C.u) + fabsf(X.v - C.v) > 1e-6f && pc_pt_in_tri(X, A, B, C);
+                       fabsf(X.u - C.u) + fabsf(X.v - C.v) > 1e-6f;
             };
-            if (regs) {
+            bool bad = false;
+            if constexpr (LDS) {
+                const uint32_t skip = gone | bit(p) | bit(cur) | bit(q);
 #pragma unroll
                 for (int k = 0; k < R; ++k) {
-                    const int i = lane + 64 * k;
-                    if (i >= n || ((rem >> k) & 1u) || i == p || i == cur || i == q) continue;
-                    if (inside(P2{ru[k], rv[k]})) bad = true;
+                    if (64 * k >= n) break;
+                    const P2 X{ru[k], rv[k]};
+                    const bool in = pc_pt_in_tri(X, A, B, C) && !((skip >> k) & 1u);
+                    if (ballot(in)) bad |= in && apart(X);
                 }
             } else {
                 for (int i = lane; i < n; i += 64) {
                     if (i == p || i == cur || i == q) continue;
                     if (nxt[prv[i]] != i) continue;  // removed
-                    if (inside(uv[i])) bad = true;
+                    const P2 X = uv[i];
+                    if (apart(X) && pc_pt_in_tri(X, A, B, C)) bad = true;
                 }
             }
             ear = !__any(bad);
         }
         if (ear) {
             if (lane == 0) {
-                out_tris[3 * nt] = poly[p];
-                out_tris[3 * nt + 1] = poly[cur];
-                out_tris[3 * nt + 2] = poly[q];
-                nxt[p] = q;
-                prv[q] = p;
+                out_tris[3 * nt] = p;
+                out_tris[3 * nt + 1] = cur;
+                out_tris[3 * nt + 2] = q;
+                if (LDS) {
+                    s->c.nxt[p] = (uint16_t)q;
+                    s->c.prv[q] = (uint16_t)p;
+                } else {
+                    nxt[p] = q;
+                    prv[q] = p;
+                }
             }
-            if (lane == (cur & 63)) rem |= 1u << (cur >> 6);
-            __threadfence_block();
+            if (LDS) gone |= bit(cur);
+            order();
             ++nt;
             --remaining;
-            cur = q;
             lap = 0;
         } else {
-            cur = q;
+            p = cur;
+            A = B;
             ++lap;
         }
+        cur = q;
+        B = C;
+        q = next(q);
+        C = P(q);
     }
     if (remaining == 3) {
-        const int p = prv[cur], q = nxt[cur];
         if (lane == 0) {
-            out_tris[3 * nt] = poly[p];
-            out_tris[3 * nt + 1] = poly[cur];
-            out_tris[3 * nt + 2] = poly[q];
+            out_tris[3 * nt] = p;
+            out_tris[3 * nt + 1] = cur;
+            out_tris[3 * nt + 2] = q;
         }
         ++nt;
     }
+    __threadfence_block();
+    for (int i = lane; i < 3 * nt; i += 64) out_tris[i] = poly[out_tris[i]];
     __threadfence_block();
     return nt;
 }
@@ -331,7 +397,6 @@ struct PcCapWork {
     int* prv;                // [W] ear-clip ring
     int* nxt;                // [W]
     int* capbuf;             // [3W] cap triangles
-    uint8_t* refl;           // [W] reflex flags
     int* extra;              // [n_extra] caller's per-triangle scratch
     uint32_t H;
 };
@@ -346,7 +411,7 @@ __device__ __forceinline__ uint32_t pc_cap_hash_size(int E) {
 __device__ __forceinline__ unsigned long long pc_cap_bytes(unsigned long long E, uint32_t H, unsigned long long n_extra) {
     const unsigned long long W = E + 2ull * PC_MAX_LOOPS + 4ull;
     return 8ull * H + 8ull * E + 4ull * E * 7 + 4ull * E + 8ull * E + W * (4ull + 8ull + 4ull + 4ull + 12ull) +
-           al16(W) + 4ull * n_extra + 256ull;
+           16ull + 4ull * n_extra + 256ull;
 }
 __device__ inline PcCapWork pc_cap_carve(char* C, unsigned long long E, uint32_t H) {
     const unsigned long long W = E + 2ull * PC_MAX_LOOPS + 4ull;
@@ -368,9 +433,134 @@ __device__ inline PcCapWork pc_cap_carve(char* C, unsigned long long E, uint32_t
     w.prv = (int*)(w.wuv + W);
     w.nxt = w.prv + W;
     w.capbuf = w.nxt + W;
-    w.refl = (uint8_t*)(w.capbuf + 3 * W);
-    w.extra = (int*)(w.refl + al16(W));
+    w.extra = w.capbuf + 3 * W;
     return w;
+}
+
+// Boundary loops: the edges' successors, the loops they form (numbered by
+// their lowest edge), and the loops' vertices laid out loop by loop in poly,
+// reversed (a cap edge runs b -> a for boundary edge (a, b)). Arrays of nb
+// entries in LDS (nb <= PC_CAP_LDS) or global memory; jl and jr are the global
+// ones' second buffers. False when the boundary is open or has too many loops.
+// Everything but a boundary with touching loops is block-parallel: walking the
+// edges on one thread was a chain of two to three dependent reads per edge,
+// half of a cut's time.
+template <bool LDS, class I, class F>
+__device__ inline bool pc_loops(const int2* be, int nb, F successor, I* succ, I* lab, I* rank, I* jmp, int* tmp, I* jl,
+                                I* jr, int* poly, PcLDS* s) {
+    constexpr int PER = PC_CAP_LDS / PC_T;
+    const int tid = threadIdx.x;
+    if (tid < 2) s->flag[tid] = 0;
+    __syncthreads();
+    for (int j = tid; j < nb; j += PC_T) {
+        const int e = successor(j);
+        if (e < 0) s->flag[0] = 1;
+        succ[j] = (I)(e < 0 ? 0 : e);
+        tmp[j] = 0;
+    }
+    __syncthreads();
+    if (s->flag[0]) return false;  // open boundary: the cut cannot be capped
+    // non-manifold vertices (two loops touching): give the second out-edge
+    // of a vertex to the second in-edge so every edge has a distinct successor
+    for (int j = tid; j < nb; j += PC_T)
+        if (atomicAdd(&tmp[succ[j]], 1) > 0) s->flag[1] = 1;
+    __syncthreads();
+    if (s->flag[1]) {
+        if (tid == 0) {
+            int bad = 0;
+            for (int j = 0; j < nb; ++j) {
+                if (tmp[succ[j]] <= 1) continue;
+                // reassign: find another edge starting at the same vertex not yet taken
+                const int v = be[succ[j]].x;
+                for (int q = 0; q < nb; ++q)
+                    if (be[q].x == v && tmp[q] == 0) {
+                        tmp[succ[j]]--;
+                        succ[j] = (I)q;
+                        tmp[q] = 1;
+                        break;
+                    }
+            }
+            for (int j = 0; j < nb; ++j)
+                if (tmp[j] != 1) bad = 1;
+            s->flag[0] = bad;
+        }
+        __syncthreads();
+        if (s->flag[0]) return false;
+    }
+    // one step of pointer jumping over (val, jmp): read everything, then write
+    auto jump = [&](I* val, auto combine) {
+        if constexpr (LDS) {
+            I a[PER], b[PER];
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int j = tid + u * PC_T;
+                a[u] = b[u] = 0;
+                if (j < nb) { a[u] = (I)combine(j); b[u] = jmp[jmp[j]]; }
+            }
+            __syncthreads();
+#pragma unroll
+            for (int u = 0; u < PER; ++u) {
+                const int j = tid + u * PC_T;
+                if (j < nb) { val[j] = a[u]; jmp[j] = b[u]; }
+            }
+        } else {
+            for (int j = tid; j < nb; j += PC_T) { jl[j] = (I)combine(j); jr[j] = jmp[jmp[j]]; }
+            __syncthreads();
+            for (int j = tid; j < nb; j += PC_T) { val[j] = jl[j]; jmp[j] = jr[j]; }
+        }
+        __syncthreads();
+    };
+    // loop labels by pointer jumping: label = min edge index on the cycle
+    for (int j = tid; j < nb; j += PC_T) { lab[j] = (I)j; jmp[j] = succ[j]; }
+    __syncthreads();
+    for (int step = 1; step < nb; step <<= 1) jump(lab, [&](int j) { return min((int)lab[j], (int)lab[jmp[j]]); });
+    // rank along the loop from its head (the edge of that index), by
+    // predecessor jumps
+    for (int j = tid; j < nb; j += PC_T) tmp[succ[j]] = j;
+    __syncthreads();
+    for (int j = tid; j < nb; j += PC_T) {
+        const bool head = lab[j] == (I)j;
+        rank[j] = head ? 0 : 1;
+        jmp[j] = head ? (I)j : (I)tmp[j];
+    }
+    __syncthreads();
+    for (int step = 1; step < nb; step <<= 1)
+        jump(rank, [&](int j) { return (int)rank[j] + (jmp[j] != (I)j ? (int)rank[jmp[j]] : 0); });
+    // loop ids in head order, on wave 0
+    if (tid < 64) {
+        int nl = 0;
+        for (int b = 0; b < nb; b += 64) {
+            const int j = b + tid;
+            const bool head = j < nb && lab[j] == (I)j;
+            const unsigned long long m = ballot(head);
+            if (head) tmp[j] = nl + mask_rank(m);
+            nl += (int)__popcll(m);
+        }
+        if (tid == 0) {
+            s->n_loops = nl;
+            s->fail = nl > PC_MAX_LOOPS;
+        }
+    }
+    __syncthreads();
+    if (s->fail) return false;
+    const int nl = s->n_loops;
+    // loop sizes -> starts
+    for (int l = tid; l < nl; l += PC_T) s->loop_parent[l] = 0;
+    __syncthreads();
+    for (int j = tid; j < nb; j += PC_T) atomicAdd(&s->loop_parent[tmp[lab[j]]], 1);
+    __syncthreads();
+    if (tid == 0) {
+        int o = 0;
+        for (int l = 0; l < nl; ++l) { s->loop_start[l] = o; o += s->loop_parent[l]; }
+        s->loop_start[nl] = o;
+    }
+    __syncthreads();
+    for (int j = tid; j < nb; j += PC_T) {
+        const int l = tmp[lab[j]];
+        const int sz = s->loop_start[l + 1] - s->loop_start[l];
+        poly[s->loop_start[l] + (sz - 1 - (int)rank[j])] = be[j].x;
+    }
+    return true;
 }
 
 // Cap polygons of the positive side's boundary edges be[0, nb) (directed
@@ -400,7 +590,6 @@ __device__ inline int pc_cap_from_edges(const PcCapWork& w, int nb, const float*
     int* prv = w.prv;
     int* nxt = w.nxt;
     int* capbuf = w.capbuf;
-    uint8_t* refl = w.refl;
     int* hkey = (int*)w.ek;
     int* hval = hkey + w.H;
     if (tid == 0) s->fail = 0;
@@ -421,106 +610,23 @@ __device__ inline int pc_cap_from_edges(const PcCapWork& w, int nb, const float*
         atomicMin(&hval[h], j);
     }
     __syncthreads();
-    for (int j = tid; j < nb; j += PC_T) {
+    auto successor = [&](int j) {
         const int v = be[j].y;
         uint32_t h = pc_hash((unsigned long long)(unsigned)v) & (w.H - 1);
-        int e = -1;
         for (uint32_t probe = 0; probe < w.H; ++probe) {
             const int k = hkey[h];
-            if (k == v) { e = hval[h]; break; }
+            if (k == v) return hval[h];
             if (k == -1) break;
             h = (h + 1) & (w.H - 1);
         }
-        succ[j] = e;
-    }
-    __syncthreads();
-    // non-manifold vertices (two loops touching): give the second out-edge
-    // of a vertex to the second in-edge so every edge has a distinct successor
-    for (int j = tid; j < nb; j += PC_T) tmp[j] = 0;
-    __syncthreads();
-    for (int j = tid; j < nb; j += PC_T)
-        if (succ[j] >= 0) atomicAdd(&tmp[succ[j]], 1);
-    __syncthreads();
-    if (tid == 0) {
-        int bad = 0;
-        for (int j = 0; j < nb && !bad; ++j) {
-            if (succ[j] < 0) { bad = 1; break; }
-            if (tmp[succ[j]] > 1) {
-                // reassign: find another edge starting at the same vertex not yet taken
-                const int v = be[succ[j]].x;
-                for (int q = 0; q < nb; ++q)
-                    if (be[q].x == v && tmp[q] == 0) {
-                        tmp[succ[j]]--;
-                        succ[j] = q;
-                        tmp[q] = 1;
-                        break;
-                    }
-            }
-        }
-        for (int j = 0; j < nb && !bad; ++j)
-            if (tmp[j] != 1) bad = 1;
-        s->fail = bad;
-    }
-    __syncthreads();
-    if (s->fail) return -1;  // open boundary: the cut cannot be capped
-    // loop labels by pointer jumping: label = min edge index on the cycle
-    for (int j = tid; j < nb; j += PC_T) { lab[j] = j; jmp[j] = succ[j]; }
-    __syncthreads();
-    for (int step = 1; step < nb; step <<= 1) {
-        for (int j = tid; j < nb; j += PC_T) { jl[j] = min(lab[j], lab[jmp[j]]); jr[j] = jmp[jmp[j]]; }
-        __syncthreads();
-        for (int j = tid; j < nb; j += PC_T) { lab[j] = jl[j]; jmp[j] = jr[j]; }
-        __syncthreads();
-    }
-    // rank along the loop from its head: walk backwards via doubling on the
-    // predecessor-free formulation: rank = number of steps from head
-    for (int j = tid; j < nb; j += PC_T) { rank[j] = (j == lab[j]) ? 0 : 1; jmp[j] = j; }
-    __syncthreads();
-    // predecessor pointers
-    for (int j = tid; j < nb; j += PC_T) tmp[succ[j]] = j;
-    __syncthreads();
-    for (int j = tid; j < nb; j += PC_T) jmp[j] = (j == lab[j]) ? j : tmp[j];
-    __syncthreads();
-    for (int step = 1; step < nb; step <<= 1) {
-        for (int j = tid; j < nb; j += PC_T) { jl[j] = rank[j] + (jmp[j] != j ? rank[jmp[j]] : 0); jr[j] = jmp[jmp[j]]; }
-        __syncthreads();
-        for (int j = tid; j < nb; j += PC_T) { rank[j] = jl[j]; jmp[j] = jr[j]; }
-        __syncthreads();
-    }
-    // loop table: heads are edges with lab == j
-    if (tid == 0) {
-        int nl = 0, off = 0;
-        for (int j = 0; j < nb; ++j)
-            if (lab[j] == j) {
-                if (nl >= PC_MAX_LOOPS) { s->fail = 1; break; }
-                s->loop_start[nl] = off;
-                tmp[j] = nl;  // head -> loop id
-                ++nl;
-                off = off;  // sizes filled below
-            }
-        s->n_loops = nl;
-    }
-    __syncthreads();
-    if (s->fail) return -1;
+        return -1;
+    };
+    const bool small = nb <= PC_CAP_LDS;
+    if (small ? !pc_loops<true>(be, nb, successor, s->e.succ, s->e.lab, s->e.rank, s->e.jmp, s->e.tmp,
+                                (uint16_t*)nullptr, (uint16_t*)nullptr, poly, s)
+              : !pc_loops<false>(be, nb, successor, succ, lab, rank, jmp, tmp, jl, jr, poly, s))
+        return -1;
     const int nl = s->n_loops;
-    // loop sizes -> starts
-    if (tid < nl) s->loop_parent[tid] = 0;
-    __syncthreads();
-    for (int j = tid; j < nb; j += PC_T) atomicAdd(&s->loop_parent[tmp[lab[j]] ], 1);
-    __syncthreads();
-    if (tid == 0) {
-        int o = 0;
-        for (int l = 0; l < nl; ++l) { s->loop_start[l] = o; o += s->loop_parent[l]; }
-        s->loop_start[nl] = o;
-    }
-    __syncthreads();
-    // cap polygons wind opposite to the positive side's boundary: a cap
-    // edge runs b -> a for boundary edge (a, b); lay loops out reversed
-    for (int j = tid; j < nb; j += PC_T) {
-        const int l = tmp[lab[j]];
-        const int sz = s->loop_start[l + 1] - s->loop_start[l];
-        poly[s->loop_start[l] + (sz - 1 - rank[j])] = be[j].x;
-    }
     // projection drops the dominant axis of the plane normal
     const float anx = fabsf(pa), any_ = fabsf(pb), anz = fabsf(pc);
     const int pu = (anx >= any_ && anx >= anz) ? 1 : 0;
@@ -535,18 +641,24 @@ __device__ inline int pc_cap_from_edges(const PcCapWork& w, int nb, const float*
     // ---- wave 0: orientation, nesting, bridging, ear clipping ------------
     if (tid < 64) {
         const int lane = tid;
-        // signed areas: one FP64 pass per loop in vertex order on lane 0 (a
-        // fixed summation order keeps orientation and nesting reproducible)
-        if (lane == 0)
-            for (int l = 0; l < nl; ++l) {
-                const int b0 = s->loop_start[l], sz = s->loop_start[l + 1] - b0;
-                double a = 0.0;
-                for (int i = 0; i < sz; ++i) {
+        // signed areas: FP64 sums per loop in vertex order (a fixed order keeps
+        // orientation and nesting reproducible)
+        for (int l = 0; l < nl; ++l) {
+            const int b0 = s->loop_start[l], sz = s->loop_start[l + 1] - b0;
+            double a = 0.0;
+            for (int c0 = 0; c0 < sz; c0 += 64) {
+                // 64 terms at once, added in order
+                const int i = c0 + lane;
+                double t = 0.0;
+                if (i < sz) {
                     const P2 p = uv[b0 + i], q = uv[b0 + (i + 1 == sz ? 0 : i + 1)];
-                    a += (double)p.u * (double)q.v - (double)q.u * (double)p.v;
+                    t = (double)p.u * (double)q.v - (double)q.u * (double)p.v;
                 }
-                s->loop_area[l] = (float)(a * 0.5);
+                const int m = min(64, sz - c0);
+                for (int k = 0; k < m; ++k) a += read_lane_d(t, k);
             }
+            if (lane == 0) s->loop_area[l] = (float)(a * 0.5);
+        }
         __threadfence_block();
         // nesting: parent = smallest enclosing loop (ray casting from loop i's first vertex)
         for (int l = 0; l < nl; ++l) {
@@ -720,7 +832,8 @@ __device__ inline int pc_cap_from_edges(const PcCapWork& w, int nb, const float*
                     n = nn;
                 }
                 if (s->fail) break;
-                const int got = pc_earclip(pid, n, puv, prv, nxt, refl, capbuf + 3 * ncap);
+                const int got = n <= PC_CAP_LDS ? pc_earclip<true>(pid, n, puv, prv, nxt, capbuf + 3 * ncap, s)
+                                                : pc_earclip<false>(pid, n, puv, prv, nxt, capbuf + 3 * ncap, s);
                 if (got != n - 2) { if (lane == 0) s->fail = 1; __threadfence_block(); break; }
                 ncap += got;
             }

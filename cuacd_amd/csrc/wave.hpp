@@ -26,6 +26,9 @@ template <class T> __device__ __forceinline__ T uniform(T v) {
 }
 
 __device__ __forceinline__ int read_lane(int v, int l) { return __builtin_amdgcn_readlane(v, l); }
+__device__ __forceinline__ double read_lane_d(double v, int l) {
+    return __hiloint2double(read_lane(__double2hiint(v), l), read_lane(__double2loint(v), l));
+}
 __device__ __forceinline__ float read_lane(float v, int l) {
     return __int_as_float(__builtin_amdgcn_readlane(__float_as_int(v), l));
 }
