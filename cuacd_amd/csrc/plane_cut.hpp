@@ -59,7 +59,7 @@ struct PcResult {
 
 // Boundaries of up to PC_CAP_LDS edges (and polygons of as many vertices) are
 // linked, labelled and ear-clipped in LDS.
-constexpr int PC_CAP_LDS = 512;
+constexpr int PC_CAP_LDS = 1024;
 
 struct PcLDS {
     union {
@@ -221,13 +221,15 @@ __device__ __forceinline__ bool pc_pt_in_tri(P2 X, P2 A, P2 B, P2 C) {
 // triangles (vertex ids) to out_tris and returns that count.
 //
 // A serial chain: a step's vertex follows from the last step's verdict. With
-// LDS (up to PC_CAP_LDS vertices) the ring and the coordinates live in LDS and
-// every lane keeps its share of the vertices in registers; the candidate's
-// corners are carried from step to step, so a step costs two dependent LDS
-// reads and the containment test, whose distance checks run only where some
-// vertex is in the triangle. Triangles are written as ring positions and
-// translated afterwards (a load per clip would stall the wave). With the ring
-// in global memory (larger polygons) a step is two dependent memory reads.
+// LDS (up to PC_CAP_LDS vertices) the ring and the coordinates live there, the
+// candidate's corners are carried from step to step, and the next one is read
+// while the test runs. Vertices 64 k .. 64 k + 63 are consecutive on the loop,
+// so most such blocks lie far from the small triangle: lane k keeps block k's
+// box, and only the blocks whose box meets the triangle's are tested (see
+// `far`). Triangles are written as ring positions and translated afterwards (a
+// load per clip would stall the wave). 393 vertices took 1.0M cycles with
+// every block tested. With the ring in global memory (larger polygons) a step
+// is two dependent memory reads.
 template <bool LDS>
 __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv, int* nxt, int* out_tris, PcLDS* s) {
     const int lane = lane_id();
@@ -243,10 +245,8 @@ __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv,
             __threadfence_block();
         }
     };
-    // lane l keeps vertices l + 64 k in registers with a bit each that is set
-    // once the vertex is removed (or was never there)
-    constexpr int R = LDS ? PC_CAP_LDS / 64 : 1;
-    float ru[R], rv[R];
+    // lane l answers for vertices l + 64 k: bit k set once the vertex is
+    // removed (or was never there)
     uint32_t gone = 0;
     float mnu = 3.4e38f, mxu = -3.4e38f, mnv = 3.4e38f, mxv = -3.4e38f;
     auto init = [&](int i) {
@@ -265,18 +265,22 @@ __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv,
         }
         return x;
     };
+    // lane k: bounds of block k
+    float bu0 = 3.4e38f, bu1 = -3.4e38f, bv0 = 3.4e38f, bv1 = -3.4e38f;
     if constexpr (LDS) {
-#pragma unroll
-        for (int k = 0; k < R; ++k) {
+        static_assert(PC_CAP_LDS <= 64 * 32, "a bit per block");
+        for (int k = 0; 64 * k < n; ++k) {
             const int i = lane + 64 * k;
-            ru[k] = rv[k] = 0.0f;
+            float u0 = 3.4e38f, u1 = -3.4e38f, v0 = 3.4e38f, v1 = -3.4e38f;
             if (i < n) {
                 const P2 x = init(i);
-                ru[k] = x.u;
-                rv[k] = x.v;
+                u0 = u1 = x.u;
+                v0 = v1 = x.v;
             } else {
                 gone |= 1u << k;
             }
+            u0 = wave_min_f(u0); u1 = wave_max_f(u1); v0 = wave_min_f(v0); v1 = wave_max_f(v1);
+            if (lane == k) { bu0 = u0; bu1 = u1; bv0 = v0; bv1 = v1; }
         }
     } else {
         for (int i = lane; i < n; i += 64) (void)init(i);
@@ -289,6 +293,8 @@ __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv,
     int nt = 0, remaining = n, cur = 0, lap = 0;
     int p = prev(0), q = next(0);
     P2 A = P(p), B = P(cur), C = P(q);
+    int q2 = next(q);  // the vertex after q, whatever becomes of the candidate
+    P2 D = P(q2);
     while (remaining > 3) {
         const float cr = cross2(A, B, C);
         bool ear;
@@ -307,6 +313,8 @@ __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv,
             q = next(cur);
             A = P(p);
             C = P(q);
+            q2 = next(q);
+            D = P(q2);
             ear = true;
         } else if (cr < -1e-9f) {
             ear = false;
@@ -320,11 +328,28 @@ __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv,
             bool bad = false;
             if constexpr (LDS) {
                 const uint32_t skip = gone | bit(p) | bit(cur) | bit(q);
-#pragma unroll
-                for (int k = 0; k < R; ++k) {
-                    if (64 * k >= n) break;
-                    const P2 X{ru[k], rv[k]};
-                    const bool in = pc_pt_in_tri(X, A, B, C) && !((skip >> k) & 1u);
+                const float u0 = fminf(A.u, fminf(B.u, C.u)), u1 = fmaxf(A.u, fmaxf(B.u, C.u));
+                const float v0 = fminf(A.v, fminf(B.v, C.v)), v1 = fmaxf(A.v, fmaxf(B.v, C.v));
+                const float e = fmaxf(u1 - u0, v1 - v0);
+                // A vertex more than e / 4 outside the triangle's box, by
+                // D' > e / 4 on its farthest axis, fails the closed test below
+                // (thresholds 1e-10 on the three cross products) when
+                // cr >= 1e-4 e^2 (cr > 1e-9 here): its negative barycentric
+                // coordinates sum to at least D' / e, so some product is below
+                // -cr D' / (2 e) <= -cr / 8 <= -1.25e-10, and the largest is
+                // above (1 + D' / e) cr / 3; their FP32 errors, at most
+                // 4 eps sqrt(2) e 5 sqrt(2) D' = 2.4e-6 e D', are under 5 % of
+                // cr D' / (2 e) >= 5e-5 e D'. Thinner triangles test every block.
+                const float m = 0.26f * e;
+                const bool far = cr >= 1e-4f * e * e &&
+                                 (bu0 > u1 + m || bu1 < u0 - m || bv0 > v1 + m || bv1 < v0 - m);
+                uint32_t blocks = (uint32_t)ballot(64 * lane < n && !far);
+                while (blocks) {
+                    const int k = __builtin_ctz(blocks);
+                    blocks &= blocks - 1;
+                    const int i = min(lane + 64 * k, n - 1);
+                    const P2 X{s->c.u[i], s->c.v[i]};
+                    const bool in = !((skip >> k) & 1u) && pc_pt_in_tri(X, A, B, C);
                     if (ballot(in)) bad |= in && apart(X);
                 }
             } else {
@@ -362,8 +387,10 @@ __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv,
         }
         cur = q;
         B = C;
-        q = next(q);
-        C = P(q);
+        q = q2;
+        C = D;
+        q2 = next(q);
+        D = P(q2);
     }
     if (remaining == 3) {
         if (lane == 0) {
@@ -1274,6 +1301,29 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
         t.s2 = sgn(t.v2);
         return t;
     };
+    // triangle k of the wave's walk, whose indices were read one step ahead
+    int ahead0 = 0, ahead1 = 0, ahead2 = 0;
+    auto read_ahead = [&](int k) {
+        k = min(k, nt - 1);
+        ahead0 = T[3 * k];
+        ahead1 = T[3 * k + 1];
+        ahead2 = T[3 * k + 2];
+    };
+    auto take = [&](int k_next) {
+        PcTri t;
+        t.v0 = ahead0;
+        t.v1 = ahead1;
+        t.v2 = ahead2;
+        read_ahead(k_next);
+        t.s0 = sgn(t.v0);
+        t.s1 = sgn(t.v1);
+        t.s2 = sgn(t.v2);
+        return t;
+    };
+    // special: an edge crosses, or two vertices lie on the plane
+    auto is_special = [](const PcTri& t, int c) {
+        return ((c >> 4) & 7) || ((t.s0 == 0) + (t.s1 == 0) + (t.s2 == 0) >= 2);
+    };
     // an edge crosses when its ends' signs differ with on-plane counted positive
     auto xe = [](int sa, int sb) { return (sa >= 0) != (sb >= 0); };
     auto ncross = [&](const PcTri& t) { return (int)xe(t.s0, t.s1) + (int)xe(t.s1, t.s2) + (int)xe(t.s2, t.s0); };
@@ -1322,21 +1372,20 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
     if (tid == 0) { s->cnt[0] = 0; s->fail = 0; }
     // the wave's special triangles (crossing an edge, or with two vertices on
     // the plane), in triangle order from sl[tb]: the passes that only concern
-    // them walk this list instead of the whole triangle range
-    int* sl = (int*)pc_alloc(pool, 4ull * nt + 16, s, 1, err, 1);
+    // them walk this list instead of the whole triangle range; spos: their
+    // first output positions on both sides
+    int* sl = (int*)pc_alloc(pool, al16(4ull * nt) + 8ull * nt + 16, s, 1, err, 1);
     if (!sl) { R.status = -1; return R; }
+    int2* spos = (int2*)((char*)sl + al16(4ull * nt));
     int nsl = 0;  // wave-uniform
     {
         int cnp = 0, cnn = 0, cnc = 0, anyp = 0, anyn = 0;
+        read_ahead(tb + lane);
         for (int k0 = tb; k0 < te; k0 += 64) {
             const int k = k0 + lane;
-            PcTri t{0, 0, 0, 0, 0, 0};
-            int c = 0;
-            if (k < te) {
-                t = load(k);
-                c = code(t);
-            }
-            const bool special = k < te && (((c >> 4) & 7) || ((t.s0 == 0) + (t.s1 == 0) + (t.s2 == 0) >= 2));
+            const PcTri t = take(k + 64);
+            const int c = k < te ? code(t) : 0;
+            const bool special = k < te && is_special(t, c);
             const unsigned long long sm = ballot(special);
             if (special) sl[tb + nsl + mask_rank(sm)] = k;
             nsl += (int)__popcll(sm);
@@ -1760,23 +1809,46 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
             o[5] = rmap(side, q.b2);
         }
     };
+    // whole triangles go straight to their side; the special ones (their new
+    // vertices are hash lookups in memory) only get their positions, and are
+    // written 64 at a time below - a few of them in most steps of this walk
+    // took three quarters of its time
     {
-        int bp = bnp, bn = bnn;
+        int bp = bnp, bn = bnn, js = 0;
+        read_ahead(tb + lane);
         for (int k0 = tb; k0 < te; k0 += 64) {
             const int k = k0 + lane;
-            PcTri t{0, 0, 0, 0, 0, 0};
-            int c = 0;
-            if (k < te) {
-                t = load(k);
-                c = code(t);
-            }
+            const PcTri t = take(k + 64);
+            const int c = k < te ? code(t) : 0;
             const int np_ = c & 3, nn_ = (c >> 2) & 3;
             const int incl = wave_incl_scan(np_ | (nn_ << 16));
-            if (np_ && otp) put_pieces(0, pieces(t, c, 0), otp + 3 * (bp + (incl & 0xFFFF) - np_));
-            if (nn_ && otn) put_pieces(1, pieces(t, c, 1), otn + 3 * (bn + (incl >> 16) - nn_));
+            const int op = bp + (incl & 0xFFFF) - np_, on = bn + (incl >> 16) - nn_;
+            const bool special = k < te && is_special(t, c);
+            const unsigned long long sm = ballot(special);
+            if (special) {
+                spos[tb + js + mask_rank(sm)] = make_int2(op, on);
+            } else if (k < te) {
+                const int side = np_ ? 0 : 1;
+                int* o = side ? otn : otp;
+                if (o) {
+                    o += 3 * (side ? on : op);
+                    o[0] = rmap(side, t.v0);
+                    o[1] = rmap(side, t.v1);
+                    o[2] = rmap(side, t.v2);
+                }
+            }
+            js += (int)__popcll(sm);
             const int tot = read_lane(incl, 63);
             bp += tot & 0xFFFF;
             bn += tot >> 16;
+        }
+        __syncthreads();
+        for (int j = lane; j < nsl; j += 64) {
+            const PcTri t = load(sl[tb + j]);
+            const int c = code(t);
+            const int2 at = spos[tb + j];
+            if ((c & 3) && otp) put_pieces(0, pieces(t, c, 0), otp + 3 * at.x);
+            if (((c >> 2) & 3) && otn) put_pieces(1, pieces(t, c, 1), otn + 3 * at.y);
         }
     }
     for (int k = tid; k < n_cap; k += PC_T) {

@@ -28,7 +28,7 @@ def _check(ctx, v, t, plane):
         assert np.asarray(g).tobytes() == np.ascontiguousarray(w, g.dtype).tobytes()
 
 
-@pytest.mark.parametrize("n", [3, 31, 32, 33, 127, 128, 255, 256, 257, 300, 600])
+@pytest.mark.parametrize("n", [3, 31, 32, 33, 127, 128, 255, 256, 257, 300, 511, 512, 513, 700])
 @pytest.mark.parametrize("waves", [0, 7])
 def test_cap_of_one_loop_matches_oracle(ctx, n, waves):
     # the side walls are split by their diagonals: a horizontal cut meets 2 n edges
