@@ -85,7 +85,7 @@ __device__ __forceinline__ unsigned long long dh_head(DHeap* hp, int c, int s) {
 // Pop one block of class c from stripe s starting from head value `old`;
 // nullptr if the stripe is (or becomes) empty.
 __device__ inline char* dh_pop_from(DPool* pool, DHeap* hp, int c, int s, unsigned long long old) {
-    char* base = pool->base;
+    char* base = in_hbm(pool->base);
     while ((uint32_t)old != DH_EMPTY) {
         uint32_t off = (uint32_t)old;
         DBlockHdr* b = (DBlockHdr*)(base + ((unsigned long long)off << 8));
@@ -118,6 +118,7 @@ __device__ inline void dh_push_chain(DHeap* hp, int c, int s, DBlockHdr* last, u
 // Allocate `bytes` user bytes from heap `h` (0 = output heap, 1 = scratch).
 // Returns nullptr and sets KERR_HEAP_OOM in *err on exhaustion.
 __device__ inline void* heap_alloc(DPool* pool, int h, unsigned long long bytes, int* err) {
+    pool = in_hbm(pool);
     DHeap* hp = h ? &pool->scratch : &pool->heap;
     const int c = dh_class_of(bytes + DH_HDR);
     if (c >= DH_NCLASS) { err_or(err, KERR_HEAP_OOM); return nullptr; }
@@ -141,7 +142,7 @@ __device__ inline void* heap_alloc(DPool* pool, int h, unsigned long long bytes,
         unsigned long long sz = 256ull << c;
         unsigned long long o = fetch_add_relaxed(&pool->bump, sz);
         if (o + sz > pool->capacity) { err_or(err, KERR_HEAP_OOM); return nullptr; }
-        blk = pool->base + o;
+        blk = in_hbm(pool->base) + o;
     }
     DBlockHdr* hd = (DBlockHdr*)blk;
     hd->meta = dh_meta(c, h, bytes);
@@ -156,7 +157,8 @@ __device__ inline void* heap_alloc(DPool* pool, int h, unsigned long long bytes,
 // no-op; a block whose header does not carry the live magic sets KERR_HEAP_CORRUPT.
 __device__ inline void heap_free(DPool* pool, void* p, int* err) {
     if (!p) return;
-    char* blk = (char*)p - DH_HDR;
+    pool = in_hbm(pool);
+    char* blk = in_hbm((char*)p) - DH_HDR;
     DBlockHdr* hd = (DBlockHdr*)blk;
     const unsigned long long meta = hd->meta;
     const int c = (int)(meta >> 56);
@@ -187,6 +189,7 @@ __device__ inline void heap_free(DPool* pool, void* p, int* err) {
 // the wave waits for it): one per batch instead of one per block.
 template <int N>
 __device__ inline void heap_free_n(DPool* pool, void* const (&ps)[N], int* err) {
+    pool = in_hbm(pool);
     DBlockHdr* hd[N];
     unsigned long long old[N];
     const int s = dh_stripe();
@@ -195,7 +198,7 @@ __device__ inline void heap_free_n(DPool* pool, void* const (&ps)[N], int* err) 
         hd[i] = nullptr;
         old[i] = 0;
         if (!ps[i]) continue;
-        DBlockHdr* h = (DBlockHdr*)((char*)ps[i] - DH_HDR);
+        DBlockHdr* h = (DBlockHdr*)(in_hbm((char*)ps[i]) - DH_HDR);
         const unsigned long long meta = h->meta;
         const int c = (int)(meta >> 56);
         const int hid = (int)((meta >> 48) & 0xFF);

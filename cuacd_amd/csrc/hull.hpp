@@ -28,15 +28,11 @@
 
 namespace cuacd {
 
-template <int AS, class T> using asptr = __attribute__((address_space(AS))) T*;
-
 // clang vector types (not HIP's wrapper classes) so they load and store
 // through address-space-qualified pointers as single ds/global ops
 typedef float f4v __attribute__((ext_vector_type(4)));
 typedef unsigned short u4v __attribute__((ext_vector_type(4)));
 typedef short s4v __attribute__((ext_vector_type(4)));
-constexpr int AS_GLOBAL = 1;
-constexpr int AS_LDS = 3;
 
 constexpr float QUANT_STEPS = 10216.0f;  // grid span (cuda/hull_dandc.cuh:1374-1376)
 
@@ -1883,6 +1879,7 @@ __device__ HullCanon hull_canon(const HullWS<AS> w, HullBlockLDS* sb, const Hull
 template <int AS, int NW>
 __device__ void hull_canon_write(const HullWS<AS> w, const HullResult& r, int* __restrict__ out_tris) {
     constexpr int T = 64 * NW;
+    int* out = in_hbm(out_tris);
     const int FC = w.FC;
     auto succ_of = [&](int e) { return fpl_geti(w.fpl[e / 3], e % 3); };
     auto end_of = [&](int e) { const int h = e / 3, j = e % 3; return u4_get(w.fv[h], j == 2 ? 0 : j + 1); };
@@ -1897,9 +1894,9 @@ __device__ void hull_canon_write(const HullWS<AS> w, const HullResult& r, int* _
             if (w.vref[b]) {
                 const int o = w.vout[b];
                 if (prev >= 0) {
-                    out_tris[3 * t] = c0;
-                    out_tris[3 * t + 1] = prev;
-                    out_tris[3 * t + 2] = o;
+                    out[3 * t] = c0;
+                    out[3 * t + 1] = prev;
+                    out[3 * t + 2] = o;
                     ++t;
                 }
                 prev = o;

@@ -34,7 +34,7 @@ __device__ __forceinline__ bool la_hull_item(LaHullTask& t, const HullWS<AS> w, 
                                              int* err, int* retry = nullptr, int task_id = -1, bool multi = false) {
     constexpr int T = 64 * NW;
     const int tid = threadIdx.x;
-    const float* P = t.filt ? t.filt : t.pts;
+    const float* P = in_hbm(t.filt ? t.filt : t.pts);
     const int n = t.filt ? t.nf : t.n;
     if (n < 4) {
         if (tid == 0) { t.vol = 0.0; t.hnv = t.hnt = 0; t.hv = nullptr; t.ht = nullptr; }
@@ -120,9 +120,10 @@ __device__ __forceinline__ bool la_hull_item(LaHullTask& t, const HullWS<AS> w, 
         return true;
     }
     auto pos = [&](int p, float* o3) {
-        o3[0] = P[3ll * p];
-        o3[1] = P[3ll * p + 1];
-        o3[2] = P[3ll * p + 2];
+        const float* q = in_hbm(P) + 3ll * p;
+        o3[0] = q[0];
+        o3[1] = q[1];
+        o3[2] = q[2];
     };
     const HullCanon hc = hull_canon<AS, NW>(w, sb, r, n, pos);
     if (hc.nt < 0) {
@@ -145,7 +146,7 @@ __device__ __forceinline__ bool la_hull_item(LaHullTask& t, const HullWS<AS> w, 
     // full heap leaves it out without an error
     if (tid == 0) sb->red[0] = (unsigned long long)heap_alloc(pool, 0, vb + 12ull * nt, t.emit == 2 ? nullptr : err);
     __syncthreads();
-    float* chunk = (float*)sb->red[0];
+    float* chunk = in_hbm((float*)sb->red[0]);
     __syncthreads();
     if (!chunk) {
         if (tid == 0) {
@@ -706,32 +707,18 @@ __global__ __launch_bounds__(PC_T, 4) void la_cut_kernel(LaCutTask* tasks, int n
 // both sides (in index order); the crossing points - one per undirected edge
 // with strictly opposite signs, in order of first occurrence over (triangle,
 // edge) - come from that short list alone.
-__global__ __launch_bounds__(PC_T) void la_score_kernel(LaScoreTask* tasks, int n, DPool* pool, int* err,
-                                                        int lds_nv) {
-    __shared__ PcLDS s;
-    extern __shared__ __align__(16) unsigned char pc_dyn[];
-    __shared__ double dsum[2][PC_T / 64];
-    __shared__ int wcnt[PC_T / 64];
-    // the candidates of one item's part are consecutive tasks: groups of 8 per XCD
-    const int slot = (int)xcd_group_slot(blockIdx.x, gridDim.x, 8u);
-    if (slot >= n) return;
-    LaScoreTask& T = tasks[slot];
+// One flag byte per vertex - bits 0-1 sign code (1 positive, 2 negative, 0 on
+// the plane), bit 2 in the positive point set, bit 3 in the negative one - in
+// fl: LDS when the mesh fits the launch's dynamic LDS, else the heap chunk F.
+template <bool LDS>
+__device__ __forceinline__ void la_score_item(LaScoreTask& T, uint8_t* fl, char* F, PcLDS& s, double (*dsum)[PC_T / 64],
+                                              int* wcnt, DPool* pool, int* err) {
     const int tid = threadIdx.x, wv = tid >> 6;
-    const float* V = T.v;
-    const int* Tr = T.t;
+    const float* V = in_hbm(T.v);
+    const int* Tr = in_hbm(T.t);
+    fl = LDS ? in_lds(fl) : in_hbm(fl);
     const int nv = T.nv, nt = T.nt;
     const float pa = T.plane[0], pb = T.plane[1], pc = T.plane[2], pd = T.plane[3];
-    // One flag byte per vertex - bits 0-1 sign code (1 positive, 2 negative, 0
-    // on the plane), bit 2 in the positive point set, bit 3 in the negative
-    // one - in LDS when the mesh fits the launch's dynamic LDS, else in a heap
-    // chunk of its own.
-    const bool flags_in_lds = nv <= lds_nv;
-    char* F = nullptr;
-    if (!flags_in_lds) {
-        F = (char*)pc_alloc(pool, al16(nv), &s, 1, err, 1);
-        if (!F) return;
-    }
-    uint8_t* fl = flags_in_lds ? pc_dyn : (uint8_t*)F;
     for (int i = tid; i < nv; i += PC_T) {
         const float d = pc_side(pa, pb, pc, pd, V[3 * i], V[3 * i + 1], V[3 * i + 2]);
         fl[i] = d > PC_EPS ? 1 : (d < -PC_EPS ? 2 : 0);
@@ -1012,6 +999,25 @@ __global__ __launch_bounds__(PC_T) void la_score_kernel(LaScoreTask* tasks, int 
     }
 }
 
+__global__ __launch_bounds__(PC_T) void la_score_kernel(LaScoreTask* tasks, int n, DPool* pool, int* err,
+                                                        int lds_nv) {
+    __shared__ PcLDS s;
+    extern __shared__ __align__(16) unsigned char pc_dyn[];
+    __shared__ double dsum[2][PC_T / 64];
+    __shared__ int wcnt[PC_T / 64];
+    // the candidates of one item's part are consecutive tasks: groups of 8 per XCD
+    const int slot = (int)xcd_group_slot(blockIdx.x, gridDim.x, 8u);
+    if (slot >= n) return;
+    LaScoreTask& T = tasks[slot];
+    if (T.nv <= lds_nv) {
+        la_score_item<true>(T, pc_dyn, nullptr, s, dsum, wcnt, pool, err);
+    } else {
+        char* F = (char*)pc_alloc(pool, al16(T.nv), &s, 1, err, 1);
+        if (!F) return;
+        la_score_item<false>(T, (uint8_t*)F, F, s, dsum, wcnt, pool, err);
+    }
+}
+
 // ---------------------------------------------------------------------------
 // Connected components (reference cuda/postprocess.cuh:139-527)
 // ---------------------------------------------------------------------------
@@ -1039,8 +1045,8 @@ __global__ __launch_bounds__(PC_T) void la_comp_kernel(LaCompTask* tasks, int n,
     if ((int)blockIdx.x >= n) return;
     LaCompTask& T = tasks[blockIdx.x];
     const int tid = threadIdx.x;
-    const float* V = T.v;
-    const int* Tr = T.t;
+    const float* V = in_hbm(T.v);
+    const int* Tr = in_hbm(T.t);
     const int nv = T.nv, nt = T.nt;
     if (nv <= 0 || nt <= 0) {
         if (tid == 0) T.n_comp = 0;
@@ -1178,8 +1184,8 @@ __global__ __launch_bounds__(PC_T) void la_edges_kernel(LaEdgeTask* tasks, int n
     if ((int)blockIdx.x >= n) return;
     LaEdgeTask& T = tasks[blockIdx.x];
     const int tid = threadIdx.x;
-    const float* V = T.v;
-    const int* Tr = T.t;
+    const float* V = in_hbm(T.v);
+    const int* Tr = in_hbm(T.t);
     const int nt = T.nt;
     if (T.nv <= 0 || nt < 2) {
         if (tid == 0) T.count = 0;

@@ -126,6 +126,7 @@ __device__ __forceinline__ int pc_ht_find(const unsigned long long* keys, uint32
 // Block-wide exclusive scan over n elements of f(i) (int). Contiguous chunks.
 template <class F>
 __device__ int pc_block_scan(int n, int* out, PcLDS* s, F f) {
+    s = in_lds(s);
     const int tid = threadIdx.x, wv = tid >> 6;
     const int per = (n + PC_T - 1) / PC_T;
     const int b = min(n, tid * per), e = min(n, b + per);
@@ -155,7 +156,7 @@ __device__ __forceinline__ void* pc_alloc(DPool* pool, unsigned long long bytes,
     __syncthreads();
     void* p = s->ptr[slot];
     __syncthreads();
-    return p;
+    return in_hbm((char*)p);
 }
 
 __device__ __forceinline__ unsigned long long al16(unsigned long long x) { return (x + 15ull) & ~15ull; }
@@ -184,6 +185,9 @@ __device__ inline PcMesh pc_copy_mesh(const float* V, const int* T, int nv, int 
 
 // FP64 volume of a mesh chunk (anchored at vertex 0), block-uniform.
 __device__ inline double pc_volume(const float* v, const int* t, int nt, PcLDS* s) {
+    v = in_hbm(v);
+    t = in_hbm(t);
+    s = in_lds(s);
     double acc = 0.0;
     if (nt > 0) {
         const double ax = v[0], ay = v[1], az = v[2];
@@ -234,6 +238,12 @@ template <bool LDS>
 __device__ inline int pc_earclip(const int* poly, int n, const P2* uv, int* prv, int* nxt, int* out_tris, PcLDS* s) {
     const int lane = lane_id();
     if (n < 3) return 0;
+    s = in_lds(s);
+    poly = in_hbm(poly);
+    uv = in_hbm(uv);
+    prv = in_hbm(prv);
+    nxt = in_hbm(nxt);
+    out_tris = in_hbm(out_tris);
     auto P = [&](int i) { return LDS ? P2{s->c.u[i], s->c.v[i]} : uv[i]; };
     auto next = [&](int i) -> int { return LDS ? (int)s->c.nxt[i] : nxt[i]; };
     auto prev = [&](int i) -> int { return LDS ? (int)s->c.prv[i] : prv[i]; };
@@ -477,6 +487,14 @@ __device__ inline bool pc_loops(const int2* be, int nb, F successor, I* succ, I*
                                 I* jr, int* poly, PcLDS* s) {
     constexpr int PER = PC_CAP_LDS / PC_T;
     const int tid = threadIdx.x;
+    be = in_hbm(be);
+    poly = in_hbm(poly);
+    s = in_lds(s);
+    succ = LDS ? in_lds(succ) : in_hbm(succ);
+    lab = LDS ? in_lds(lab) : in_hbm(lab);
+    rank = LDS ? in_lds(rank) : in_hbm(rank);
+    jmp = LDS ? in_lds(jmp) : in_hbm(jmp);
+    tmp = LDS ? in_lds(tmp) : in_hbm(tmp);
     if (tid < 2) s->flag[tid] = 0;
     __syncthreads();
     for (int j = tid; j < nb; j += PC_T) {
@@ -602,22 +620,25 @@ __device__ inline bool pc_loops(const int2* be, int nb, F successor, I* succ, I*
 __device__ inline int pc_cap_from_edges(const PcCapWork& w, int nb, const float* __restrict__ V, int nv,
                                         const float* newv, float pa, float pb, float pc, PcLDS* s) {
     const int tid = threadIdx.x;
-    int2* be = w.be;
-    int* succ = w.succ;
-    int* lab = w.lab;
-    int* rank = w.rank;
-    int* jmp = w.jmp;
-    int* jl = w.jl;
-    int* jr = w.jr;
-    int* tmp = w.tmp;
-    int* poly = w.poly;
-    P2* uv = w.uv;
-    int* wid = w.wid;
-    P2* wuv = w.wuv;
-    int* prv = w.prv;
-    int* nxt = w.nxt;
-    int* capbuf = w.capbuf;
-    int* hkey = (int*)w.ek;
+    V = in_hbm(V);
+    newv = in_hbm(newv);
+    s = in_lds(s);
+    int2* be = in_hbm(w.be);
+    int* succ = in_hbm(w.succ);
+    int* lab = in_hbm(w.lab);
+    int* rank = in_hbm(w.rank);
+    int* jmp = in_hbm(w.jmp);
+    int* jl = in_hbm(w.jl);
+    int* jr = in_hbm(w.jr);
+    int* tmp = in_hbm(w.tmp);
+    int* poly = in_hbm(w.poly);
+    P2* uv = in_hbm(w.uv);
+    int* wid = in_hbm(w.wid);
+    P2* wuv = in_hbm(w.wuv);
+    int* prv = in_hbm(w.prv);
+    int* nxt = in_hbm(w.nxt);
+    int* capbuf = in_hbm(w.capbuf);
+    int* hkey = (int*)in_hbm(w.ek);
     int* hval = hkey + w.H;
     if (tid == 0) s->fail = 0;
     __syncthreads();
@@ -878,6 +899,9 @@ __device__ inline PcResult plane_cut_block(const float* __restrict__ V, const in
                                            float pa, float pb, float pc, float pd, DPool* pool, int* err,
                                            PcLDS* s) {
     const int tid = threadIdx.x;
+    V = in_hbm(V);
+    T = in_hbm(T);
+    s = in_lds(s);
     PcResult R;
     R.pos = PcMesh{nullptr, nullptr, 0, 0, 0.0};
     R.neg = PcMesh{nullptr, nullptr, 0, 0, 0.0};
@@ -1268,6 +1292,10 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
                                                PcLDS* s, unsigned char* dyn) {
     constexpr int NW = PC_T / 64;
     const int tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
+    V = in_hbm(V);
+    T = in_hbm(T);
+    s = in_lds(s);
+    dyn = in_lds(dyn);
     PcResult R;
     R.pos = PcMesh{nullptr, nullptr, 0, 0, 0.0};
     R.neg = PcMesh{nullptr, nullptr, 0, 0, 0.0};

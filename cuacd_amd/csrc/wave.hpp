@@ -9,6 +9,21 @@
 
 namespace cuacd {
 
+template <int AS, class T> using asptr = __attribute__((address_space(AS))) T*;
+constexpr int AS_GLOBAL = 1;
+constexpr int AS_LDS = 3;
+
+// A generic pointer whose memory is known, so that its accesses compile to
+// global or ds instructions: a flat access counts as outstanding in both
+// memories, and a wait for one of them waits for everything in flight. (A cut
+// of 24k triangles 894 us with its 1,800 flat accesses, 825 us without; a
+// 64-mesh decomposition 459 and 425 ms.)
+// (Through an integer: a pair of pointer casts would cancel.)
+template <class T> __device__ __forceinline__ T* in_hbm(T* p) { return (T*)(asptr<AS_GLOBAL, T>)(uintptr_t)p; }
+template <class T> __device__ __forceinline__ T* in_lds(T* p) {
+    return (T*)(asptr<AS_LDS, T>)(uint32_t)(uintptr_t)(p);  // the low half of a generic LDS address is the offset
+}
+
 constexpr int WAVE = 64;
 
 __device__ __forceinline__ int lane_id() { return __lane_id(); }
