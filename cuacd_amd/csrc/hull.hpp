@@ -108,28 +108,19 @@ template <int AS> struct HullWS {
     // multi-apex scratch (LDS workspaces with several waves; null otherwise)
     asptr<AS_LDS, uint32_t> mfm;    // [FC/2] per face, 16 bits (face f in word f/2, bits 16 (f&1) up):
                                     // bit r visited by candidate r, bit 8+r visible from it
-    asptr<AS_LDS, uint32_t> mfmax;  // [FC] per face: best conflict key (quantised distance, point index);
-                                    // only for up to 8192 vertices (hull_ma_layout)
-    asptr<AS_LDS, unsigned long long> msk;  // [MA_W] per wave share: best (conflict key << 32 | face)
-    asptr<AS_LDS, uint8_t> mfcone;  // [FC] candidate whose cone replaced the face this round
-    asptr<AS_LDS, uint16_t> mlist;  // [MA_W][MA_CAP][5]: visible faces, ha, hb, hface, hnew (ranks >= 1)
+    asptr<AS_LDS, uint16_t> mst;    // [FC] round that replaced the face << 3 | rank of the candidate that did
+    asptr<AS_LDS, uint16_t> mlist;  // [MA_W][5][MA_CAP]: visible faces, ha, hb, hface, hnew
     asptr<AS_LDS, uint8_t> mhedge;  // [MA_W][MA_CAP]
-    asptr<AS_LDS, int> mcand;       // [MA_W][MA_CI] candidate table, then [MA_W] conflict rows, misc
+    asptr<AS_LDS, int> mcand;       // [MA_W][MA_CI] candidate table, then [MA_W] keys, [2][MA_W] apex indices
     asptr<AS_LDS, f4v> mcpl;        // [MA_W][MA_CPL] planes of each accepted cone's faces, horizon order
     int VC, FC, NP;
 };
 
-// Candidate lists of the multi-apex rounds: candidate 0 uses the workspace's
-// own arrays, the others LDS scratch; with a workspace in global memory both
-// are addressed through generic pointers.
-template <int AS, class T> struct MaList { using type = T*; };
-template <class T> struct MaList<AS_LDS, T> { using type = asptr<AS_LDS, T>; };
-
-// Multi-apex rounds: at most MA_W candidates, MA_CAP visible faces and
-// horizon edges for each candidate but the first (which uses the main arrays).
+// Multi-apex rounds: at most MA_W candidates, MA_CAP visible faces and horizon
+// edges for each (the first takes the main arrays when its region is larger).
 // The planes of a cone of at most MA_CPL faces are also kept in cone order, so
 // that the points of the faces it replaced scan them without an id lookup.
-constexpr int MA_W = 8, MA_CAP = 128, MA_CI = 12, MA_CPL = 32;
+constexpr int MA_W = 8, MA_CAP = 128, MA_CI = 8, MA_CPL = 32;
 
 // LDS scratch of the multi-apex rounds for fc faces, carved from p (16-byte
 // aligned sub-arrays; p == nullptr only sizes it). An LDS workspace carries
@@ -144,14 +135,10 @@ __host__ __device__ __forceinline__ unsigned hull_ma_layout(char* p, unsigned fc
         return r;
     };
     w->mfm = (asptr<AS_LDS, uint32_t>)take((fc + 1u) / 2u * 4u);
-    w->msk = (asptr<AS_LDS, unsigned long long>)take(MA_W * 8u);
-    // per-face keys while they fit (2 + 4 + 1 bytes per face); above 8192
-    // vertices (3 bytes per face) the rounds reduce keys per wave share
-    if (fc <= 2u * 8192u + 8u) w->mfmax = (asptr<AS_LDS, uint32_t>)take(fc * 4u);
-    w->mfcone = (asptr<AS_LDS, uint8_t>)take(fc);
+    w->mst = (asptr<AS_LDS, uint16_t>)take(fc * 2u);
     w->mlist = (asptr<AS_LDS, uint16_t>)take(MA_W * MA_CAP * 5 * 2u);
     w->mhedge = (asptr<AS_LDS, uint8_t>)take(MA_W * MA_CAP);
-    w->mcand = (asptr<AS_LDS, int>)take((MA_W * MA_CI + MA_W + 16) * 4u);
+    w->mcand = (asptr<AS_LDS, int>)take((MA_W * MA_CI + 3 * MA_W) * 4u);
     w->mcpl = (asptr<AS_LDS, f4v>)take(MA_W * MA_CPL * 16u);
     return off;
 }
@@ -586,13 +573,11 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
     int nvert = 4, ftop = 4, nfree = 0;
     if constexpr (MULTI) {
         // ---- multi-apex rounds ---------------------------------------------
-        // Each round takes the farthest conflict point of every face, keeps
-        // the best face of each wave's share of the faces (ids interleaved
-        // over the waves; at most NW
-        // candidates, the first being the overall best), and lets wave r find
-        // the visible region of candidate r. Two candidates conflict when one's
-        // visible region meets the other's visited faces (its visible region
-        // and their neighbours); a conflict-free set of candidates (greedy by
+        // Each round every wave takes the farthest conflict point among its
+        // own points as a candidate (ranked over the waves by key) and finds
+        // its visible region. Two candidates conflict when one's visible
+        // region meets the other's visited faces (its visible region and
+        // their neighbours); a conflict-free set of candidates (greedy by
         // rank) is inserted at once. For such a set, inserting them together
         // gives the hull of inserting them one after another: a candidate sees
         // none of another's cone faces, since a walk over visible faces from
@@ -600,206 +585,95 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         // other, which would then be in its own visible region. Candidates may
         // be non-extreme points (their distances are quantised); the exact
         // incremental construction still ends at the unique hull.
+        // A round is four barriers long and bound by the chain of LDS reads
+        // between them, so nothing in it walks all faces but the visibility
+        // test, marks are cleared where they were set, and every wave works
+        // out the accepted set for itself. (Candidates per share of the faces
+        // took block-wide passes over points and faces and ten barriers a round:
+        // 21-31k cycles at 1000-2000 points and 78k at 12000, here 13-20k and
+        // 44k with 0.85 to 0.95 of the insertions; 192 clouds of 5-12000 points
+        // 68 -> 36 ms.)
         static_assert(NW > 1 && NW <= MA_W, "multi-apex rounds need several waves");
-        // a conflict key is the face's best point: its quantised distance
-        // above the high bits, its (inverted) local index in the low ones
-        static_assert(PPL * T <= 16384, "multi-apex keys hold point indices below 16384");
-        constexpr uint32_t IMASK =
-            PPL * T <= 2048 ? 0x7FFu : (PPL * T <= 4096 ? 0xFFFu : (PPL * T <= 8192 ? 0x1FFFu : 0x3FFFu));
-        using L16 = typename MaList<AS, uint16_t>::type;
-        using L8 = typename MaList<AS, uint8_t>::type;
+        // a conflict key is a point's quantised distance above the high bits,
+        // its (inverted) local index in the low ones; 0: inside, or a vertex
+        static_assert((PPL & (PPL - 1)) == 0 && (NW & (NW - 1)) == 0 && PPL * T <= 16384,
+                      "keys hold the point index in their low bits");
+        constexpr uint32_t IM = (uint32_t)(PPL * T) - 1u;
+        // faces up to which every face is tested against the apex (sizes with
+        // the planes in LDS); more are walked from the conflict face
+        constexpr int FLAT = AS == AS_LDS ? 4096 : 512;
+        using M16 = asptr<AS_LDS, uint16_t>;
         // the 16 mark bits of face f in its word
         auto mw = [&](int f) { return w.mfm + (f >> 1); };
         auto msh = [](int f) { return (uint32_t)(f & 1) << 4; };
-        const int wv = tid >> 6, lane = tid & 63;
-        asptr<AS_LDS, int> cand = w.mcand;
-        asptr<AS_LDS, int> crow = w.mcand + MA_W * MA_CI;
-        asptr<AS_LDS, int> misc = w.mcand + MA_W * MA_CI + MA_W;
-        auto lvis = [&](int r) { return w.mlist + (r * 5 + 0) * MA_CAP; };
-        auto lha = [&](int r) { return w.mlist + (r * 5 + 1) * MA_CAP; };
-        auto lhb = [&](int r) { return w.mlist + (r * 5 + 2) * MA_CAP; };
-        auto lhf = [&](int r) { return w.mlist + (r * 5 + 3) * MA_CAP; };
-        auto lhn = [&](int r) { return w.mlist + (r * 5 + 4) * MA_CAP; };
+        const int wv = uniform(tid >> 6), lane = tid & 63;
+        asptr<AS_LDS, int> cand = w.mcand;                      // [rank] region sizes, conflicts, apex
+        asptr<AS_LDS, int> pub = w.mcand + MA_W * MA_CI;        // [wave] candidate key
+        asptr<AS_LDS, int> dup = pub + MA_W;                    // [round parity][rank] lowest index of the apex
+        auto lst = [&](int r, int a) { return w.mlist + (r * 5 + a) * MA_CAP; };
         auto wsync = [&]() {
             __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "workgroup");
             __builtin_amdgcn_wave_barrier();
         };
-        if (tid < MA_W) w.msk[tid] = 0ull;
-        __syncthreads();
+        auto mkkey = [&](float t, int k) {
+            return (__float_as_uint(fmaxf(t, 1e-6f)) & ~IM) | (IM - (uint32_t)(k * T + tid));
+        };
+        const f4v dead = mk_f4(0.0f, 0.0f, 0.0f, -1.0f);
+        uint32_t key[PPL];
+#pragma unroll
+        for (int k = 0; k < PPL; ++k) {
+            key[k] = conf[k] >= 0 ? mkkey(dist[k], k) : 0u;
+            conf[k] = max(conf[k], 0);
+        }
+        asptr<AS_LDS, uint32_t> stw = (asptr<AS_LDS, uint32_t>)w.mst;
+        for (int q = tid; q < FC / 2; q += T) {
+            w.mfm[q] = 0u;
+            stw[q] = 0u;
+        }
+        int pvid = 0;  // lane r: vertex of the last round's candidate r
+        bool pacc = false;
         for (int it = 1;; ++it) {
-            if constexpr (PPL * T <= 8192) {
-                // A: clear the per-face marks and best keys
-                for (int f = tid; f < ftop; f += T) w.mfmax[f] = 0u;
-                for (int q = tid; q < (ftop + 1) >> 1; q += T) w.mfm[q] = 0u;
-                if (tid < MA_W) crow[tid] = 0;
+            // a face's stamp: the round that replaced it (13 bits, cleared
+            // before they repeat) and the rank of the candidate that did
+            const int tag = (it - 1) % 8191 + 1;
+            if (it > 1 && tag == 1) {
                 __syncthreads();
-                // B: best conflict key per face (quantised distance, lowest index)
-#pragma unroll
-                for (int k = 0; k < PPL; ++k)
-                    if (conf[k] >= 0) {
-                        const uint32_t key = (fkey(dist[k]) & ~IMASK) | (IMASK - (uint32_t)(k * T + tid));
-                        __hip_atomic_fetch_max(&w.mfmax[conf[k]], key, __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-                    }
-                __syncthreads();
-                // C: candidates - the best face of each wave's faces (face
-                // ids interleaved over the waves, so every wave has faces)
-                uint64_t bk = 0;
-                for (int f = wv + NW * lane; f < ftop; f += NW * 64) {
-                    const uint32_t k32 = w.mfmax[f];
-                    const uint64_t v = ((uint64_t)k32 << 32) | (uint32_t)f;
-                    if (k32 && v > bk) bk = v;
-                }
-                bk = wave_max_u64(bk);
-                if (lane == 0) w.msk[wv] = bk;
-                __syncthreads();
-            } else {
-                // A: clear the per-face marks. B (same interval: it reads no
-                // shared state): the same candidates without per-face keys -
-                // the best conflict point over the faces of each share (face
-                // f is in share f % NW), as (key << 32 | face): per lane and
-                // share, then over the wave, then over the waves
-                for (int q = tid; q < (ftop + 1) >> 1; q += T) w.mfm[q] = 0u;
-                if (tid < MA_W) crow[tid] = 0;
-                uint64_t sk[NW];
-#pragma unroll
-                for (int q = 0; q < NW; ++q) sk[q] = 0;
-#pragma unroll
-                for (int k = 0; k < PPL; ++k)
-                    if (conf[k] >= 0) {
-                        const uint32_t key = (fkey(dist[k]) & ~IMASK) | (IMASK - (uint32_t)(k * T + tid));
-                        const uint64_t v = ((uint64_t)key << 32) | (uint32_t)conf[k];
-                        const int sh = conf[k] % NW;
-#pragma unroll
-                        for (int q = 0; q < NW; ++q)
-                            if (q == sh && v > sk[q]) sk[q] = v;
-                    }
-#pragma unroll
-                for (int q = 0; q < NW; ++q) {
-                    sk[q] = wave_max_u64(sk[q]);
-                    if (lane == 0 && sk[q])
-                        __hip_atomic_fetch_max(&w.msk[q], (unsigned long long)sk[q], __ATOMIC_RELAXED,
-                                               __HIP_MEMORY_SCOPE_WORKGROUP);
-                }
-                __syncthreads();
+                for (int q = tid; q < FC / 2; q += T) stw[q] = 0u;
             }
-            uint64_t rk[NW];
-            int ncand = 0;
+            uint32_t sk = key[0];
 #pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                rk[q] = w.msk[q];
-                ncand += rk[q] != 0;
-            }
-            if (ncand == 0) break;
-            // the owners of the candidate points publish them at their rank,
-            // in descending key order (keys differ: they hold distinct face ids)
-#pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                if (!rk[q]) continue;
-                const int ip = (int)(IMASK - ((uint32_t)(rk[q] >> 32) & IMASK));
-                if (tid == ip % T) {
-                    int rank = 0;
-#pragma unroll
-                    for (int o = 0; o < NW; ++o) rank += rk[o] > rk[q];
-                    const int slot = ip / T;
-                    cand[rank * MA_CI + 0] = (int)(uint32_t)(rk[q] >> 32);
-                    cand[rank * MA_CI + 1] = (int)(uint32_t)rk[q];
-                    cand[rank * MA_CI + 2] = ip;
-                    cand[rank * MA_CI + 3] = pick(px, slot);
-                    cand[rank * MA_CI + 4] = pick(py, slot);
-                    cand[rank * MA_CI + 5] = pick(pz, slot);
-                }
-            }
+            for (int k = 1; k < PPL; ++k) sk = max(sk, key[k]);
+            sk = wave_max_u32(sk);
+            const int ip = (int)(IM - (sk & IM)), own = ip & 63, slot = ip / T;
+            const int qx = read_lane(hull_pick(px, slot), own), qy = read_lane(hull_pick(py, slot), own),
+                      qz = read_lane(hull_pick(pz, slot), own), f0 = read_lane(hull_pick(conf, slot), own);
+            if (lane == 0) pub[wv] = (int)sk;
             __syncthreads();
-            // the share maxima were read before the barrier above: clear them
-            // for the next round (several barriers before its first update)
-            if (tid < MA_W) w.msk[tid] = 0ull;
-            // D: wave r finds candidate r's visible region and, on the way, its
-            // horizon: every visible face tests its three neighbours at once
-            // (visit marks, planes and back links loaded together); the first
-            // visitor of a visible neighbour queues it, and every neighbour
-            // not visible gives a horizon edge (its test is deterministic, so
-            // every lane that reaches it agrees)
-            if (wv < ncand) {
-                const int r = wv;
-                const int f0 = cand[r * MA_CI + 1];
-                const int qx = cand[r * MA_CI + 3], qy = cand[r * MA_CI + 4], qz = cand[r * MA_CI + 5];
-                const float fqx = (float)qx, fqy = (float)qy, fqz = (float)qz;
-                L16 V = r == 0 ? (L16)w.vis : (L16)lvis(r);
-                const int vcap = r == 0 ? FC : MA_CAP;
-                L16 HA = r == 0 ? (L16)w.ha : (L16)lha(r);
-                L16 HB = r == 0 ? (L16)w.hb : (L16)lhb(r);
-                L16 HF = r == 0 ? (L16)w.hface : (L16)lhf(r);
-                L8 HE = r == 0 ? (L8)w.hedge : (L8)(w.mhedge + r * MA_CAP);
-                const int hcap = r == 0 ? VC : MA_CAP;
-                const uint32_t vb = 1u << r, sbit = 1u << (8 + r);
-                if (lane == 0) {
-                    __hip_atomic_fetch_or(mw(f0), (vb | sbit) << msh(f0), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
-                    V[0] = (uint16_t)f0;
-                }
-                wsync();
-                int head = 0, nv = 1, nh = 0;
+            int r = 0, ncand = 0;
+#pragma unroll
+            for (int q = 0; q < NW; ++q) {
+                const uint32_t o = uniform((uint32_t)pub[q]);
+                r += o > sk;
+                ncand += o != 0;
+            }
+            // points with the grid position of an inserted apex are inside the
+            // hull from then on; the vertex keeps the lowest of their indices
+            if (wv == 0 && pacc) w.vpid[pvid] = dup[((it - 1) & 1) * MA_W + lane];
+            if (ncand == 0) break;
+            asptr<AS_LDS, int> du = dup + (it & 1) * MA_W;
+            const float fqx = (float)qx, fqy = (float)qy, fqz = (float)qz;
+            const uint32_t vb = 1u << r, sbit = 1u << (8 + r);
+            // the candidate's visible faces V and its horizon: edges HA -> HB,
+            // the face beyond HF and its edge slot HE there
+            auto region = [&](auto V, auto HA, auto HB, auto HF, auto HE, int vcap, int hcap, int* nv_, int* nh_) {
+                int nv = 0, nh = 0;
                 bool over = false;
-                while (head < nv) {
-                    const int cnt = min(nv - head, 64);
-                    const bool act = lane < cnt;
-                    int f = 0;
-                    u4v fvl = {0, 0, 0, 0}, nb = {0, 0, 0, 0};
-                    if (act) {
-                        f = V[head + lane];
-                        fvl = w.fv[f];
-                        nb = w.fn[f];
-                    }
-                    const int gg[3] = {nb.x, nb.y, nb.z};
-                    const int vv[3] = {fvl.x, fvl.y, fvl.z};
-                    uint32_t old[3] = {vb, vb, vb};
-                    bool vis[3] = {false, false, false};
-                    int back[3] = {0, 0, 0};
-                    if (act) {
-                        f4v pl[3];
-                        u4v gn[3];
-#pragma unroll
-                        for (int e = 0; e < 3; ++e) {
-                            old[e] = __hip_atomic_fetch_or(mw(gg[e]), vb << msh(gg[e]), __ATOMIC_RELAXED,
-                                                           __HIP_MEMORY_SCOPE_WORKGROUP) >> msh(gg[e]);
-                            pl[e] = w.fpl[gg[e]];
-                            gn[e] = w.fn[gg[e]];
-                        }
-#pragma unroll
-                        for (int e = 0; e < 3; ++e) {
-                            // face_above on the loaded plane
-                            const float t = fmaf(pl[e].x, fqx, fmaf(pl[e].y, fqy, fmaf(pl[e].z, fqz, pl[e].w)));
-                            bool above = t > HULL_FILTER_EPS;
-                            if (!above && t >= -HULL_FILTER_EPS) {
-                                const u4v gv = w.fv[gg[e]];
-                                above = orient_exact(w.vq[gv.x], w.vq[gv.y], w.vq[gv.z], qx, qy, qz) > 0.0;
-                            }
-                            vis[e] = above;
-                            back[e] = (gn[e].x == f) ? 0 : ((gn[e].y == f) ? 1 : 2);
-                        }
-                    }
-                    head += cnt;
-                    int add = 0;
+                auto horizon = [&](const bool (&h)[3], const int (&vv)[3], const int (&gg)[3], const int (&back)[3]) {
 #pragma unroll
                     for (int e = 0; e < 3; ++e) {
-                        const bool ap = act && vis[e] && !(old[e] & vb);
-                        if (ap)
-                            __hip_atomic_fetch_or(mw(gg[e]), sbit << msh(gg[e]), __ATOMIC_RELAXED,
-                                                  __HIP_MEMORY_SCOPE_WORKGROUP);
-                        const uint64_t m = ballot(ap);
-                        const int pos = nv + add + mask_rank(m);
-                        if (ap) {
-                            if (pos < vcap) V[pos] = (uint16_t)gg[e];
-                            else over = true;
-                        }
-                        add += __popcll(m);
-                    }
-#pragma unroll
-                    for (int e = 0; e < 3; ++e) {
-                        const bool h = act && !vis[e];
-                        const uint64_t m = ballot(h);
+                        const uint64_t m = ballot(h[e]);
                         const int pos = nh + mask_rank(m);
-                        if (h && pos < hcap) {
+                        if (h[e] && pos < hcap) {
                             HA[pos] = (uint16_t)vv[e];
                             HB[pos] = (uint16_t)vv[e == 2 ? 0 : e + 1];
                             HF[pos] = (uint16_t)gg[e];
@@ -807,216 +681,345 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
                         }
                         nh += __popcll(m);
                     }
-                    nv += add;
+                };
+                if (ftop <= FLAT) {
+                    for (int b = 0; b < ftop; b += 64) {
+                        const int f = b + lane;
+                        const f4v pl = w.fpl[min(f, FC - 1)];
+                        const float t = fmaf(pl.x, fqx, fmaf(pl.y, fqy, fmaf(pl.z, fqz, pl.w)));
+                        bool v = t > HULL_FILTER_EPS;
+                        const bool amb = fabsf(t) <= HULL_FILTER_EPS && f < ftop;
+                        if (ballot(amb) && amb) {
+                            const u4v c = w.fv[f];
+                            v = orient_exact(w.vq[c.x], w.vq[c.y], w.vq[c.z], qx, qy, qz) > 0.0;
+                        }
+                        v = v && f < ftop;
+                        const uint64_t m = ballot(v);
+                        if (v) {
+                            const int pos = nv + mask_rank(m);
+                            __hip_atomic_fetch_or(mw(f), (vb | sbit) << msh(f), __ATOMIC_RELAXED,
+                                                  __HIP_MEMORY_SCOPE_WORKGROUP);
+                            if (pos < vcap) V[pos] = (uint16_t)f;
+                        }
+                        nv += __popcll(m);
+                    }
+                    over = nv > vcap;
+                    nv = min(nv, vcap);
                     wsync();
-                    if (nv > vcap) { over = true; nv = vcap; break; }
+                    for (int b = 0; b < nv; b += 64) {
+                        const bool act = b + lane < nv;
+                        const int f = V[act ? b + lane : 0];
+                        const u4v fvl = w.fv[f], nb = w.fn[f];
+                        const int gg[3] = {nb.x, nb.y, nb.z}, vv[3] = {fvl.x, fvl.y, fvl.z};
+                        int back[3];
+                        bool h[3];
+                        u4v gn[3];
+#pragma unroll
+                        for (int e = 0; e < 3; ++e) {
+                            gn[e] = w.fn[gg[e]];
+                            h[e] = act && !((*mw(gg[e]) >> msh(gg[e])) & sbit);
+                        }
+#pragma unroll
+                        for (int e = 0; e < 3; ++e) {
+                            back[e] = (gn[e].x == f) ? 0 : ((gn[e].y == f) ? 1 : 2);
+                            if (h[e])
+                                __hip_atomic_fetch_or(mw(gg[e]), vb << msh(gg[e]), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
+                        }
+                        horizon(h, vv, gg, back);
+                    }
+                } else {
+                    // every visible face tests its three neighbours at once
+                    // (marks, planes and back links loaded together); the first
+                    // visitor of a visible neighbour queues it, and every
+                    // neighbour not visible gives a horizon edge (its test is
+                    // deterministic, so every lane that reaches it agrees)
+                    if (lane == 0) {
+                        __hip_atomic_fetch_or(mw(f0), (vb | sbit) << msh(f0), __ATOMIC_RELAXED,
+                                              __HIP_MEMORY_SCOPE_WORKGROUP);
+                        V[0] = (uint16_t)f0;
+                    }
+                    wsync();
+                    int head = 0;
+                    nv = 1;
+                    while (head < nv) {
+                        const int cnt = min(nv - head, 64);
+                        const bool act = lane < cnt;
+                        int f = 0;
+                        u4v fvl = {0, 0, 0, 0}, nb = {0, 0, 0, 0};
+                        if (act) {
+                            f = V[head + lane];
+                            fvl = w.fv[f];
+                            nb = w.fn[f];
+                        }
+                        const int gg[3] = {nb.x, nb.y, nb.z}, vv[3] = {fvl.x, fvl.y, fvl.z};
+                        uint32_t old[3] = {vb, vb, vb};
+                        bool vis[3] = {false, false, false}, h[3];
+                        int back[3] = {0, 0, 0};
+                        if (act) {
+                            f4v pl[3];
+                            u4v gn[3];
+#pragma unroll
+                            for (int e = 0; e < 3; ++e) {
+                                old[e] = __hip_atomic_fetch_or(mw(gg[e]), vb << msh(gg[e]), __ATOMIC_RELAXED,
+                                                               __HIP_MEMORY_SCOPE_WORKGROUP) >> msh(gg[e]);
+                                pl[e] = w.fpl[gg[e]];
+                                gn[e] = w.fn[gg[e]];
+                            }
+#pragma unroll
+                            for (int e = 0; e < 3; ++e) {
+                                // face_above on the loaded plane
+                                const float t = fmaf(pl[e].x, fqx, fmaf(pl[e].y, fqy, fmaf(pl[e].z, fqz, pl[e].w)));
+                                bool above = t > HULL_FILTER_EPS;
+                                if (!above && t >= -HULL_FILTER_EPS) {
+                                    const u4v gv = w.fv[gg[e]];
+                                    above = orient_exact(w.vq[gv.x], w.vq[gv.y], w.vq[gv.z], qx, qy, qz) > 0.0;
+                                }
+                                vis[e] = above;
+                                back[e] = (gn[e].x == f) ? 0 : ((gn[e].y == f) ? 1 : 2);
+                            }
+                        }
+                        head += cnt;
+                        int add = 0;
+#pragma unroll
+                        for (int e = 0; e < 3; ++e) {
+                            const bool ap = act && vis[e] && !(old[e] & vb);
+                            if (ap)
+                                __hip_atomic_fetch_or(mw(gg[e]), sbit << msh(gg[e]), __ATOMIC_RELAXED,
+                                                      __HIP_MEMORY_SCOPE_WORKGROUP);
+                            const uint64_t m = ballot(ap);
+                            const int pos = nv + add + mask_rank(m);
+                            if (ap && pos < vcap) V[pos] = (uint16_t)gg[e];
+                            add += __popcll(m);
+                            h[e] = act && !vis[e];
+                        }
+                        horizon(h, vv, gg, back);
+                        nv += add;
+                        wsync();
+                        if (nv > vcap) { over = true; nv = vcap; break; }
+                    }
                 }
-                over = ballot(over) != 0;
+                *nv_ = nv;
+                *nh_ = min(nh, hcap);
+                return !over && nh >= 3 && nh <= hcap;
+            };
+            // the lists in LDS hold MA_CAP entries; the best candidate's region
+            // goes to the workspace's own arrays when it is larger
+            int nv = 0, nh = 0;
+            bool ok = false, big = false;
+            if (sk != 0) {
+                ok = region(lst(r, 0), lst(r, 1), lst(r, 2), lst(r, 3), w.mhedge + r * MA_CAP, MA_CAP, MA_CAP, &nv, &nh);
+                if (!ok && r == 0) {
+                    for (int q = lane; q < FC / 2; q += 64)
+                        __hip_atomic_fetch_and(w.mfm + q, ~((vb | sbit) * 0x10001u), __ATOMIC_RELAXED,
+                                               __HIP_MEMORY_SCOPE_WORKGROUP);
+                    wsync();
+                    big = true;
+                    ok = region(w.vis, w.ha, w.hb, w.hface, w.hedge, FC, VC, &nv, &nh);
+                }
                 if (lane == 0) {
-                    cand[r * MA_CI + 6] = nv;
-                    cand[r * MA_CI + 7] = nh;
-                    cand[r * MA_CI + 8] = (!over && nh >= 3 && nh <= hcap) ? 1 : 0;
+                    asptr<AS_LDS, int> c = cand + r * MA_CI;
+                    c[0] = nv;
+                    c[1] = nh;
+                    c[2] = ok ? 1 : 0;
+                    c[4] = qx;
+                    c[5] = qy;
+                    c[6] = qz;
+                    c[7] = big ? 1 : 0;
+                    du[r] = ip;
                 }
             }
             __syncthreads();
-            // E: conflicts - candidate r's visible faces against the others' visited faces
-            for (int f = tid; f < ftop; f += T) {
-                const uint32_t m = (w.mfm[f >> 1] >> msh(f)) & 0xFFFFu;
-                uint32_t sv = (m >> 8) & 0xFFu;
-                const uint32_t vis_by = m & 0xFFu;
-                while (sv) {
-                    const int r = __ffs(sv) - 1;
-                    sv &= sv - 1;
-                    const uint32_t o = vis_by & ~(1u << r);
-                    if (o) __hip_atomic_fetch_or(&crow[r], (int)o, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+            // conflicts: the candidate's visible faces that others visited
+            if (sk != 0) {
+                uint32_t row = 0;
+                for (int j = lane; j < nv; j += 64) {
+                    const int f = big ? (int)w.vis[j] : (int)lst(r, 0)[j];
+                    row |= *mw(f) >> msh(f);
                 }
+                row &= 0xFFu & ~vb;
+#pragma unroll
+                for (int b = 0; b < MA_W; ++b) row |= ballot((row >> b) & 1u) ? 1u << b : 0u;
+                if (lane == 0) cand[r * MA_CI + 3] = (int)row;
             }
             __syncthreads();
-            // F: wave 0 accepts greedily by rank and assigns vertex and face
-            // ids: lane r loads candidate r's sizes and conflict row, the rank
-            // walk runs on scalar broadcasts, then each accepted lane writes
-            // its cone's extra face ids (from the free list, then the top)
-            if (wv == 0) {
-                const int nc = __builtin_amdgcn_readfirstlane(ncand);
-                int c_nv = 0, c_nh = 0, c_ok = 0, c_row = 0;
-                if (lane < nc) {
-                    c_nv = cand[lane * MA_CI + 6];
-                    c_nh = cand[lane * MA_CI + 7];
-                    c_ok = cand[lane * MA_CI + 8];
-                    c_row = crow[lane];
-                }
-                uint32_t acc = 0, blocked = 0;  // blocked: visited the visible faces of an accepted one
-                int nacc = 0, st = HULL_OK;
-                int nf = __builtin_amdgcn_readfirstlane(nfree), ft = __builtin_amdgcn_readfirstlane(ftop);
-                const int nv0 = __builtin_amdgcn_readfirstlane(nvert);
-                int my_vid = 0, my_free = 0, my_ff = 0, my_top = 0;
-                for (int r = 0; r < nc; ++r) {
-                    const int nv = read_lane(c_nv, r), nh = read_lane(c_nh, r);
-                    const uint32_t row = (uint32_t)read_lane(c_row, r);
-                    if (!read_lane(c_ok, r)) {
-                        if (r == 0) { st = HULL_OVERFLOW; break; }
-                        continue;
-                    }
-                    if ((row & acc) || ((blocked >> r) & 1u)) continue;
-                    const int extra = nh > nv ? nh - nv : 0;
-                    const int from_free = min(extra, nf);
-                    const int from_top = extra - from_free;
-                    if (nv0 + nacc >= VC || ft + from_top > FC) {
-                        if (r == 0) { st = HULL_OVERFLOW; break; }
-                        continue;
-                    }
-                    if (lane == r) {
-                        my_vid = nv0 + nacc;
-                        my_free = nf;
-                        my_ff = from_free;
-                        my_top = ft;
-                    }
-                    nf -= from_free;
-                    ft += from_top;
-                    ++nacc;
-                    acc |= 1u << r;
-                    blocked |= row;
-                }
-                // the surplus visible faces of the accepted cones go back to the free list
-                int my_push = 0;
-                for (int r = 0; r < nc; ++r)
-                    if ((acc >> r) & 1u) {
-                        const int nv = read_lane(c_nv, r), nh = read_lane(c_nh, r);
-                        if (lane == r) my_push = nf;
-                        nf += nv > nh ? nv - nh : 0;
-                    }
-                if (lane < nc && ((acc >> lane) & 1u)) {
-                    L16 HN = lane == 0 ? (L16)w.hnew : (L16)lhn(lane);
-                    const int extra = c_nh > c_nv ? c_nh - c_nv : 0;
-                    for (int k = 0; k < extra; ++k)
-                        HN[c_nv + k] = k < my_ff ? w.ffree[my_free - 1 - k] : (uint16_t)(my_top + k - my_ff);
-                    cand[lane * MA_CI + 9] = my_vid;
-                    cand[lane * MA_CI + 10] = my_push;
-                }
-                if (lane == 0) {
-                    misc[0] = (int)acc;
-                    misc[1] = nacc;
-                    misc[2] = ft;
-                    misc[3] = nf;
-                    misc[4] = st;
-                }
+            // accept greedily by rank, and assign vertex and face ids: lane q
+            // holds candidate q's sizes
+            int c_nv = 0, c_nh = 0, c_ok = 1, c_row = 0;
+            if (lane < ncand) {
+                c_nv = cand[lane * MA_CI + 0];
+                c_nh = cand[lane * MA_CI + 1];
+                c_ok = cand[lane * MA_CI + 2];
+                c_row = cand[lane * MA_CI + 3];
             }
-            __syncthreads();
-            const uint32_t acc = (uint32_t)misc[0];
-            if (misc[4] != HULL_OK) { res.status = HULL_OVERFLOW; break; }
-            // G: wave r builds the cone of accepted candidate r
-            if (wv < ncand && ((acc >> wv) & 1u)) {
-                const int r = wv;
-                const int nv = cand[r * MA_CI + 6], nh = cand[r * MA_CI + 7];
-                const int vid = cand[r * MA_CI + 9], push = cand[r * MA_CI + 10];
-                const int qx = cand[r * MA_CI + 3], qy = cand[r * MA_CI + 4], qz = cand[r * MA_CI + 5];
-                L16 V = r == 0 ? (L16)w.vis : (L16)lvis(r);
-                L16 HA = r == 0 ? (L16)w.ha : (L16)lha(r);
-                L16 HB = r == 0 ? (L16)w.hb : (L16)lhb(r);
-                L16 HF = r == 0 ? (L16)w.hface : (L16)lhf(r);
-                L8 HE = r == 0 ? (L8)w.hedge : (L8)(w.mhedge + r * MA_CAP);
-                L16 HN = r == 0 ? (L16)w.hnew : (L16)lhn(r);
+            const bool lost = ballot(c_ok == 0) != 0;  // a region was cut off: its marks are not all listed
+            uint32_t acc = 0, blocked = 0;  // blocked: visited the visible faces of an accepted one
+            int my_vid = 0, my_free = 0, my_ff = 0, my_top = 0, my_push = 0;
+            const int c_extra = c_ok ? max(c_nh - c_nv, 0) : 0;
+            const bool room = nvert + NW <= VC && ftop + wave_sum_i(c_extra) <= FC;
+#pragma unroll
+            for (int q = 0; q < NW; ++q) {
+                const uint32_t row = (uint32_t)read_lane(c_row, q);
+                if (q >= ncand || !read_lane(c_ok, q) || (row & acc) || ((blocked >> q) & 1u)) continue;
+                if (!room && acc) continue;  // at the workspace's end: one at a time
+                acc |= 1u << q;
+                blocked |= row;
+            }
+            {
+                // extra face ids: from the free list, then the top; surplus
+                // visible faces of the accepted cones go back to the free list
+                const bool in = lane < ncand && ((acc >> lane) & 1u);
+                const int own2 = in ? c_extra | (max(c_nv - c_nh, 0) << 16) : 0;
+                const int incl = wave_incl_scan(own2), tot = read_lane(incl, 63);
+                const int before = read_lane(incl - own2, r), mx = read_lane(own2, r) & 0xFFFF;
+                const int used = before & 0xFFFF, all = tot & 0xFFFF;
+                const int rank = __popc(acc & ((1u << r) - 1u));
+                my_vid = nvert + rank;
+                my_free = nfree - min(used, nfree);
+                my_ff = min(mx, my_free);
+                my_top = ftop + max(used - nfree, 0);
+                my_push = nfree - min(all, nfree) + (int)((uint32_t)before >> 16);
+                pvid = nvert + __popc(acc & ((1u << (lane & 31)) - 1u));
+                const int top = ftop + max(all - nfree, 0);
+                // the first candidate is always taken: no room for it, or no
+                // lists for its region, means that the workspace is too small
+                if (!(acc & 1u) || nvert >= VC || top > FC) res.status = HULL_OVERFLOW;
+                nfree = nfree - min(all, nfree) + (int)((uint32_t)tot >> 16);
+                nvert += __popc(acc);
+                ftop = top;
+            }
+            if (res.status != HULL_OK) break;
+            pacc = lane < MA_W && ((acc >> lane) & 1u);
+            const bool mine = sk != 0 && ((acc >> r) & 1u);
+            // the accepted candidate's cone
+            auto cone = [&](auto V, auto HA, auto HB, auto HF, auto HE, auto HN) {
                 if (lane == 0) {
-                    w.vq[vid] = mk_s4(qx, qy, qz, 0);
-                    w.vpid[vid] = cand[r * MA_CI + 2];
+                    w.vq[my_vid] = mk_s4(qx, qy, qz, 0);
+                    w.vpid[my_vid] = ip;
                 }
-                const int mx = max(nh, nv);
-                for (int j = lane; j < mx; j += 64) {
-                    if (j < nv) w.mfcone[V[j]] = (uint8_t)r;
-                    if (j < nh) {
-                        if (j < nv) HN[j] = V[j];
+                for (int j = lane; j < max(nh, nv); j += 64) {
+                    int id;
+                    if (j < nv) {
+                        id = V[j];
+                        w.mst[id] = (uint16_t)((tag << 3) | r);
+                        if (j >= nh) {
+                            u4v t = w.fn[id];
+                            t.w = 0;
+                            w.fn[id] = t;
+                            w.fpl[id] = dead;
+                        }
                     } else {
-                        const int f = V[j];
-                        w.ffree[push + (j - nh)] = (uint16_t)f;
-                        u4v t = w.fn[f];
-                        t.w = 0;
-                        w.fn[f] = t;
-                        u4v u = w.fv[f];
-                        u.w = (uint16_t)it;
-                        w.fv[f] = u;
+                        const int x = j - nv;
+                        id = x < my_ff ? (int)w.ffree[my_free - 1 - x] : my_top + x - my_ff;
                     }
+                    if (j < nh) HN[j] = (uint16_t)id;
                 }
                 wsync();
                 const s4v sp = mk_s4(qx, qy, qz, 0);
-                for (int j = lane; j < nh; j += 64) {
-                    const int a = HA[j], c = HB[j];
+                const int a0 = lane < nh ? (int)HA[lane] : -1, c0 = lane < nh ? (int)HB[lane] : -1;
+                for (int b = 0; b < nh; b += 64) {
+                    const int j = b + lane;
+                    const int a = j < nh ? (int)HA[j] : -1, c = j < nh ? (int)HB[j] : -1;
                     int nx = 0, pv = 0;  // cone faces across (c, apex) and (apex, a)
-                    for (int k = 0; k < nh; ++k) {
-                        if (HA[k] == c) nx = k;
-                        if (HB[k] == a) pv = k;
+                    if (nh <= 64) {
+                        for (int k = 0; k < nh; ++k) {
+                            nx = read_lane(a0, k) == c ? k : nx;
+                            pv = read_lane(c0, k) == a ? k : pv;
+                        }
+                    } else {
+                        for (int k = 0; k < nh; ++k) {
+                            if (HA[k] == c) nx = k;
+                            if (HB[k] == a) pv = k;
+                        }
                     }
-                    const int id = HN[j];
-                    w.fv[id] = mk_u4(a, c, vid, (uint16_t)it);
-                    w.fn[id] = mk_u4(HF[j], HN[nx], HN[pv], 1);
-                    const f4v pl = face_set_plane(w, id, w.vq[a], w.vq[c], sp);
-                    if (nh <= MA_CPL) w.mcpl[r * MA_CPL + j] = pl;
+                    if (j < nh) {
+                        const int id = HN[j], g = HF[j], hn = HN[nx], hp = HN[pv];
+                        w.fv[id] = mk_u4(a, c, my_vid, 0);
+                        w.fn[id] = mk_u4(g, hn, hp, 1);
+                        asptr<AS, uint16_t> slotp = ((asptr<AS, uint16_t>)&w.fn[g]) + HE[j];
+                        *slotp = (uint16_t)id;
+                        const f4v pl = face_set_plane(w, id, w.vq[a], w.vq[c], sp);
+                        if (j < MA_CPL) w.mcpl[r * MA_CPL + j] = pl;
+                    } else if (j < MA_CPL) {
+                        w.mcpl[r * MA_CPL + j] = dead;  // scans go four planes at a time
+                    }
                 }
-                wsync();
-                for (int j = lane; j < nh; j += 64) {
-                    asptr<AS, uint16_t> slotp = ((asptr<AS, uint16_t>)&w.fn[HF[j]]) + HE[j];
-                    *slotp = HN[j];
-                }
+            };
+            if (mine) {
+                if (big) cone(w.vis, w.ha, w.hb, w.hface, w.hedge, w.hnew);
+                else cone(lst(r, 0), lst(r, 1), lst(r, 2), lst(r, 3), w.mhedge + r * MA_CAP, lst(r, 4));
             }
-            nvert += misc[1];
-            ftop = misc[2];
-            nfree = misc[3];
+            // the marks go back to zero where they were set
+            if (lost) {
+                for (int q = tid; q < FC / 2; q += T) w.mfm[q] = 0u;
+            } else if (sk != 0) {
+                const M16 m16 = (M16)w.mfm;
+                for (int j = lane; j < nv; j += 64) m16[big ? (int)w.vis[j] : (int)lst(r, 0)[j]] = 0;
+                for (int j = lane; j < nh; j += 64) m16[big ? (int)w.hface[j] : (int)lst(r, 3)[j]] = 0;
+            }
             __syncthreads();
-            // H: accepted apexes leave the conflict sets; points of replaced
-            // faces move to the cone that replaced them
+            // the accepted apex leaves the conflict sets, and the surplus
+            // faces are free (the ids taken above were read before the barrier)
+            if (mine) {
 #pragma unroll
-            for (int q = 0; q < NW; ++q) {
-                if (q >= ncand || !((acc >> q) & 1u)) continue;
-                const int ip = cand[q * MA_CI + 2];
-                const int own = ip % T, slot = ip / T;
-#pragma unroll
-                for (int k = 0; k < PPL; ++k) {
-                    const int m = -(int)(tid == own && k == slot);
-                    conf[k] = (conf[k] & ~m) | (-2 & m);
-                }
+                for (int k = 0; k < PPL; ++k) key[k] = key[k] == sk ? 0u : key[k];
+                for (int j = nh + lane; j < nv; j += 64)
+                    w.ffree[my_push + (j - nh)] = big ? (uint16_t)w.vis[j] : (uint16_t)lst(r, 0)[j];
             }
-            // the lane's points whose face was replaced this round, as a bit
-            // mask: the wave then loops as often as its busiest lane needs,
-            // not once per point slot that any lane needs
+            // points of replaced faces move to the cone that replaced them:
+            // each lane's as a bit mask, so the wave loops as often as its
+            // busiest lane needs
             uint32_t need = 0;
 #pragma unroll
             for (int k = 0; k < PPL; ++k) {
-                const int c = conf[k];
-                if (c >= 0 && w.fv[c].w == (uint16_t)it) need |= 1u << k;
+                const uint32_t st = w.mst[conf[k]];
+                need |= (key[k] != 0u && (int)(st >> 3) == tag ? 1u : 0u) << k;
             }
-            while (need) {
-                const int k = __ffs(need) - 1;
+            while (ballot(need != 0)) {
+                const bool act = need != 0;
+                const int k = act ? __ffs(need) - 1 : 0;
                 need &= need - 1;
-                const int c = pick(conf, k);
-                const int qx = pick(px, k), qy = pick(py, k), qz = pick(pz, k);
-                const int r = w.mfcone[c];
-                const int nh = cand[r * MA_CI + 7];
-                L16 HN = r == 0 ? (L16)w.hnew : (L16)lhn(r);
-                // the cone's planes in cone order when it kept them (the same
-                // test as face_above, on the same plane values), else by id
-                const bool cp = nh <= MA_CPL;
-                const asptr<AS_LDS, f4v> CP = w.mcpl + r * MA_CPL;
-                const float fx = (float)qx, fy = (float)qy, fz = (float)qz;
+                const int x = hull_pick(px, k), y = hull_pick(py, k), z = hull_pick(pz, k);
+                const int rr = act ? w.mst[hull_pick(conf, k)] & 7 : 0;
+                const asptr<AS_LDS, int> c = cand + rr * MA_CI;
+                const int rn = act ? c[1] : 0;
+                const asptr<AS_LDS, f4v> CP = w.mcpl + rr * MA_CPL;
+                const float fx = (float)x, fy = (float)y, fz = (float)z;
                 int bj = -1;
-                float bd = 0.0f;
-                for (int j = 0; j < nh; ++j) {
-                    const f4v pl = cp ? CP[j] : w.fpl[HN[j]];
-                    const float t = fmaf(pl.x, fx, fmaf(pl.y, fy, fmaf(pl.z, fz, pl.w)));
-                    bool above = t > HULL_FILTER_EPS;
-                    if (!above && t >= -HULL_FILTER_EPS) {
-                        const u4v v = w.fv[HN[j]];
-                        above = orient_exact(w.vq[v.x], w.vq[v.y], w.vq[v.z], qx, qy, qz) > 0.0;
-                    }
-                    if (above && (bj < 0 || t > bd)) {
-                        bj = j;
-                        bd = t;
+                float bd = HULL_FILTER_EPS, near = rn <= MA_CPL ? 1.0f : 0.0f;
+                for (int j = 0; j < min(rn, MA_CPL); j += 4) {
+                    f4v pl[4];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) pl[u] = CP[j + u];
+#pragma unroll
+                    for (int u = 0; u < 4; ++u) {
+                        const float t = fmaf(pl[u].x, fx, fmaf(pl[u].y, fy, fmaf(pl[u].z, fz, pl[u].w)));
+                        near = fminf(near, fabsf(t));
+                        bj = t > bd ? j + u : bj;
+                        bd = fmaxf(bd, t);
                     }
                 }
-                const int best = bj >= 0 ? (int)HN[bj] : -1;
+                auto id_of = [&](int j) { return c[7] ? (int)w.hnew[j] : (int)lst(rr, 4)[j]; };
+                const bool amb = act && near <= HULL_FILTER_EPS;
+                if (ballot(amb) && amb) {  // some test is within the filter's error: decide all exactly
+                    bj = -1;
+                    for (int j = 0; j < rn; ++j) {
+                        float t;
+                        if (face_above(w, id_of(j), x, y, z, &t) && (bj < 0 || t > bd)) {
+                            bj = j;
+                            bd = t;
+                        }
+                    }
+                    if (bj < 0 && x == c[4] && y == c[5] && z == c[6])
+                        __hip_atomic_fetch_min(&du[rr], k * T + tid, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                }
+                const int best = act ? id_of(max(bj, 0)) : 0;
+                const uint32_t nk = bj >= 0 ? mkkey(bd, k) : 0u;
 #pragma unroll
                 for (int kk = 0; kk < PPL; ++kk)
-                    if (kk == k) {
+                    if (act && kk == k) {
                         conf[kk] = best;
-                        dist[kk] = bd;
+                        key[kk] = nk;
                     }
             }
         }

@@ -259,7 +259,7 @@ __global__ __launch_bounds__(64 * BLOCK_NW) void hull_lds_kernel(HullItemArgs a,
 }
 
 // The same with the faces and vertices in global workspace blockIdx.x; the
-// rounds' marks and keys in dynamic LDS (hull_ma_bytes(VC)).
+// rounds' marks and stamps in dynamic LDS (hull_ma_bytes(VC)).
 template <int PPL>
 __global__ __launch_bounds__(64 * BLOCK_NW) void hull_block_kernel(HullItemArgs a, int mode) {
     extern __shared__ __align__(16) char lds[];

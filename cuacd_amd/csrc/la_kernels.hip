@@ -255,7 +255,7 @@ __global__ __launch_bounds__(64 * NW) void la_hull_ldsv(LaHullTask* tasks, const
 
 // Workspace slot blockIdx.x of gws; ids[0, n), or the first min(*dcount, n)
 // when dcount is given, strided over the grid.
-// With `multi`, multi-apex rounds: their per-face marks and keys in the
+// With `multi`, multi-apex rounds: their per-face marks and stamps in the
 // dynamic LDS (hull_ma_bytes(VC)), the faces and vertices in the global
 // workspace.
 template <int PPL>
@@ -1713,7 +1713,7 @@ using BlockFn = void (*)(LaHullTask*, const int*, int, const int*, char*, unsign
                          DPool*, int*);
 
 // Multi-apex rounds for an HBM-workspace kernel of vc vertices (knob
-// multi_hbm; their LDS scratch, 3 bytes per face and 15.5 KB, fits up to
+// multi_hbm; their LDS scratch, 4 bytes per face and 15.4 KB, fits up to
 // 16384 vertices): the flag, and the dynamic LDS it needs, set on the kernel.
 int block_multi(gpu_ctx_t ctx, BlockFn k, int vc, int* multi, unsigned* lds) {
     *multi = (hull_multi_hbm() && vc <= 16384) ? 1 : 0;

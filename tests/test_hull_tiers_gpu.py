@@ -55,3 +55,22 @@ def test_cloud_above_the_stated_maximum_reports_capacity(ctx):
     nv, nt, err = host
     assert nv[0] == len(LO.hull_mesh(clouds[0])[0]) and err[0] == 0
     assert err[1] != 0 and err[2] != 0
+
+
+@pytest.mark.parametrize("kind", ["disc", "twice"])
+@pytest.mark.parametrize("n", [600, 1500, 4000, 9000])
+def test_multi_apex_rounds_at_their_limits_match_oracle(ctx, kind, n):
+    """A region of more faces than the LDS lists hold; points of one grid position owned by different waves."""
+    if kind == "disc":
+        a = np.random.default_rng(n).permutation(n - 2) * (2 * np.pi / (n - 2))
+        c = np.stack([np.cos(a), np.sin(a), np.zeros_like(a)], 1)
+        c = np.concatenate([c, [[0.0, 0.0, 3 / 5108], [0.1, 0.0, -1 / 5108]]]).astype(np.float32)
+    else:
+        half = _sphere(n // 2, n).astype(np.float64)
+        order = np.random.default_rng(n).permutation(2 * len(half))
+        c = np.concatenate([half, half * (1 - 1e-6)])[order].astype(np.float32)
+    (hv, ht, vol), = ctx.batch_hull_dandc_mesh([c])
+    ev, et, evol = LO.hull_mesh(c)
+    assert hv.tobytes() == np.asarray(ev, np.float32).tobytes()
+    assert np.array_equal(ht, et)
+    assert abs(vol - evol) <= 1e-12 * max(abs(evol), 1e-30)
