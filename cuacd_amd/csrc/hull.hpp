@@ -591,8 +591,8 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
         // out the accepted set for itself. (Candidates per share of the faces
         // took block-wide passes over points and faces and ten barriers a round:
         // 21-31k cycles at 1000-2000 points and 78k at 12000, here 13-20k and
-        // 44k with 0.85 to 0.95 of the insertions; 192 clouds of 5-12000 points
-        // 68 -> 36 ms.)
+        // 32k with 0.85 to 0.95 of the insertions; 192 clouds of 5-12000 points
+        // 68 -> 33 ms.)
         static_assert(NW > 1 && NW <= MA_W, "multi-apex rounds need several waves");
         // a conflict key is a point's quantised distance above the high bits,
         // its (inverted) local index in the low ones; 0: inside, or a vertex
@@ -619,11 +619,17 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
             return (__float_as_uint(fmaxf(t, 1e-6f)) & ~IM) | (IM - (uint32_t)(k * T + tid));
         };
         const f4v dead = mk_f4(0.0f, 0.0f, 0.0f, -1.0f);
+        // a point in three registers: x and y, z above its conflict face (any
+        // face where the key is 0), its key (with a register each for x, y,
+        // z, face and distance the rounds of 32 points a lane spilled: 44k
+        // cycles each, 32k without)
         uint32_t key[PPL];
+        int xy[PPL], zc[PPL];
 #pragma unroll
         for (int k = 0; k < PPL; ++k) {
             key[k] = conf[k] >= 0 ? mkkey(dist[k], k) : 0u;
-            conf[k] = max(conf[k], 0);
+            xy[k] = (px[k] & 0xFFFF) | (py[k] << 16);
+            zc[k] = (pz[k] << 16) | max(conf[k], 0);
         }
         asptr<AS_LDS, uint32_t> stw = (asptr<AS_LDS, uint32_t>)w.mst;
         for (int q = tid; q < FC / 2; q += T) {
@@ -645,8 +651,8 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
             for (int k = 1; k < PPL; ++k) sk = max(sk, key[k]);
             sk = wave_max_u32(sk);
             const int ip = (int)(IM - (sk & IM)), own = ip & 63, slot = ip / T;
-            const int qx = read_lane(hull_pick(px, slot), own), qy = read_lane(hull_pick(py, slot), own),
-                      qz = read_lane(hull_pick(pz, slot), own), f0 = read_lane(hull_pick(conf, slot), own);
+            const int pxy = read_lane(hull_pick(xy, slot), own), pzc = read_lane(hull_pick(zc, slot), own);
+            const int qx = (int)(short)pxy, qy = pxy >> 16, qz = pzc >> 16, f0 = pzc & 0xFFFF;
             if (lane == 0) pub[wv] = (int)sk;
             __syncthreads();
             int r = 0, ncand = 0;
@@ -972,15 +978,16 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
             uint32_t need = 0;
 #pragma unroll
             for (int k = 0; k < PPL; ++k) {
-                const uint32_t st = w.mst[conf[k]];
+                const uint32_t st = w.mst[zc[k] & 0xFFFF];
                 need |= (key[k] != 0u && (int)(st >> 3) == tag ? 1u : 0u) << k;
             }
             while (ballot(need != 0)) {
                 const bool act = need != 0;
                 const int k = act ? __ffs(need) - 1 : 0;
                 need &= need - 1;
-                const int x = hull_pick(px, k), y = hull_pick(py, k), z = hull_pick(pz, k);
-                const int rr = act ? w.mst[hull_pick(conf, k)] & 7 : 0;
+                const int hxy = hull_pick(xy, k), hzc = hull_pick(zc, k);
+                const int x = (int)(short)hxy, y = hxy >> 16, z = hzc >> 16;
+                const int rr = act ? w.mst[hzc & 0xFFFF] & 7 : 0;
                 const asptr<AS_LDS, int> c = cand + rr * MA_CI;
                 const int rn = act ? c[1] : 0;
                 const asptr<AS_LDS, f4v> CP = w.mcpl + rr * MA_CPL;
@@ -1018,7 +1025,7 @@ __device__ __forceinline__ HullResult block_quickhull(const HullWS<AS> w, HullBl
 #pragma unroll
                 for (int kk = 0; kk < PPL; ++kk)
                     if (act && kk == k) {
-                        conf[kk] = best;
+                        zc[kk] = (z << 16) | best;
                         key[kk] = nk;
                     }
             }
