@@ -178,29 +178,41 @@ __host__ __device__ __forceinline__ unsigned hull_ws_layout(char* p, int vc, int
     w.fpl = (asptr<AS, f4v>)take(fc * 16u);
     w.fv = (asptr<AS, u4v>)take(fc * 8u);
     w.fn = (asptr<AS, u4v>)take(fc * 8u);
-    w.fstamp = (asptr<AS, int>)take(fc * 4u);
     w.fvis = (asptr<AS, uint8_t>)take((fc + 63u) / 64u * 64u);
     w.ffree = (asptr<AS, uint16_t>)take(fc * 2u);
     w.vis = (asptr<AS, uint16_t>)take(fc * 2u);
     w.vq = (asptr<AS, s4v>)take(v * 8u);
     w.vpid = (asptr<AS, int>)take(v * 4u);
-    w.smap = (asptr<AS, uint16_t>)take(v * 2u);
-    w.emap = (asptr<AS, uint16_t>)take(v * 2u);
-    if (kind == HULL_WS_WAVE) {
-        w.hz = (asptr<AS, u4v>)take(v * 8u);
-        w.pq = (asptr<AS, s4v>)take((unsigned)np * 8u);
-        w.cpl = (asptr<AS, f4v>)take(WAVE_CPL * 16u);
-    } else {
+    const bool multi = kind == HULL_WS_MULTI && AS == AS_LDS;
+    if (!multi) {
+        w.smap = (asptr<AS, uint16_t>)take(v * 2u);
+        w.emap = (asptr<AS, uint16_t>)take(v * 2u);
+    }
+    if (kind != HULL_WS_WAVE) {
         w.hface = (asptr<AS, uint16_t>)take(v * 2u);
         w.hedge = (asptr<AS, uint8_t>)take(v);
         w.ha = (asptr<AS, uint16_t>)take(v * 2u);
         w.hb = (asptr<AS, uint16_t>)take(v * 2u);
     }
     w.hnew = (asptr<AS, uint16_t>)take(v * 2u);
+    // what only the quickhull uses shares its bytes with what only the
+    // canonical form does (the block's single-apex steps use fstamp themselves)
+    const unsigned o0 = off;
+    unsigned o1 = off;
+    if (kind == HULL_WS_WAVE) {
+        w.hz = (asptr<AS, u4v>)take(v * 8u);
+        w.pq = (asptr<AS, s4v>)take((unsigned)np * 8u);
+        w.cpl = (asptr<AS, f4v>)take(WAVE_CPL * 16u);
+        o1 = off;
+        off = o0;
+    } else if (multi) {
+        o1 = o0 + hull_ma_layout(p ? p + o0 : nullptr, fc, &w);
+    }
+    w.fstamp = (asptr<AS, int>)take(fc * 4u);
     w.vout = (asptr<AS, uint16_t>)take(v * 2u);
     w.vref = (asptr<AS, uint8_t>)take(v);
     w.cv = (asptr<AS, int>)take(v * 8u);
-    if (kind == HULL_WS_MULTI && AS == AS_LDS) off += hull_ma_layout(p ? p + off : nullptr, fc, &w);
+    if (o1 > off) off = o1;
     // bm / wpre / ctr live in HullBlockLDS (hull_ws_attach)
     w.VC = vc;
     w.FC = (int)fc;

@@ -96,8 +96,8 @@ __device__ __forceinline__ bool la_hull_item(LaHullTask& t, const HullWS<AS> w, 
     if constexpr (NW >= 8 && PPL * T <= 16384) {
         // multi-apex rounds (the workspace was carved or attached with their
         // scratch; the four-wave tiers keep single-apex steps and do not
-        // compile them); the point index field of their keys holds 14 bits
-        if (multi && n <= PPL * T) r = hull_quickhull<PPL, AS, NW, true>(w, sb, n, px, py, pz);
+        // compile them)
+        if (multi) r = hull_quickhull<PPL, AS, NW, true>(w, sb, n, px, py, pz);
         else r = hull_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
     } else {
         r = hull_quickhull<PPL, AS, NW>(w, sb, n, px, py, pz);
