@@ -287,8 +287,8 @@ __global__ __launch_bounds__(64 * LA_BLOCK_NW) void la_hull_block(LaHullTask* ta
 // full set's. Three launches over the same list, one record per set between
 // them: the extremes (one wave per set, passes over the points), the rough
 // hull of the 80 extreme points (one wave per set: its insertion steps need
-// no block barrier, and many sets share a CU), the filter (four waves).
-constexpr int KD_T = 256;
+// no block barrier, and many sets share a CU), the filter (eight waves).
+constexpr int KD_T = 512;
 constexpr int KD_NW = KD_T / 64;
 constexpr int KD_NE = 2 * KDOP_AXES_N;   // extreme points
 constexpr int KD_MAXPL = 2 * 128 + 8;    // rough faces kept as filter planes
@@ -462,13 +462,17 @@ __global__ __launch_bounds__(64) void la_kdop_rough_kernel(LaHullTask* tasks, co
 // strictly inside a solid whose vertices are points of the set, so it cannot
 // be an extreme point; quantized duplicates share the decision. (Both grids
 // are right-handed, so the faces keep their outward orientation.) The kept
-// points, in input order, go to a scratch copy.
+// points, in input order, go to a scratch copy. Most points are inside and
+// read every plane from LDS: four planes a step keep the reads in flight (one
+// a step was a chain of LDS latencies), and eight waves a set shorten the
+// largest sets, which a level waits for. Against four waves at a plane a step,
+// eager scoring of 720 cuts 19.8 -> 18.3 ms, 960 in a plan 11.9 -> 11.1.
 __global__ __launch_bounds__(KD_T) void la_kdop_filter_kernel(LaHullTask* tasks, const int* ids, int n,
                                                               const int* dcount, const KdopRec* rec, int2* res,
                                                               DPool* pool, int* err) {
     __shared__ double4 dpl[KD_MAXPL];
     __shared__ float4 fpl[KD_MAXPL];  // the same planes in FP32 ...
-    __shared__ float fbd[KD_MAXPL];   // ... and a bound on that form's error
+    __shared__ float4 fbd[KD_MAXPL / 4];  // ... and a bound on that form's error
     __shared__ int s_cnt[KD_NW];
     __shared__ unsigned long long s_filt;
     if ((int)blockIdx.x >= (dcount ? min(*dcount, n) : n)) return;
@@ -476,7 +480,7 @@ __global__ __launch_bounds__(KD_T) void la_kdop_filter_kernel(LaHullTask* tasks,
     if (R.status != 0) return;
     LaHullTask& t = tasks[ids[blockIdx.x]];
     const int tid = threadIdx.x, lane = lane_id(), wv = tid >> 6;
-    const float* P = t.pts;
+    const float* P = in_hbm(t.pts);
     const int np = t.n;
     const QFrame full = R.full;
     const int npl = R.npl;
@@ -501,12 +505,17 @@ __global__ __launch_bounds__(KD_T) void la_kdop_filter_kernel(LaHullTask* tasks,
         // |w| (grid coordinates are below 8192 in magnitude); 2^-20 T is four
         // times that sum
         fpl[c] = make_float4((float)nx, (float)ny, (float)nz, (float)pw);
-        fbd[c] = (float)((fabs(nx) + fabs(ny) + fabs(nz)) * 8192.0 + fabs(pw)) * 0x1p-20f;
+        ((float*)fbd)[c] = (float)((fabs(nx) + fabs(ny) + fabs(nz)) * 8192.0 + fabs(pw)) * 0x1p-20f;
+    }
+    const int npl4 = (npl + 3) & ~3;
+    for (int c = npl + tid; c < npl4; c += KD_T) {  // planes nothing is near
+        fpl[c] = make_float4(0.0f, 0.0f, 0.0f, 1e30f);
+        ((float*)fbd)[c] = 0.0f;
     }
     // filtered buffer: the points on or outside some rough face, in input order
     if (tid == 0) s_filt = (unsigned long long)heap_alloc(pool, 1, 12ull * (np + KD_NE), err);
     __syncthreads();
-    float* filt = (float*)s_filt;
+    float* filt = in_hbm((float*)s_filt);
     if (!filt) {
         if (tid == 0) { t.err = KERR_KDOP_SCRATCH_OOM; res[blockIdx.x] = make_int2(-1, 0); }
         return;
@@ -527,14 +536,25 @@ __global__ __launch_bounds__(KD_T) void la_kdop_filter_kernel(LaHullTask* tasks,
             // bound; only the rest take the exact test, so the decision is
             // the exact one.
             const float fx = (float)qx, fy = (float)qy, fz = (float)qz;
-            for (int f = 0; f < npl; ++f) {
-                const float4 pf = fpl[f];
-                const float sf = fmaf(pf.x, fx, fmaf(pf.y, fy, fmaf(pf.z, fz, -pf.w)));
-                const float bf = fbd[f];
-                if (sf > bf) { keep = true; break; }
-                if (sf >= -bf) {
-                    const double4 pl = dpl[f];
-                    if (pl.x * qx + pl.y * qy + pl.z * qz - pl.w >= 0.0) { keep = true; break; }
+            for (int f = 0; f < npl4 && !keep; f += 4) {
+                const float4 b4 = fbd[f >> 2];
+                const float bf[4] = {b4.x, b4.y, b4.z, b4.w};
+                float sf[4];
+                bool near = false;
+#pragma unroll
+                for (int u = 0; u < 4; ++u) {
+                    const float4 pf = fpl[f + u];
+                    sf[u] = fmaf(pf.x, fx, fmaf(pf.y, fy, fmaf(pf.z, fz, -pf.w)));
+                    keep = keep || sf[u] > bf[u];
+                    near = near || sf[u] >= -bf[u];
+                }
+                if (near && !keep) {
+#pragma unroll
+                    for (int u = 0; u < 4; ++u)
+                        if (sf[u] >= -bf[u]) {
+                            const double4 pl = dpl[f + u];
+                            keep = keep || pl.x * qx + pl.y * qy + pl.z * qz - pl.w >= 0.0;
+                        }
                 }
             }
         }
