@@ -1521,78 +1521,6 @@ __device__ __forceinline__ int hull_rank_vertices(const HullWS<AS> w, HullBlockL
     return carry;
 }
 
-template <int AS, int NW>
-__device__ __forceinline__ int hull_count_faces(const HullWS<AS> w, HullBlockLDS* sb, const HullResult& r) {
-    int c = 0;
-    for (int f = threadIdx.x; f < r.ftop; f += 64 * NW) c += w.fn[f].w ? 1 : 0;
-    return block_sum_i<NW>(c, sb);
-}
-
-// Write triangles (output vertex indices) in face-id order; returns count.
-template <int AS, int NW>
-__device__ __forceinline__ int hull_write_tris(const HullWS<AS> w, HullBlockLDS* sb, const HullResult& r,
-                                      int* __restrict__ out_tris) {
-    const int tid = threadIdx.x;
-    int base = 0;
-    for (int b = 0; b < r.ftop; b += 64 * NW) {
-        const int f = b + tid;
-        const bool alive = f < r.ftop && w.fn[f].w;
-        const uint64_t m = ballot(alive);
-        int wbase = 0;
-        if (NW > 1) {
-            const int wv = tid >> 6;
-            if (lane_id() == 0) sb->bc[wv] = __popcll(m);
-            __syncthreads();
-            for (int i = 0; i < wv; ++i) wbase += sb->bc[i];
-        }
-        if (alive) {
-            const int t = base + wbase + mask_rank(m);
-            const u4v v = w.fv[f];
-            out_tris[3 * t + 0] = w.vout[v.x];
-            out_tris[3 * t + 1] = w.vout[v.y];
-            out_tris[3 * t + 2] = w.vout[v.z];
-        }
-        if (NW > 1) {
-            int tot = 0;
-            for (int i = 0; i < NW; ++i) tot += sb->bc[i];
-            base += tot;
-            __syncthreads();
-        } else {
-            base += __popcll(m);
-        }
-    }
-    return base;
-}
-
-// FP64 divergence-theorem volume over live faces, original fp32 coordinates
-// of the point with local id p fetched by `pos(p, xyz)`. Anchored at the first
-// vertex of the lowest live face to avoid cancellation. Block-uniform result.
-template <int AS, int NW, class PosFn>
-__device__ __forceinline__ double hull_volume_f64(const HullWS<AS> w, HullBlockLDS* sb, const HullResult& r, PosFn pos) {
-    int f0 = 0;
-    for (int b = 0; b < r.ftop; b += 64) {
-        const uint64_t m = ballot(b + lane_id() < r.ftop && w.fn[b + lane_id()].w);
-        if (m) { f0 = b + __builtin_ffsll((long long)m) - 1; break; }
-    }
-    float a[3];
-    pos(w.vpid[w.fv[f0].x], a);
-    const double ax = a[0], ay = a[1], az = a[2];
-    double acc = 0.0;
-    for (int f = threadIdx.x; f < r.ftop; f += 64 * NW) {
-        if (!w.fn[f].w) continue;
-        const u4v v = w.fv[f];
-        float p0[3], p1[3], p2[3];
-        pos(w.vpid[v.x], p0);
-        pos(w.vpid[v.y], p1);
-        pos(w.vpid[v.z], p2);
-        const double x0 = p0[0] - ax, y0 = p0[1] - ay, z0 = p0[2] - az;
-        const double x1 = p1[0] - ax, y1 = p1[1] - ay, z1 = p1[2] - az;
-        const double x2 = p2[0] - ax, y2 = p2[1] - ay, z2 = p2[2] - az;
-        acc += x0 * (y1 * z2 - z1 * y2) + y0 * (z1 * x2 - x1 * z2) + z0 * (x1 * y2 - y1 * x2);
-    }
-    return block_sum_d<NW>(acc, sb) / 6.0;
-}
-
 // ---------------------------------------------------------------------------
 // Canonical form of a finished hull
 // ---------------------------------------------------------------------------
