@@ -1483,7 +1483,8 @@ using WaveFn = void (*)(LaHullTask*, const int*, int, const int*, int, int*, DPo
 //     (CUACD_HULL_W8, 0..15; default 5). On the 64-mesh search step a
 //     513-1024-point hull takes 0.38 ms on eight waves against 0.69 ms on
 //     four (two workgroups per CU against three), and the step went from
-//     2.05 s to 1.96 s; the 257-512-point tier packs better on four waves
+//     2.05 s to 1.96 s; the 257-512-point bits matter only with wide_min
+//     below 512, where that tier packs better on four waves
 //   14 multi_hbm: multi-apex rounds in the HBM-workspace tiers (their
 //     per-face marks in LDS; CUACD_HULL_MULTI_HBM, 0/1;
 //     default 1). These tiers hold the hulls with the most corners, so the
