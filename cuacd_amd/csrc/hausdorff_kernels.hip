@@ -271,14 +271,17 @@ __global__ __launch_bounds__(HD_T) void hd_query_kernel(const HdTask* __restrict
         }
         return p;
     };
+    // a snapshot of the running maximum, one value for the whole wave: the
+    // other waves raise it meanwhile, and lanes that read it one by one could
+    // disagree about a branch that the wave's reductions have to take together
     auto cur = [&] {
-        return __uint_as_float(__hip_atomic_load(&s.cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP));
+        return __uint_as_float(uniform(__hip_atomic_load(&s.cur, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP)));
     };
     // exact searches of the listed samples [0, n), a wave each
     auto search = [&](int n) {
-        for (int k = wv; k < n; k += HD_T / 64) {
-            const int j = s.list[k];
-            const float u = s.ub[j], c = cur();
+        for (int k = uniform(wv); k < n; k += HD_T / 64) {
+            const int j = uniform((int)s.list[k]);
+            const float u = __uint_as_float(uniform(__float_as_uint(s.ub[j]))), c = cur();
             if (!(u > c)) continue;
             const float d = hd_wave_nearest_d2(bvh, {s.px[j], s.py[j], s.pz[j]}, u, c);
             if (d > c && lane_id() == 0) atomicMax(&s.cur, __float_as_uint(d));

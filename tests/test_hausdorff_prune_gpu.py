@@ -40,3 +40,16 @@ def test_reference_sampler_is_the_same_alone_and_in_a_batch(ctx, copies):
             got, want = (ab[i + k * len(p)], ba[i + k * len(p)]), (one[0][0], one[1][0])
             # the nearest triangle is the same up to the rounding of two squared distances
             assert np.allclose(got, want, rtol=2e-6, atol=0)
+
+
+@pytest.mark.parametrize("copies", [1, 24])
+def test_running_maximum_shared_by_waves_gives_the_same_bits(ctx, copies):
+    """Waves raise the maximum while others search against it: no interleaving may lose a distance or change one."""
+    p = _pairs() + [tuple(datasets.noisy_icospheres(2, 3, 0.1, seed=7))]
+    n = 3000  # several batches of samples per workgroup and several workgroups per pair
+    want = None
+    for _ in range(6):
+        ab, ba = ctx.batch_hausdorff([x for x, _ in p] * copies, [y for _, y in p] * copies, n_samples=n)
+        got = np.stack([ab, ba]).reshape(2, copies, len(p))
+        want = got[:, :1] if want is None else want
+        assert np.array_equal(got, np.broadcast_to(want, got.shape))
