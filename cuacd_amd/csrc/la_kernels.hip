@@ -1625,10 +1625,14 @@ int launch_wave_ids(HullCall& hc, int sk, LaHullTask* d_tasks, const int* d_ids,
     const int kid = ppl == 1 ? KT_HULL_W1 : ppl == 2 ? KT_HULL_W2 : ppl == 4 ? KT_HULL_W4 : ppl == 8 ? KT_HULL_W8
                                                                                                      : KT_HULL_W16;
     // the device-counted call (score plans) keeps the four- and eight-wave
-    // kernels above 256 points and one launch for the tiers below: a plan's
-    // replay with one-wave first passes ended in a memory fault whose cause
-    // was not found
-    const int wm = dcnt && hull_wide_min() > 0 ? std::min(hull_wide_min(), 256) : hull_wide_min();
+    // kernels above 256 points, whatever the knob says, and one launch for the
+    // tiers below: a plan's replay with one-wave first passes ended in a memory
+    // fault. The kernel is not the cause by its indexes: on the CPU, with every
+    // workspace access checked, it stays in bounds at 1/8 to 7/8 of the
+    // vertices and its retries give the full capacity's hulls. A plan's arena
+    // holds four retry lists, and such passes would add a fifth
+    int wm = hull_wide_min();
+    if (dcnt && (wm <= 0 || wm > 256)) wm = 256;
     if (wm > 0 && ppl >= 8 && 64 * ppl > wm && hull_half_cap()) {
         // first pass with a reduced vertex capacity (several hulls per CU),
         // then the sets whose hulls did not fit, at full capacity
