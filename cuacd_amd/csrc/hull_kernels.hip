@@ -335,7 +335,8 @@ int launch_wave(gpu_ctx_t ctx, HullItemArgs a, int maxn, int mode) {
 }
 
 // Kernel and workspace of the global-memory tier for clouds of up to maxn
-// points; raises the kernel's dynamic-LDS limit to the rounds' scratch.
+// points. The dynamic-LDS limit is the kernel's, and calls on other threads may
+// launch it with other sizes: it is set to what the largest one needs.
 int block_shape(gpu_ctx_t ctx, HullItemArgs* a, int maxn, KernelFn k4, KernelFn k8, KernelFn k16, KernelFn k32,
                 KernelFn* k, unsigned* lds) {
     constexpr int T = 64 * BLOCK_NW;
@@ -344,7 +345,8 @@ int block_shape(gpu_ctx_t ctx, HullItemArgs* a, int maxn, KernelFn k4, KernelFn 
     a->VC = a->NP;
     a->gws_stride = (hull_ws_bytes<AS_GLOBAL>(a->VC, a->NP) + 255ull) & ~255ull;
     *lds = hull_ma_bytes(a->VC);
-    HIP_TRY(hipFuncSetAttribute((const void*)*k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds));
+    HIP_TRY(hipFuncSetAttribute((const void*)*k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)hull_ma_bytes(BLOCK_MAX)));
     return 0;
 }
 

@@ -1739,11 +1739,15 @@ using BlockFn = void (*)(LaHullTask*, const int*, int, const int*, char*, unsign
 
 // Multi-apex rounds for an HBM-workspace kernel of vc vertices (knob
 // multi_hbm; their LDS scratch, 4 bytes per face and 15.4 KB, fits up to
-// 16384 vertices): the flag, and the dynamic LDS it needs, set on the kernel.
+// 16384 vertices): the flag, and the dynamic LDS it needs. The kernel's limit
+// is set to what its largest launch needs, since other threads' calls may
+// launch it with other sizes.
 int block_multi(gpu_ctx_t ctx, BlockFn k, int vc, int* multi, unsigned* lds) {
     *multi = (hull_multi_hbm() && vc <= 16384) ? 1 : 0;
     *lds = *multi ? hull_ma_bytes(vc) : 0u;
-    if (*lds > 0) HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds));
+    if (*lds > 0)
+        HIP_TRY(hipFuncSetAttribute((const void*)k, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)hull_ma_bytes(HULL_NP_MAX)));
     return 0;
 }
 
