@@ -1453,10 +1453,11 @@ using WaveFn = void (*)(LaHullTask*, const int*, int, const int*, int, int*, DPo
 //     sets (CUACD_HULL_LDSB8_VCAP, 0 = none: straight to the HBM tier; else
 //     64..1024; default 1024); hulls with more corners are redone in the HBM
 //     tier
-//   9 cut_lds_verts: plane cuts of meshes with up to this many vertices keep
-//     their per-vertex state in LDS and write no per-triangle scratch
-//     (CUACD_CUT_LDS_VERTS, 0 = every cut on the heap-scratch path, else
-//     256..110592; default 98304); bit-identical halves either way
+//   9 cut_lds_verts: plane cuts of meshes with up to this many vertices (at
+//     most PC_LDS_VERTS_FIT, about 106 thousand) keep their per-vertex state
+//     in LDS and write no per-triangle scratch (CUACD_CUT_LDS_VERTS, 0 = every
+//     cut on the heap-scratch path, else 256..110592; default 98304);
+//     bit-identical halves either way
 //   10 lpt: each hull tier's sets are launched largest first (CUACD_HULL_LPT,
 //     0/1; default 0): the longest insertion chains start on the first
 //     workgroups and the short ones fill in behind them. On the 64-mesh
@@ -2329,7 +2330,7 @@ int la_launch_score(gpu_ctx_t ctx, LaScoreTask* d_tasks, int n, int max_nv) {
     const size_t lds = lds_nv > 0 ? ((size_t)lds_nv + 15) / 16 * 16 : 0;
     if (lds > 0)
         HIP_TRY(hipFuncSetAttribute((const void*)la_score_kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
-                                    (int)lds));
+                                    PC_LDS_VERTS_MAX));
     hipLaunchKernelGGL(la_score_kernel, dim3(n), dim3(PC_T), lds, ctx->stream, d_tasks, n, ctx->d_pool, ctx->d_err,
                        lds_nv);
     HIP_TRY(hipGetLastError());
@@ -2385,11 +2386,14 @@ int cut_lds_verts() {
 
 int pc_lds_launch(gpu_ctx_t ctx, const void* kernel, int max_nv, int* lds_nv, size_t* lds_bytes) {
     (void)ctx;
-    const int cap = cut_lds_verts();
+    const int cap = std::min(cut_lds_verts(), PC_LDS_VERTS_FIT);
     *lds_nv = std::min(std::max(max_nv, 0), cap);
     *lds_bytes = *lds_nv > 0 ? (size_t)pc_lds_bytes(*lds_nv) : 0;
+    // the kernel's limit, for the largest launch: other threads' calls may
+    // launch it with other meshes
     if (*lds_bytes > 0)
-        HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)*lds_bytes));
+        HIP_TRY(hipFuncSetAttribute(kernel, hipFuncAttributeMaxDynamicSharedMemorySize,
+                                    (int)pc_lds_bytes(PC_LDS_VERTS_FIT)));
     return 0;
 }
 

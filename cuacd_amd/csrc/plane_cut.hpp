@@ -41,8 +41,7 @@ constexpr int PC_T = 256;
 constexpr float PC_EPS = 1e-6f;
 constexpr int PC_MAX_LOOPS = 256;
 constexpr unsigned long long PC_EMPTY = ~0ull;
-// most vertices of an LDS-resident cut (its dynamic LDS stays under 152 KiB)
-constexpr int PC_LDS_VERTS_MAX = 110592;
+constexpr int PC_LDS_VERTS_MAX = 110592;  // upper end of the cut_lds_verts knob
 
 struct PcMesh {
     float* v;   // heap chunk (verts, then tris) - free with heap_free(v)
@@ -1276,6 +1275,12 @@ __device__ inline PcResult plane_cut_block(const float* __restrict__ V, const in
 __host__ __device__ constexpr unsigned long long pc_lds_bytes(long long nv) {
     return ((unsigned long long)nv + 15ull) / 16ull * 16ull + 24ull * (((unsigned long long)nv + 63ull) / 64ull);
 }
+
+// Most vertices of an LDS-resident cut: what a CU's 160 KiB hold beside the
+// kernel's static LDS (88 bytes per 64 vertices). Larger meshes take
+// plane_cut_block, whatever the knob says.
+constexpr unsigned long long PC_CU_LDS = 160ull * 1024ull;
+constexpr int PC_LDS_VERTS_FIT = (int)((PC_CU_LDS - sizeof(PcLDS) - 512ull) / pc_lds_bytes(64) * 64ull);
 
 // One triangle as the LDS-resident cut sees it: vertex ids and signs, kept in
 // scalars (no private arrays, so nothing is placed in scratch memory).
