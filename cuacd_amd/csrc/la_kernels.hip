@@ -648,7 +648,7 @@ __global__ __launch_bounds__(256) void la_union_kernel(LaHullTask* tasks, const 
 // ---------------------------------------------------------------------------
 // Level-0 cut: both closed halves (kept in heap 0), volumes and boxes
 // ---------------------------------------------------------------------------
-__device__ inline void la_block_bbox(const float* v, int nv, float* lo, float* hi, PcLDS* s, float (*scr)[6]) {
+__device__ inline void la_block_bbox(const float* v, int nv, float* lo, float* hi, PcShared* s, float (*scr)[6]) {
     float mn[3] = {1e30f, 1e30f, 1e30f}, mx[3] = {-1e30f, -1e30f, -1e30f};
     for (int i = threadIdx.x; i < nv; i += PC_T)
         for (int j = 0; j < 3; ++j) {
@@ -731,7 +731,7 @@ __global__ __launch_bounds__(PC_T, 4) void la_cut_kernel(LaCutTask* tasks, int n
 // the plane), bit 2 in the positive point set, bit 3 in the negative one - in
 // fl: LDS when the mesh fits the launch's dynamic LDS, else the heap chunk F.
 template <bool LDS>
-__device__ __forceinline__ void la_score_item(LaScoreTask& T, uint8_t* fl, char* F, PcLDS& s, double (*dsum)[PC_T / 64],
+__device__ __forceinline__ void la_score_item(LaScoreTask& T, uint8_t* fl, char* F, PcShared& s, double (*dsum)[PC_T / 64],
                                               int* wcnt, DPool* pool, int* err) {
     const int tid = threadIdx.x, wv = tid >> 6;
     const float* V = in_hbm(T.v);
@@ -1021,7 +1021,7 @@ __device__ __forceinline__ void la_score_item(LaScoreTask& T, uint8_t* fl, char*
 
 __global__ __launch_bounds__(PC_T) void la_score_kernel(LaScoreTask* tasks, int n, DPool* pool, int* err,
                                                         int lds_nv) {
-    __shared__ PcLDS s;
+    __shared__ PcShared s;
     extern __shared__ __align__(16) unsigned char pc_dyn[];
     __shared__ double dsum[2][PC_T / 64];
     __shared__ int wcnt[PC_T / 64];
@@ -1059,7 +1059,7 @@ __device__ inline void uf_union(int* par, int a, int b) {
 }
 
 __global__ __launch_bounds__(PC_T) void la_comp_kernel(LaCompTask* tasks, int n, DPool* pool, int* err) {
-    __shared__ PcLDS s;
+    __shared__ PcShared s;
     __shared__ double dred[PC_T / 64];
     __shared__ float scr[PC_T / 64][6];
     if ((int)blockIdx.x >= n) return;
@@ -1200,7 +1200,7 @@ __device__ inline bool la_unit_normal(const float* V, const int* Tr, int f, floa
 
 __global__ __launch_bounds__(PC_T) void la_edges_kernel(LaEdgeTask* tasks, int n, float cos_pos, float cos_neg,
                                                         int pos_mode, int neg_mode, DPool* pool, int* err) {
-    __shared__ PcLDS s;
+    __shared__ PcShared s;
     if ((int)blockIdx.x >= n) return;
     LaEdgeTask& T = tasks[blockIdx.x];
     const int tid = threadIdx.x;
@@ -1290,7 +1290,7 @@ __global__ __launch_bounds__(PC_T) void la_edges_kernel(LaEdgeTask* tasks, int n
 }
 
 __global__ __launch_bounds__(PC_T) void la_bbox_kernel(LaBoxTask* tasks, int n) {
-    __shared__ PcLDS s;
+    __shared__ PcShared s;
     __shared__ float scr[PC_T / 64][6];
     if ((int)blockIdx.x >= n) return;
     LaBoxTask& T = tasks[blockIdx.x];

@@ -56,11 +56,26 @@ struct PcResult {
     int has_box;  // 1: PcLDS::boxr holds both halves' vertex bounds (LDS-resident cut, status 0)
 };
 
+// Block-wide scratch of the mesh kernels (scans, sums, broadcast pointers).
+struct PcShared {
+    int ired[PC_T / 64];
+    double dred[PC_T / 64];
+    int cnt[8];
+    int wtot[PC_T / 64][4];
+    float box[PC_T / 64][12];
+    float boxr[12];  // positive side min xyz, max xyz; negative side min xyz, max xyz
+    void* ptr[4];
+    int fail;
+};
+static_assert(sizeof(PcShared) <= 512, "scratch that every mesh kernel's workgroups carry");
+
 // Boundaries of up to PC_CAP_LDS edges (and polygons of as many vertices) are
 // linked, labelled and ear-clipped in LDS.
 constexpr int PC_CAP_LDS = 1024;
 
-struct PcLDS {
+// What a cut has beside that: the cap builder's loops and work arrays. 16 KB,
+// which kernels that build no cap leave to their workgroups' number per CU.
+struct PcLDS : PcShared {
     union {
         struct {  // boundary edges
             uint16_t succ[PC_CAP_LDS], lab[PC_CAP_LDS], rank[PC_CAP_LDS], jmp[PC_CAP_LDS];
@@ -72,15 +87,7 @@ struct PcLDS {
         } c;
     };
     int flag[2];
-    int ired[PC_T / 64];
-    double dred[PC_T / 64];
-    int cnt[8];
-    int wtot[PC_T / 64][4];
-    float box[PC_T / 64][12];
-    float boxr[12];  // positive side min xyz, max xyz; negative side min xyz, max xyz
-    void* ptr[4];
     int n_loops;
-    int fail;
     int loop_start[PC_MAX_LOOPS + 1];
     int loop_parent[PC_MAX_LOOPS];
     int loop_hole[PC_MAX_LOOPS];
@@ -124,7 +131,7 @@ __device__ __forceinline__ int pc_ht_find(const unsigned long long* keys, uint32
 
 // Block-wide exclusive scan over n elements of f(i) (int). Contiguous chunks.
 template <class F>
-__device__ int pc_block_scan(int n, int* out, PcLDS* s, F f) {
+__device__ int pc_block_scan(int n, int* out, PcShared* s, F f) {
     s = in_lds(s);
     const int tid = threadIdx.x, wv = tid >> 6;
     const int per = (n + PC_T - 1) / PC_T;
@@ -149,7 +156,7 @@ __device__ int pc_block_scan(int n, int* out, PcLDS* s, F f) {
     return tot;
 }
 
-__device__ __forceinline__ void* pc_alloc(DPool* pool, unsigned long long bytes, PcLDS* s, int slot, int* err,
+__device__ __forceinline__ void* pc_alloc(DPool* pool, unsigned long long bytes, PcShared* s, int slot, int* err,
                                           int heap_id) {
     if (threadIdx.x == 0) s->ptr[slot] = heap_alloc(pool, heap_id, bytes ? bytes : 16, err);
     __syncthreads();
@@ -167,7 +174,7 @@ struct P2 {
 __device__ __forceinline__ float cross2(P2 a, P2 b, P2 c) { return (b.u - a.u) * (c.v - a.v) - (b.v - a.v) * (c.u - a.u); }
 
 // Whole-mesh copy to one side (no crossing edges or failed cap).
-__device__ inline PcMesh pc_copy_mesh(const float* V, const int* T, int nv, int nt, DPool* pool, PcLDS* s, int* err) {
+__device__ inline PcMesh pc_copy_mesh(const float* V, const int* T, int nv, int nt, DPool* pool, PcShared* s, int* err) {
     PcMesh m{nullptr, nullptr, 0, 0, 0.0};
     const unsigned long long vb = al16(12ull * nv), tb = al16(12ull * nt);
     float* chunk = (float*)pc_alloc(pool, vb + tb, s, 0, err, 0);
@@ -183,7 +190,7 @@ __device__ inline PcMesh pc_copy_mesh(const float* V, const int* T, int nv, int 
 }
 
 // FP64 volume of a mesh chunk (anchored at vertex 0), block-uniform.
-__device__ inline double pc_volume(const float* v, const int* t, int nt, PcLDS* s) {
+__device__ inline double pc_volume(const float* v, const int* t, int nt, PcShared* s) {
     v = in_hbm(v);
     t = in_hbm(t);
     s = in_lds(s);
