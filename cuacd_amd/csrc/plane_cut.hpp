@@ -1412,11 +1412,9 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
     if (tid == 0) { s->cnt[0] = 0; s->fail = 0; }
     // the wave's special triangles (crossing an edge, or with two vertices on
     // the plane), in triangle order from sl[tb]: the passes that only concern
-    // them walk this list instead of the whole triangle range; spos: their
-    // first output positions on both sides
-    int* sl = (int*)pc_alloc(pool, al16(4ull * nt) + 8ull * nt + 16, s, 1, err, 1);
+    // them walk this list instead of the whole triangle range
+    int* sl = (int*)pc_alloc(pool, 4ull * nt + 16, s, 1, err, 1);
     if (!sl) { R.status = -1; return R; }
-    int2* spos = (int2*)((char*)sl + al16(4ull * nt));
     int nsl = 0;  // wave-uniform
     {
         int cnp = 0, cnn = 0, cnc = 0, anyp = 0, anyn = 0;
@@ -1453,18 +1451,19 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
         cnp = wave_sum_i(cnp);
         cnn = wave_sum_i(cnn);
         cnc = wave_sum_i(cnc);
-        if (lane == 0) { s->wtot[wv][0] = cnp; s->wtot[wv][1] = cnn; s->wtot[wv][2] = cnc; }
+        if (lane == 0) { s->wtot[wv][0] = cnp; s->wtot[wv][1] = cnn; s->wtot[wv][2] = cnc; s->wtot[wv][3] = nsl; }
         if (__any(anyp) && lane == 0) atomicOr(&s->cnt[0], 1);
         if (__any(anyn) && lane == 0) atomicOr(&s->cnt[0], 2);
     }
     __syncthreads();
     const int sides = s->cnt[0];
-    int bnp = 0, bnn = 0, bnc = 0, npt = 0, nnt = 0, n_cross_inst = 0;
+    int bnp = 0, bnn = 0, bnc = 0, bsl = 0, npt = 0, nnt = 0, n_cross_inst = 0, n_special = 0;
     for (int q = 0; q < NW; ++q) {
-        if (q < wv) { bnp += s->wtot[q][0]; bnn += s->wtot[q][1]; bnc += s->wtot[q][2]; }
+        if (q < wv) { bnp += s->wtot[q][0]; bnn += s->wtot[q][1]; bnc += s->wtot[q][2]; bsl += s->wtot[q][3]; }
         npt += s->wtot[q][0];
         nnt += s->wtot[q][1];
         n_cross_inst += s->wtot[q][2];
+        n_special += s->wtot[q][3];
     }
     __syncthreads();
     if (n_cross_inst == 0 && (!(sides & 1) || !(sides & 2))) {
@@ -1481,7 +1480,8 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
     // ---- stage B: crossing edges (lowest instance owns), new vertices -------
     uint32_t H = 16;
     while ((int)H < 2 * n_cross_inst + 2) H <<= 1;
-    const unsigned long long szB = 16ull * H + al16(12ull * n_cross_inst) + 64;
+    const unsigned long long oS = 16ull * H + al16(12ull * n_cross_inst);
+    const unsigned long long szB = oS + 8ull * n_special + 64;
     char* B = (char*)pc_alloc(pool, szB, s, 2, err, 1);
     if (!B) {
         if (tid == 0) heap_free(pool, sl, err);
@@ -1492,6 +1492,7 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
     int* hmin = (int*)(B + 8ull * H);  // lowest instance of the edge
     int* hid = hmin + H;               // vertex id of the edge's crossing point
     float* newv = (float*)(B + 16ull * H);
+    int2* spos = (int2*)(B + oS) + bsl;  // the wave's special triangles' first output positions on both sides
     for (uint32_t i = tid; i < H; i += PC_T) { hk[i] = PC_EMPTY; hmin[i] = 0x7fffffff; }
     __syncthreads();
     auto ekey = [](int a, int b) {
@@ -1866,7 +1867,7 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
             const bool special = k < te && is_special(t, c);
             const unsigned long long sm = ballot(special);
             if (special) {
-                spos[tb + js + mask_rank(sm)] = make_int2(op, on);
+                spos[js + mask_rank(sm)] = make_int2(op, on);
             } else if (k < te) {
                 const int side = np_ ? 0 : 1;
                 int* o = side ? otn : otp;
@@ -1886,7 +1887,7 @@ __device__ inline PcResult plane_cut_block_lds(const float* __restrict__ V, cons
         for (int j = lane; j < nsl; j += 64) {
             const PcTri t = load(sl[tb + j]);
             const int c = code(t);
-            const int2 at = spos[tb + j];
+            const int2 at = spos[j];
             if ((c & 3) && otp) put_pieces(0, pieces(t, c, 0), otp + 3 * at.x);
             if (((c >> 2) & 3) && otn) put_pieces(1, pieces(t, c, 1), otn + 3 * at.y);
         }
