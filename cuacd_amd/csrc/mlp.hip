@@ -65,7 +65,7 @@ __host__ __device__ __forceinline__ float bf2f(bf16_t b) {
 }
 
 // ---------------------------------------------------------------------------
-// GEMM: C[M x N] = alpha * A[M x K] . B[K x N] (+ bias[n]) (ReLU) (* (mask > 0))
+// GEMM (the layer-by-layer path): C[M x N] = A[M x K] . B[K x N] (+ bias[n]) (ReLU)
 // A(m, k) = A[m * sam + k * sak], B(k, n) = B[k * sbk + n * sbn] (BF16), so
 // transposed operands are strides. 64 x 64 output tile per 256-thread
 // workgroup, K in steps of 32 staged through LDS; each wave owns a 32 x 32
@@ -79,17 +79,12 @@ struct GemmArgs {
     long long sam, sak;
     const bf16_t* B;
     long long sbk, sbn;
-    float alpha;
-    const float* bias;   // [N] or null
+    const float* bias;  // [N] or null
     int relu;
-    const bf16_t* mask;  // [M x N] with row stride ldm, or null: out *= (mask > 0)
-    long long ldm;
-    float* C;            // FP32 out (row stride ldc) or null
+    float* C;           // FP32 out (row stride ldc) or null
     long long ldc;
-    bf16_t* Cb;          // BF16 out (row stride ldcb) or null
+    bf16_t* Cb;         // BF16 out (row stride ldcb) or null
     long long ldcb;
-    int kchunk;          // split K: workgroup z covers k in [z kchunk, (z + 1) kchunk)
-    float* part;         // split K: raw partial sums [gridDim.z x M x N] (epilogue in the reduction)
 };
 
 constexpr int GM = 64, GN = 64, GK = 32, GKP = GK + 8;  // LDS rows padded by 16 bytes
@@ -106,20 +101,19 @@ __global__ __launch_bounds__(256) void mlp_gemm_kernel(GemmArgs g) {
 #pragma unroll
         for (int j = 0; j < 2; ++j) acc[i][j] = f4v_t{0.f, 0.f, 0.f, 0.f};
     const int lr = tid >> 2, lk = (tid & 3) * 8;  // loader: one row (or column), 8 consecutive k
-    const int kb = blockIdx.z * g.kchunk, ke = min(g.K, kb + g.kchunk);
-    for (int k0 = kb; k0 < ke; k0 += GK) {
+    for (int k0 = 0; k0 < g.K; k0 += GK) {
         {
             const int m = m0 + lr;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int k = k0 + lk + j;
-                As[lr][lk + j] = (m < g.M && k < ke) ? g.A[(long long)m * g.sam + (long long)k * g.sak] : (bf16_t)0;
+                As[lr][lk + j] = (m < g.M && k < g.K) ? g.A[(long long)m * g.sam + (long long)k * g.sak] : (bf16_t)0;
             }
             const int n = n0 + lr;
 #pragma unroll
             for (int j = 0; j < 8; ++j) {
                 const int k = k0 + lk + j;
-                Bt[lr][lk + j] = (n < g.N && k < ke) ? g.B[(long long)k * g.sbk + (long long)n * g.sbn] : (bf16_t)0;
+                Bt[lr][lk + j] = (n < g.N && k < g.K) ? g.B[(long long)k * g.sbk + (long long)n * g.sbn] : (bf16_t)0;
             }
         }
         __syncthreads();
@@ -152,14 +146,9 @@ __global__ __launch_bounds__(256) void mlp_gemm_kernel(GemmArgs g) {
             for (int r = 0; r < 4; ++r) {
                 const int m = m0 + wm + 16 * i + 4 * (lane >> 4) + r;
                 if (m >= g.M) continue;
-                if (g.part) {
-                    g.part[((long long)blockIdx.z * g.M + m) * g.N + n] = acc[i][j][r];
-                    continue;
-                }
-                float v = g.alpha * acc[i][j][r];
+                float v = acc[i][j][r];
                 if (g.bias) v += g.bias[n];
                 if (g.relu) v = fmaxf(v, 0.0f);
-                if (g.mask && !(bf2f(g.mask[(long long)m * g.ldm + n]) > 0.0f)) v = 0.0f;
                 if (g.C) g.C[(long long)m * g.ldc + n] = v;
                 if (g.Cb) g.Cb[(long long)m * g.ldcb + n] = f2bf(v);
             }
@@ -717,21 +706,6 @@ __global__ __launch_bounds__(256) void mlp_grad_reduce(GradJobs jobs, float* g, 
     else g[J.b_off + i - rows * cols] = v;
 }
 
-// Split-K reduction with the GEMM's epilogue: C = alpha * sum_z part[z] ...
-__global__ void mlp_splitk_reduce(GemmArgs g, int nz) {
-    const long long i = (long long)blockIdx.x * blockDim.x + threadIdx.x;
-    if (i >= (long long)g.M * g.N) return;
-    const int m = (int)(i / g.N), n = (int)(i % g.N);
-    float v = 0.0f;
-    for (int z = 0; z < nz; ++z) v += g.part[(long long)z * g.M * g.N + i];
-    v *= g.alpha;
-    if (g.bias) v += g.bias[n];
-    if (g.relu) v = fmaxf(v, 0.0f);
-    if (g.mask && !(bf2f(g.mask[(long long)m * g.ldm + n]) > 0.0f)) v = 0.0f;
-    if (g.C) g.C[(long long)m * g.ldc + n] = v;
-    if (g.Cb) g.Cb[(long long)m * g.ldcb + n] = f2bf(v);
-}
-
 // ---------------------------------------------------------------------------
 // Elementwise / reduction kernels
 // ---------------------------------------------------------------------------
@@ -943,8 +917,9 @@ template <class T> T* carve(char*& p, size_t n) {
     return r;
 }
 
-// split-K workspace of at least n floats (grow-only; a growth waits for the
-// stream so no launch still reads the old buffer)
+// workspace of at least n floats for the weight gradients' partial sums
+// (grow-only; a growth waits for the stream so no launch still reads the old
+// buffer)
 float* part_ws(gpu_ctx_t ctx, gpu_mlp* mp, size_t n) {
     if (n > mp->part_cap) {
         if (hipStreamSynchronize(ctx->stream) != hipSuccess) return nullptr;
@@ -957,30 +932,14 @@ float* part_ws(gpu_ctx_t ctx, gpu_mlp* mp, size_t n) {
     return mp->part;
 }
 
-int gemm(gpu_ctx_t ctx, gpu_mlp* mp, int M, int N, int K, const bf16_t* A, long long sam, long long sak, const bf16_t* B,
-         long long sbk, long long sbn, const float* bias, int relu, const bf16_t* mask, long long ldm, float* C,
-         long long ldc, bf16_t* Cb, long long ldcb, float alpha = 1.0f) {
+int gemm(gpu_ctx_t ctx, int M, int N, int K, const bf16_t* A, long long sam, long long sak, const bf16_t* B,
+         long long sbk, long long sbn, const float* bias, int relu, float* C, long long ldc, bf16_t* Cb,
+         long long ldcb) {
     if (M <= 0 || N <= 0) return 0;
-    GemmArgs g{M, N, K, A, sam, sak, B, sbk, sbn, alpha, bias, relu, mask, ldm, C, ldc, Cb, ldcb, K, nullptr};
+    const GemmArgs g{M, N, K, A, sam, sak, B, sbk, sbn, bias, relu, C, ldc, Cb, ldcb};
     const int tm = (M + GM - 1) / GM, tn = (N + GN - 1) / GN;
-    // few output tiles over a long K (the weight gradients): split K across
-    // workgroups, partial sums reduced by a second kernel with the epilogue
-    int nz = 1;
-    if (tm * tn < 128 && K >= 4096) {
-        nz = std::min((1024 + tm * tn - 1) / (tm * tn), (K + 511) / 512);
-        const int kc = ((K + nz - 1) / nz + GK - 1) / GK * GK;
-        nz = (K + kc - 1) / kc;
-        g.kchunk = kc;
-        g.part = part_ws(ctx, mp, (size_t)nz * M * N);
-        REQUIRE(g.part, "mlp: split-K workspace allocation failed");
-    }
-    hipLaunchKernelGGL(mlp_gemm_kernel, dim3((unsigned)tn, (unsigned)tm, (unsigned)nz), dim3(256), 0, ctx->stream, g);
+    hipLaunchKernelGGL(mlp_gemm_kernel, dim3((unsigned)tn, (unsigned)tm), dim3(256), 0, ctx->stream, g);
     HIP_TRY(hipGetLastError());
-    if (nz > 1) {
-        const long long n = (long long)M * N;
-        hipLaunchKernelGGL(mlp_splitk_reduce, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, ctx->stream, g, nz);
-        HIP_TRY(hipGetLastError());
-    }
     return 0;
 }
 
@@ -1059,11 +1018,11 @@ int forward_layers(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* 
     hipLaunchKernelGGL(mlp_pack_points, dim3((unsigned)((R + 255) / 256)), dim3(256), 0, ctx->stream, d_pts,
                        d_planes, d_part, C, a.X, a.S);
     HIP_TRY(hipGetLastError());
-    if (int rc = gemm(ctx, mp, R, HD, KIN, a.X, KIN, 1, W + P_W1, HD, 1, Wf + P_B1, 1, nullptr, 0, nullptr, 0, a.A1, HD))
+    if (int rc = gemm(ctx, R, HD, KIN, a.X, KIN, 1, W + P_W1, HD, 1, Wf + P_B1, 1, nullptr, 0, a.A1, HD))
         return rc;
-    if (int rc = gemm(ctx, mp, R, HD, HD, a.A1, HD, 1, W + P_W2, HD, 1, Wf + P_B2, 1, nullptr, 0, nullptr, 0, a.A2, HD))
+    if (int rc = gemm(ctx, R, HD, HD, a.A1, HD, 1, W + P_W2, HD, 1, Wf + P_B2, 1, nullptr, 0, a.A2, HD))
         return rc;
-    if (int rc = gemm(ctx, mp, R, HD, HD, a.A2, HD, 1, W + P_W3, HD, 1, Wf + P_B3, 1, nullptr, 0, nullptr, 0, a.A3, HD))
+    if (int rc = gemm(ctx, R, HD, HD, a.A2, HD, 1, W + P_W3, HD, 1, Wf + P_B3, 1, nullptr, 0, a.A3, HD))
         return rc;
     hipLaunchKernelGGL(mlp_maxpool, dim3((unsigned)C), dim3(HD), 0, ctx->stream, a.A3, a.S, C, a.G);
     HIP_TRY(hipGetLastError());
@@ -1073,11 +1032,11 @@ int forward_layers(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* 
                            d_planes, C, a.Hin);
         HIP_TRY(hipGetLastError());
     }
-    if (int rc = gemm(ctx, mp, C, HD, KH, a.Hin, KH, 1, W + P_H1, HD, 1, Wf + P_C1, 1, nullptr, 0, nullptr, 0, a.B1, HD))
+    if (int rc = gemm(ctx, C, HD, KH, a.Hin, KH, 1, W + P_H1, HD, 1, Wf + P_C1, 1, nullptr, 0, a.B1, HD))
         return rc;
-    if (int rc = gemm(ctx, mp, C, HD, HD, a.B1, HD, 1, W + P_H2, HD, 1, Wf + P_C2, 1, nullptr, 0, nullptr, 0, a.B2, HD))
+    if (int rc = gemm(ctx, C, HD, HD, a.B1, HD, 1, W + P_H2, HD, 1, Wf + P_C2, 1, nullptr, 0, a.B2, HD))
         return rc;
-    return gemm(ctx, mp, C, NO, HD, a.B2, HD, 1, W + P_H3, NO, 1, Wf + P_C3, 0, nullptr, 0, a.Yw, NO, nullptr, 0);
+    return gemm(ctx, C, NO, HD, a.B2, HD, 1, W + P_H3, NO, 1, Wf + P_C3, 0, a.Yw, NO, nullptr, 0);
 }
 
 // point layers and pooling (arg: also the pooled rows)
@@ -1168,13 +1127,12 @@ int train_grads(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, const float* d_p
     return 0;
 }
 
-// Inputs staged on the device (points [P*NS*3], planes [C*4], part_of, cand
-// offsets, targets), grow-only per context call.
+// Inputs staged on the device (points [P*NS*3], planes [C*4], part_of,
+// targets), for one call.
 struct Staged {
     float* pts = nullptr;
     float* planes = nullptr;
     int* part = nullptr;
-    int* coff = nullptr;
     float* t = nullptr;
     char* base = nullptr;
     gpu_ctx_t ctx = nullptr;
@@ -1182,29 +1140,22 @@ struct Staged {
         if (base) (void)hipFreeAsync(base, ctx->stream);
     }
     int load(gpu_ctx_t c, const float* h_pts, int P, const float* h_planes, const int* h_part, int C,
-             const float* h_t, std::vector<int>& coff_h) {
+             const float* h_t) {
         ctx = c;
-        coff_h.assign(P + 1, 0);
         for (int i = 0; i < C; ++i) {
             if (h_part[i] < 0 || h_part[i] >= P) return -2;
             if (i > 0 && h_part[i] < h_part[i - 1]) return -3;
-            coff_h[h_part[i] + 1]++;
         }
-        for (int p = 0; p < P; ++p) coff_h[p + 1] += coff_h[p];
         const size_t b0 = ((size_t)P * NS * 12 + 255) / 256 * 256, b1 = ((size_t)C * 16 + 255) / 256 * 256,
-                     b2 = ((size_t)C * 4 + 255) / 256 * 256, b3 = ((size_t)(P + 1) * 4 + 255) / 256 * 256,
-                     b4 = ((size_t)C * 4 + 255) / 256 * 256;
-        if (hipMallocAsync((void**)&base, b0 + b1 + b2 + b3 + b4 + 256, c->stream) != hipSuccess) return -1;
+                     b2 = ((size_t)C * 4 + 255) / 256 * 256;
+        if (hipMallocAsync((void**)&base, b0 + b1 + 2 * b2 + 256, c->stream) != hipSuccess) return -1;
         pts = (float*)base;
         planes = (float*)(base + b0);
         part = (int*)(base + b0 + b1);
-        coff = (int*)(base + b0 + b1 + b2);
-        t = (float*)(base + b0 + b1 + b2 + b3);
+        t = (float*)(base + b0 + b1 + b2);
         if (hipMemcpyAsync(pts, h_pts, (size_t)P * NS * 12, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
             hipMemcpyAsync(planes, h_planes, (size_t)C * 16, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-            hipMemcpyAsync(part, h_part, (size_t)C * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess ||
-            hipMemcpyAsync(coff, coff_h.data(), (size_t)(P + 1) * 4, hipMemcpyHostToDevice, c->stream) !=
-                hipSuccess)
+            hipMemcpyAsync(part, h_part, (size_t)C * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess)
             return -1;
         if (h_t && hipMemcpyAsync(t, h_t, (size_t)C * 4, hipMemcpyHostToDevice, c->stream) != hipSuccess) return -1;
         return 0;
@@ -1224,7 +1175,7 @@ namespace cuacd {
 int mlp_forward_dev(gpu_ctx_t ctx, gpu_mlp* mp, const float* d_pts, int P, const float* d_planes, const int* d_part,
                     int C, float* d_out) {
     // bounded activations: slices of at most 8192 candidates (2M encoder
-    // rows) layer by layer; the fused kernel keeps those rows in LDS
+    // rows) layer by layer; the fused kernel keeps those rows in registers
     (void)P;
     const bool fused = mlp_fused_on() != 0;
     const int slice = fused ? 65536 : 8192;
@@ -1347,8 +1298,7 @@ int gpu_mlp_forward(gpu_ctx_t ctx, gpu_mlp_t m, const float* points, int n_parts
     if (n_cand == 0) return 0;
     HIP_TRY(hipSetDevice(ctx->device));
     Staged s;
-    std::vector<int> coff;
-    if (int rc = s.load(ctx, points, n_parts, planes, part_of, n_cand, nullptr, coff)) return stage_err(ctx, rc);
+    if (int rc = s.load(ctx, points, n_parts, planes, part_of, n_cand, nullptr)) return stage_err(ctx, rc);
     float* d_out = nullptr;
     HIP_TRY(hipMallocAsync((void**)&d_out, 4ll * n_cand + 16, ctx->stream));
     int rc = mlp_forward_dev(ctx, m, s.pts, n_parts, s.planes, s.part, n_cand, d_out);
@@ -1366,8 +1316,7 @@ int gpu_mlp_train_step(gpu_ctx_t ctx, gpu_mlp_t m, const float* points, int n_pa
     REQUIRE(m && n_parts > 0 && n_cand > 0, "mlp_train_step: bad arguments");
     HIP_TRY(hipSetDevice(ctx->device));
     Staged s;
-    std::vector<int> coff;
-    if (int rc = s.load(ctx, points, n_parts, planes, part_of, n_cand, targets, coff)) return stage_err(ctx, rc);
+    if (int rc = s.load(ctx, points, n_parts, planes, part_of, n_cand, targets)) return stage_err(ctx, rc);
     Act a;
     if (int rc = act_layout(ctx, m, n_cand, ACT_TRAIN, &a)) return rc;
     if (int rc = train_grads(ctx, m, s.pts, s.planes, s.part, s.t, n_cand, a)) return rc;
@@ -1447,8 +1396,7 @@ int gpu_mlp_gemm_test(gpu_ctx_t ctx, int M, int N, int K, const unsigned short* 
     HIP_TRY(hipMallocAsync((void**)&dC, 4ll * M * N, ctx->stream));
     HIP_TRY(hipMemcpyAsync(dA, A, 2 * a_len, hipMemcpyHostToDevice, ctx->stream));
     HIP_TRY(hipMemcpyAsync(dB, B, 2 * b_len, hipMemcpyHostToDevice, ctx->stream));
-    gpu_mlp tmp{};  // holds the split-K workspace of this call
-    int rc = gemm(ctx, &tmp, M, N, K, dA, sam, sak, dB, sbk, sbn, nullptr, 0, nullptr, 0, dC, N, nullptr, 0);
+    int rc = gemm(ctx, M, N, K, dA, sam, sak, dB, sbk, sbn, nullptr, 0, dC, N, nullptr, 0);
     if (rc == 0) {
         HIP_TRY(hipMemcpyAsync(C, dC, 4ll * M * N, hipMemcpyDeviceToHost, ctx->stream));
         HIP_TRY(hipStreamSynchronize(ctx->stream));
@@ -1457,7 +1405,6 @@ int gpu_mlp_gemm_test(gpu_ctx_t ctx, int M, int N, int K, const unsigned short* 
     (void)hipFreeAsync(dB, ctx->stream);
     (void)hipFreeAsync(dC, ctx->stream);
     (void)hipStreamSynchronize(ctx->stream);
-    if (tmp.part) (void)hipFree(tmp.part);
     return rc;
 }
 
