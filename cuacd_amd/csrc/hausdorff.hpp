@@ -339,9 +339,11 @@ __device__ inline float hd_wave_nearest_d2(const HdBvh& b, V3 p, float best, flo
     const int lane = lane_id();
     const int n1 = b.cnt[1], ntp = (b.nt + 3) / 4 * 4;
     const int groups = (n1 + 63) / 64;
-    // a box is passed over only when it is farther by more than the rounding
-    // of its distance and a triangle's, so the visiting order cannot change
-    // which triangle is found nearest
+    // a box is passed over only when its squared distance is 1e-5 above the
+    // bound: more than the rounding of either, so the order of visits does not
+    // show in the result. (Tilted slivers nearer than 1e-5 of their length could
+    // round by more, in the last bits: on thin sheets down to 1e-7 of their size
+    // the search gave the FP32 minimum over all triangles at every sample.)
     auto near = [&](float d) { return d * 0.99999f < best; };
     for (int g0 = 0; g0 < groups; g0 += 64) {
         const int g = g0 + lane;

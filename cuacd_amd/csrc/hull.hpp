@@ -9,14 +9,19 @@
 //
 // The algorithm is this library's own and is built for 64-lane waves:
 //   * points live in registers, PPL per thread (local point i sits in thread
-//     i % T, slot i / T, T = threads of the group), so "farthest conflict
-//     point" is one 64-bit max reduction;
+//     i % T, slot i / T, T = threads of the group), each with a key (height
+//     above its conflict face, then index), so "farthest conflict point" is
+//     one max reduction;
 //   * faces (plane, vertices, neighbours) live in a workspace that is LDS for
-//     small hulls (one wave, AS = 3) and global memory for big ones (several
-//     waves, AS = 1); the region visible from a new apex is found by a
-//     cooperative BFS over face adjacency, the horizon is extracted in
-//     parallel and the cone of new faces is stitched with per-vertex start/end
-//     maps (no serial ring walk);
+//     hulls of up to about a thousand vertices (AS = 3) and global memory for
+//     larger ones (AS = 1);
+//   * three kinds of step: one wave inserts one point at a time
+//     (wave_quickhull); several waves share one insertion (block_quickhull,
+//     single-apex: a cooperative walk over face adjacency, the cone stitched
+//     with per-vertex start/end maps); or every wave brings a candidate and
+//     those that do not touch each other go in together (MULTI rounds). The
+//     first and the last find the region visible from an apex by testing every
+//     face while there are few enough of them;
 //   * only conflict points of deleted faces are re-tested, against the new
 //     faces (quickhull outside-set reassignment).
 // Orientation predicate: fp32 plane filter with a proven error bound, and the

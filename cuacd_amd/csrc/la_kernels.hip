@@ -370,7 +370,8 @@ __global__ __launch_bounds__(64) void la_kdop_ext_kernel(LaHullTask* tasks, cons
 // Vertex capacity: the 80 extreme points (a hull of them has at most 80
 // corners, and the face arrays hold 2 * 80 + 8, the live faces plus one
 // insertion's transient pair). A smaller workspace fits more of these
-// one-wave workgroups on a CU (14 at 11.5 KB of LDS each).
+// one-wave workgroups on a CU (12 at 13.6 KB of LDS each, 11.9 of them the
+// workspace).
 constexpr int KD_VC = KD_NE;
 constexpr unsigned KD_WS = 11920;  // LDS of its workspace (la_launch_kdop checks the size)
 __global__ __launch_bounds__(64) void la_kdop_rough_kernel(LaHullTask* tasks, const int* ids, int n,
@@ -1466,10 +1467,11 @@ using WaveFn = void (*)(LaHullTask*, const int*, int, const int*, int, int*, DPo
 //     together
 //   11 b4_split: percent of the 1025-2048-point sets (the smallest) hulled by
 //     the HBM-workspace kernel on the context's stream beside the LDS tier's
-//     stream (CUACD_HULL_B4_SPLIT, 0..90; default 0): that kernel needs 5 KB
-//     of LDS, so its workgroups fit on the CUs the LDS tier fills, whose
-//     VALUs are mostly idle. On the 64-mesh search step 25 and 40 measured
-//     slower (2.43 s and 2.50 s against 2.27 s)
+//     stream (CUACD_HULL_B4_SPLIT, 0..90; default 0): its faces are in HBM, so
+//     it takes 37 KB of LDS at this size (5 KB without multi_hbm) and its
+//     workgroups fit on the CUs the LDS tier fills, whose VALUs are mostly
+//     idle. On the 64-mesh search step 25 and 40 measured slower (2.43 s and
+//     2.50 s against 2.27 s, single-apex steps)
 //   12 order: the four-wave and wave tiers of a hull call wait for the first
 //     passes of the eight-wave LDS tiers (CUACD_HULL_ORDER, 0/1; default 1).
 //     An eight-wave LDS workgroup needs a whole CU's LDS, so it only starts on
