@@ -54,10 +54,10 @@ PARAMS = dict(max_iters=100, width=30, width2=5, threshold=0.05, depth=2, max_n_
 # from their counters (profiles/lookahead_64sdf_hull_tier_counters.md):
 # counters cannot be read inside the timed run, so the line carries the
 # profiled figures beside the live HBM fraction
-HULL_VALU_BUSY = {"la_hull_ldsv<2,8>": 0.042, "la_hull_ldsv<4,8>": 0.024, "la_hull_ldsv<2,4>": 0.034,
-                  "la_hull_ldsv<8,8>": 0.024, "la_hull_block<8>": 0.004}
-HULL_TRAFFIC = {"la_hull_ldsv<2,8>": 74.90e6, "la_hull_ldsv<4,8>": 49.78e6, "la_hull_ldsv<2,4>": 59.41e6,
-                "la_hull_ldsv<8,8>": 78.93e6}
+HULL_VALU_BUSY = {"la_hull_ldsv<2,8>": 0.046, "la_hull_ldsv<4,8>": 0.028, "la_hull_wave<8>": 0.023,
+                  "la_hull_ldsv<8,8>": 0.028, "la_hull_block<8>": 0.011}
+HULL_TRAFFIC = {"la_hull_ldsv<2,8>": 74.74e6, "la_hull_ldsv<4,8>": 49.92e6, "la_hull_wave<8>": 23.72e6,
+                "la_hull_ldsv<8,8>": 80.30e6, "la_hull_block<8>": 81.38e6}
 LA_LIMITER = ("latency: each hull is a chain of dependent insertion steps (LDS reads and writes, block barriers); "
               "HBM traffic is ~1x the algorithmic bytes, so the HBM fraction only says how far from a bandwidth "
               "bound this work sits")
