@@ -176,7 +176,8 @@ __global__ __launch_bounds__(HD_T) void hd_prep_kernel(HdTask* tasks, int n_task
 // the other workgroups leave it) only skips work that cannot raise the result.
 // Bound by the BVH reads of the bounds. Walking every sample's tree, a lane
 // each, took 3.66 ms for 512 pairs of 1280-triangle meshes and their hulls,
-// 4096 samples each way.
+// 4096 samples each way; this takes 1.19 ms (1.25 before a search's sample and
+// snapshot of the maximum were scalars).
 constexpr int HD_QB = 1024, HD_BINS = 64, HD_FIRST = 16;
 
 struct HdQueryLDS {

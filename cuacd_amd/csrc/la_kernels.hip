@@ -1424,7 +1424,8 @@ using WaveFn = void (*)(LaHullTask*, const int*, int, const int*, int, int*, DPo
 // initial values from the environment, changed at run time through
 // gpu_set_tuning (the autotuner).
 //   0 wide_min: wave-tier sets above this many points run four waves per hull
-//     (CUACD_HULL_WIDE_MIN, 0 disables; default 512). With the one-wave
+//     (CUACD_HULL_WIDE_MIN, 0 disables; default 512; device-counted calls take
+//     at most 256). With the one-wave
 //     quickhull and a 3/8-capacity first pass, the 257-512-point tier of a
 //     24-mesh search takes 105 + 55 ms (retries) on one wave and 130 + 64 ms
 //     on four; at 513-1024 points one wave takes 124 + 39 ms against 83 + 21
